@@ -39,7 +39,8 @@ struct GemvParams {
   int attn_max_splits;
 };
 
-// K must be 4096 or 14336.  rows > 1 re-reads the weights once per row.
+// K must be 4096 or 14336.  rows > 1 (kEpiF32 with norm at K = 4096 only) reads the weights once
+// per 16 rows; each row is the one-row call's, bit for bit.
 int launch_gemv(int K, int epi, bool norm, GemvParams p, int rows, hipStream_t st);
 int default_ppw(int n_pairs);
 int gemv_waves(int K, int epi, int n_pairs);

@@ -15,6 +15,8 @@
 // The input vector is staged once per workgroup in LDS; with `norm` the staging
 // applies RMSNorm (rmsnorm.cu:31-63) on the way in, so no normalised copy of the
 // activations is ever written to HBM.
+#include <algorithm>
+
 #include "ie_kernels.h"
 
 namespace ie {
@@ -90,14 +92,12 @@ __device__ __forceinline__ EpiPre epi_preload(const GemvParams& p, int pair) {
 }
 
 template <int EPI>
-__device__ __forceinline__ void gemv_epilogue(const GemvParams& p, int pair, int row, float a0,
-                                              float a1, const EpiPre& e) {
+__device__ __forceinline__ void gemv_epilogue(const GemvParams& p, int pair, float a0, float a1,
+                                              const EpiPre& e) {
   if constexpr (EPI == kEpiBf16) {
-    uint16_t* o = p.out + (size_t)row * p.out_stride + 2 * pair;
-    *reinterpret_cast<uint32_t*>(o) = pack_bf2(a0, a1);
+    *reinterpret_cast<uint32_t*>(p.out + 2 * pair) = pack_bf2(a0, a1);
   } else if constexpr (EPI == kEpiF32) {
-    float* o = p.out_f32 + (size_t)row * p.out_stride + 2 * pair;
-    *reinterpret_cast<float2*>(o) = make_float2(a0, a1);
+    *reinterpret_cast<float2*>(p.out_f32 + 2 * pair) = make_float2(a0, a1);
   } else if constexpr (EPI == kEpiResid) {
     uint32_t* o = reinterpret_cast<uint32_t*>(p.out + 2 * pair);
     const uint32_t old = e.have ? e.old : *o;
@@ -212,7 +212,7 @@ __device__ __forceinline__ void issue_step(const GemvParams& p, int first, int l
 // Dot products of step t against the staged input; the row pair's epilogue after its last step.
 template <int EPI, int G, int NG>
 __device__ __forceinline__ void consume_step(const GemvParams& p, const u32x4_t* xs, int first,
-                                             int row, int lane, int t, const u32x4_t (&wa)[G],
+                                             int lane, int t, const u32x4_t (&wa)[G],
                                              const u32x4_t (&wb)[G], float& acc0, float& acc1,
                                              const EpiPre& e) {
   const int g = t % NG;
@@ -225,7 +225,7 @@ __device__ __forceinline__ void consume_step(const GemvParams& p, const u32x4_t*
   if (g == NG - 1) {
     const float a0 = wave_sum(acc0), a1 = wave_sum(acc1);
     if (lane == 0 && first + t / NG < p.n_pairs)
-      gemv_epilogue<EPI>(p, first + t / NG, row, a0, a1, e);
+      gemv_epilogue<EPI>(p, first + t / NG, a0, a1, e);
     acc0 = 0.f;
     acc1 = 0.f;
   }
@@ -249,7 +249,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvParams p) {
   __shared__ float red[WAVES];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int row = blockIdx.y;
   const int first = (blockIdx.x * WAVES + wave) * p.ppw;
   const int npairs = max(0, min(p.ppw, p.n_pairs - first));
   const int nsteps = npairs * NG;
@@ -259,7 +258,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvParams p) {
   // staging below waits for it alone.  These loads and the first two weight steps are
   // unconditional (indices clamped): a load under a branch makes the compiler's wait at the
   // join conservative, which would stall the staging until the weights arrive.
-  const u32x4_t* x4 = reinterpret_cast<const u32x4_t*>(p.x + (size_t)row * p.x_stride);
+  const u32x4_t* x4 = reinterpret_cast<const u32x4_t*>(p.x);
   u32x4_t xin[XC], nwin[XC];
   AttnItem<ATTN ? ATTN : 1> ai[ATTN ? AI : 1];
   int ns = 0;
@@ -318,25 +317,155 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvParams p) {
   if constexpr (ONE) {
 #pragma unroll
     for (int t = 0; t < NG; t += 2) {
-      consume_step<EPI, G, NG>(p, xs, first, row, lane, t, a0, b0, acc0, acc1, epre);
+      consume_step<EPI, G, NG>(p, xs, first, lane, t, a0, b0, acc0, acc1, epre);
       if (t + 2 < NG) issue_step<K, EPI, G, NG>(p, first, lane, t + 2, a0, b0);
-      consume_step<EPI, G, NG>(p, xs, first, row, lane, t + 1, a1, b1, acc0, acc1, epre);
+      consume_step<EPI, G, NG>(p, xs, first, lane, t + 1, a1, b1, acc0, acc1, epre);
       if (t + 3 < NG) issue_step<K, EPI, G, NG>(p, first, lane, t + 3, a1, b1);
     }
   } else {
     for (int t = 0; t < nsteps; t += 2) {
-      consume_step<EPI, G, NG>(p, xs, first, row, lane, t, a0, b0, acc0, acc1, epre);
+      consume_step<EPI, G, NG>(p, xs, first, lane, t, a0, b0, acc0, acc1, epre);
       if (t + 2 < nsteps) issue_step<K, EPI, G, NG>(p, first, lane, t + 2, a0, b0);
-      consume_step<EPI, G, NG>(p, xs, first, row, lane, t + 1, a1, b1, acc0, acc1, epre);
+      consume_step<EPI, G, NG>(p, xs, first, lane, t + 1, a1, b1, acc0, acc1, epre);
       if (t + 3 < nsteps) issue_step<K, EPI, G, NG>(p, first, lane, t + 3, a1, b1);
     }
   }
 }
 
+// wave_sum of R values at once (R = 4, 8 or 16): lane l receives the sum of v[l % R], added up in
+// wave_sum's order.  At each of the first log2(R) levels the lanes of a pair each keep one of two
+// values, so a level halves the values left: R - 1 selects and additions in place of R log2(R).
+// (Partners l ^ 1, l ^ 2, l ^ 4, l ^ 8, l ^ 16, l ^ 32; wave_sum's mirrors reach the same sums.)
+template <int R>
+__device__ __forceinline__ float rows_sum(float (&v)[R], int lane) {
+  const auto x4 = [](float x) { return dpp_f<0x1B>(dpp_f<kDppRowHalfMirror>(x)); };  // (l ^ 7) ^ 3
+  const auto x8 = [](float x) { return dpp_f<0x128>(x); };                           // row_ror 8
+  const auto keep = [](bool hi, float lo_v, float hi_v) { return hi ? hi_v : lo_v; };
+#pragma unroll
+  for (int i = 0; i < R / 2; ++i) {
+    const bool hi = lane & 1;
+    v[i] = keep(hi, v[2 * i], v[2 * i + 1]) + dpp_f<kDppQuadXor1>(keep(hi, v[2 * i + 1], v[2 * i]));
+  }
+#pragma unroll
+  for (int i = 0; i < R / 4; ++i) {
+    const bool hi = lane & 2;
+    v[i] = keep(hi, v[2 * i], v[2 * i + 1]) + dpp_f<kDppQuadXor2>(keep(hi, v[2 * i + 1], v[2 * i]));
+  }
+  if constexpr (R >= 8) {
+#pragma unroll
+    for (int i = 0; i < R / 8; ++i) {
+      const bool hi = lane & 4;
+      v[i] = keep(hi, v[2 * i], v[2 * i + 1]) + x4(keep(hi, v[2 * i + 1], v[2 * i]));
+    }
+  } else {
+    v[0] += x4(v[0]);
+  }
+  if constexpr (R == 16) {
+    const bool hi = lane & 8;
+    v[0] = keep(hi, v[0], v[1]) + x8(keep(hi, v[1], v[0]));
+  } else {
+    v[0] += x8(v[0]);
+  }
+  return xor32_sum(xor16_sum(v[0]));
+}
+
+// RMSNorm + the fp32 product for 2 .. R rows (the head of a batch): bound by the weight stream,
+// which is read once for all the rows.  Per row the arithmetic of gemv_kernel<4096, kEpiF32,
+// NORM, 8 waves> in the same order, so each row's logits are those of a one-row call bit for
+// bit: the row's sum of squares over 8 wave sums of 512 chunks, the same chunk -> lane split of a
+// dot product, and the sum over the lanes in wave_sum's order.
+// A workgroup stages the R normalised rows in LDS once (8 KiB each) and its waves then walk row
+// pairs gridDim x waves apart, two half-pairs of weights in flight per wave, so the staging is
+// paid once per CU, not per 8 pairs: two workgroups a CU (4 waves a SIMD), one at R = 16
+// (128 KiB of LDS; its accumulators need the registers of 2 waves a SIMD anyway).
+// The head of 2 / 4 / 8 / 16 rows: 161 / 162 / 172 / 235 us, against 147 for one row and 147 a row
+// when each row re-read the weights.  Up to 8 rows that is the weight stream (6.1-6.5 TB/s); at
+// 16 the dot products (65 M wave instructions, ~120 us of issue) come on top of it at 2 waves a
+// SIMD.  Three instances, by the rows that fit: a 4-row call in the 8-row kernel would take 7% more.
+template <int R>
+__global__ __launch_bounds__(512, R > 8 ? 2 : 4) void gemv_rows_kernel(GemvParams p, int rows) {
+  constexpr int K = kHidden, G = 4, WAVES = 8;
+  static_assert(K == 8 * 512, "one 16-byte chunk of a row per thread");
+  __shared__ u32x4_t xs[R][K / 8];
+  __shared__ float red[R][8];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+
+  u32x4_t xin[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j)
+    xin[j] = reinterpret_cast<const u32x4_t*>(p.x + (size_t)min(j, rows - 1) * p.x_stride)[tid];
+  const u32x4_t nw = reinterpret_cast<const u32x4_t*>(p.norm_w)[tid];
+  __builtin_amdgcn_sched_barrier(0);  // the input loads ahead of the weight stream
+
+  const int stride = gridDim.x * WAVES;
+  int pair = blockIdx.x * WAVES + wave;
+  u32x4_t a0[G], b0[G], a1[G], b1[G];
+  const auto issue = [&](int pr, int g0, u32x4_t (&wa)[G], u32x4_t (&wb)[G]) {
+    const uint16_t *r0, *r1;
+    rows_of_pair<kEpiF32, K>(p, min(pr, p.n_pairs - 1), r0, r1);
+    load_step<G>(reinterpret_cast<const u32x4_t*>(r0) + lane,
+                 reinterpret_cast<const u32x4_t*>(r1) + lane, g0, wa, wb);
+  };
+  issue(pair, 0, a0, b0);
+
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const float ss = wave_sum(sumsq8(xin[j]));
+    if (lane == 0) red[j][wave] = ss;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    float tot = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) tot += red[j][w];
+    const float r = rsqrtf(tot / (float)K + kRmsEps);
+    xs[j][tid] = norm8(xin[j], nw, r);
+  }
+  issue(pair, G, a1, b1);  // (after the input rows have left their registers)
+  __syncthreads();
+
+  for (; pair < p.n_pairs; pair += stride) {
+    float acc0[R], acc1[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc0[r] = acc1[r] = 0.f;
+    const auto consume = [&](int g0, const u32x4_t (&wa)[G], const u32x4_t (&wb)[G]) {
+#pragma unroll
+      for (int c = 0; c < G; ++c) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const u32x4_t xv = xs[r][(g0 + c) * 64 + lane];
+          acc0[r] = dot8(wa[c], xv, acc0[r]);
+          acc1[r] = dot8(wb[c], xv, acc1[r]);
+          // (left alone the scheduler gathers the reads of a whole half-pair and spills)
+          if (r % (R > 8 ? 4 : 2) == 1) __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    };
+    consume(0, a0, b0);
+    issue(pair + stride, 0, a0, b0);
+    consume(G, a1, b1);
+    issue(pair + stride, G, a1, b1);
+    // lane r ends with row r's two sums
+    const float v0 = rows_sum<R>(acc0, lane), v1 = rows_sum<R>(acc1, lane);
+    if (lane < rows)
+      *reinterpret_cast<float2*>(p.out_f32 + (size_t)lane * p.out_stride + 2 * pair) =
+          make_float2(v0, v1);
+  }
+}
+
+template <int R>
+int launch_rows(const GemvParams& p, int rows, hipStream_t st) {
+  const int grid = std::min((p.n_pairs + 7) / 8, R > 8 ? 256 : 512);
+  hipLaunchKernelGGL((gemv_rows_kernel<R>), dim3(grid), dim3(512), 0, st, p, rows);
+  IE_CHECK_LAUNCH();
+  return IE_OK;
+}
+
 template <int K, int EPI, bool NORM, int WAVES, bool ONE>
-int launch_o(const GemvParams& p, int rows, hipStream_t st) {
+int launch_o(const GemvParams& p, hipStream_t st) {
   const int waves = (p.n_pairs + p.ppw - 1) / p.ppw;
-  dim3 grid((waves + WAVES - 1) / WAVES, rows);
+  dim3 grid((waves + WAVES - 1) / WAVES);
   if constexpr (K == kQHeads * kHeadDim && EPI == kEpiResid && !NORM) {
     if (p.attn_part_o) {
       if (p.attn_max_splits <= kAttnFusedSplits)
@@ -355,37 +484,37 @@ int launch_o(const GemvParams& p, int rows, hipStream_t st) {
 }
 
 template <int K, int EPI, bool NORM, int WAVES>
-int launch_w(const GemvParams& p, int rows, hipStream_t st) {
-  return p.ppw == 1 ? launch_o<K, EPI, NORM, WAVES, true>(p, rows, st)
-                    : launch_o<K, EPI, NORM, WAVES, false>(p, rows, st);
+int launch_w(const GemvParams& p, hipStream_t st) {
+  return p.ppw == 1 ? launch_o<K, EPI, NORM, WAVES, true>(p, st)
+                    : launch_o<K, EPI, NORM, WAVES, false>(p, st);
 }
 
 template <int K, int EPI, bool NORM>
-int launch_t(const GemvParams& p, int rows, hipStream_t st) {
+int launch_t(const GemvParams& p, hipStream_t st) {
   const int waves = gemv_waves(K, EPI, p.n_pairs);
   if constexpr (EPI == kEpiQkvRope) {
-    if (waves == 12) return launch_w<K, EPI, NORM, 12>(p, rows, st);
+    if (waves == 12) return launch_w<K, EPI, NORM, 12>(p, st);
   }
   switch (waves) {
-    case 8: return launch_w<K, EPI, NORM, 8>(p, rows, st);
-    case 16: return launch_w<K, EPI, NORM, 16>(p, rows, st);
-    default: return launch_w<K, EPI, NORM, 4>(p, rows, st);
+    case 8: return launch_w<K, EPI, NORM, 8>(p, st);
+    case 16: return launch_w<K, EPI, NORM, 16>(p, st);
+    default: return launch_w<K, EPI, NORM, 4>(p, st);
   }
 }
 
 template <int K>
-int launch_k(int epi, bool norm, const GemvParams& p, int rows, hipStream_t st) {
+int launch_k(int epi, bool norm, const GemvParams& p, hipStream_t st) {
   switch (epi) {
-    case kEpiBf16: return norm ? launch_t<K, kEpiBf16, true>(p, rows, st)
-                               : launch_t<K, kEpiBf16, false>(p, rows, st);
-    case kEpiF32: return norm ? launch_t<K, kEpiF32, true>(p, rows, st)
-                              : launch_t<K, kEpiF32, false>(p, rows, st);
-    case kEpiResid: return norm ? launch_t<K, kEpiResid, true>(p, rows, st)
-                                : launch_t<K, kEpiResid, false>(p, rows, st);
-    case kEpiSwiglu: return norm ? launch_t<K, kEpiSwiglu, true>(p, rows, st)
-                                 : launch_t<K, kEpiSwiglu, false>(p, rows, st);
-    case kEpiQkvRope: return norm ? launch_t<K, kEpiQkvRope, true>(p, rows, st)
-                                  : launch_t<K, kEpiQkvRope, false>(p, rows, st);
+    case kEpiBf16: return norm ? launch_t<K, kEpiBf16, true>(p, st)
+                               : launch_t<K, kEpiBf16, false>(p, st);
+    case kEpiF32: return norm ? launch_t<K, kEpiF32, true>(p, st)
+                              : launch_t<K, kEpiF32, false>(p, st);
+    case kEpiResid: return norm ? launch_t<K, kEpiResid, true>(p, st)
+                                : launch_t<K, kEpiResid, false>(p, st);
+    case kEpiSwiglu: return norm ? launch_t<K, kEpiSwiglu, true>(p, st)
+                                 : launch_t<K, kEpiSwiglu, false>(p, st);
+    case kEpiQkvRope: return norm ? launch_t<K, kEpiQkvRope, true>(p, st)
+                                  : launch_t<K, kEpiQkvRope, false>(p, st);
   }
   set_error("launch_gemv: bad epilogue %d", epi);
   return IE_ERR_INVALID_ARG;
@@ -423,16 +552,28 @@ int default_ppw(int n_pairs) {
 int launch_gemv(int K, int epi, bool norm, GemvParams p, int rows, hipStream_t st) {
   IE_REQUIRE(rows >= 1 && rows <= 65535, "launch_gemv: rows=%d out of range", rows);
   IE_REQUIRE(p.n_pairs >= 1, "launch_gemv: no rows");
-  IE_REQUIRE(rows == 1 || epi == kEpiBf16 || epi == kEpiF32,
+  IE_REQUIRE(rows == 1 || (epi == kEpiF32 && norm && K == kHidden),
              "launch_gemv: epilogue %d supports one row only", epi);
   IE_REQUIRE(!p.attn_part_o || (K == kQHeads * kHeadDim && epi == kEpiResid && !norm && rows == 1 &&
                                 p.attn_part_ml && p.attn_max_splits >= 1 &&
                                 p.attn_max_splits <= kAttnFusedSplitsLong &&
                                 (p.d_seq_len || (p.pos >= 1 && p.pos <= kMaxCtx))),
              "launch_gemv: attention-partials input is for the O projection only");
+  if (rows > 1) {
+    // 16 rows a launch; the smallest instance that holds the rest
+    for (int r0 = 0; r0 < rows; r0 += 16) {
+      GemvParams q = p;
+      q.x = p.x + r0 * p.x_stride;
+      q.out_f32 = p.out_f32 + r0 * p.out_stride;
+      const int n = std::min(16, rows - r0);
+      IE_TRY(n <= 4 ? launch_rows<4>(q, n, st) : n <= 8 ? launch_rows<8>(q, n, st)
+                                                        : launch_rows<16>(q, n, st));
+    }
+    return IE_OK;
+  }
   if (p.ppw <= 0) p.ppw = default_ppw(p.n_pairs);
-  if (K == 4096) return launch_k<4096>(epi, norm, p, rows, st);
-  if (K == 14336) return launch_k<14336>(epi, norm, p, rows, st);
+  if (K == 4096) return launch_k<4096>(epi, norm, p, st);
+  if (K == 14336) return launch_k<14336>(epi, norm, p, st);
   set_error("launch_gemv: unsupported K=%d (4096 or 14336)", K);
   return IE_ERR_UNSUPPORTED;
 }

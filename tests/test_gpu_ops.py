@@ -769,6 +769,25 @@ def test_top_p_ties_and_flat_rows(hip, ctx):
             assert int(out[r].item()) == want, (r, step, int(out[r].item()), want)
 
 
+@pytest.mark.parametrize("rows", [2, 4, 5, 8, 9, 16, 17, 64])
+def test_final_norm_lm_head_rows(hip, ctx, rows):
+    """The head of 2 .. 64 rows, at the edges of its 4-, 8- and 16-row kernels and of the 16-row
+    launches: each row is the one-row call's bit for bit, and nothing is written past the last."""
+    say(f"final_norm_lm_head rows={rows}")
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    def draw(*shape, mean=0.0, std=1.0):
+        return torch.empty(shape, dtype=torch.bfloat16, device="cuda").normal_(mean, std, generator=g)
+    x, nw, wl = draw(rows, H), draw(H, mean=1.0, std=0.02), draw(V, H, std=0.02)
+    out = torch.full((rows + 1, V), 7.0, device="cuda")
+    hip.check(hip.lib.ie_final_norm_lm_head(ctx.handle, rows, P(x), P(nw), P(wl), P(out)))
+    one = torch.empty(V, device="cuda")
+    for r in range(rows):
+        hip.check(hip.lib.ie_final_norm_lm_head(ctx.handle, 1, P(x[r]), P(nw), P(wl), P(one)))
+        sync()
+        assert torch.equal(out[r], one), r
+    assert bool((out[rows] == 7.0).all())
+
+
 def test_final_norm_lm_head_sampling_config3(hip, ctx):
     """Config 3: final RMSNorm + lm_head GEMV -> fp32 logits, argmax and top-p, B=1 and B=16."""
     say("final_norm_lm_head rows=16 + argmax + top-p")
