@@ -320,21 +320,31 @@ int ie_context_create(ie_context** out, int device, void* stream) {
   ie_context* c = new ie_context;
   c->device = device;
   int rc = IE_OK;
+  size_t zeroed = 0;
   do {
     c->stream = stream_of(stream);
     if (hipStreamCreateWithFlags(&c->capture, hipStreamNonBlocking) != hipSuccess) {
       rc = IE_ERR_HIP;
       break;
     }
-    if (hipMalloc(&c->d_counters, kNumCounters * sizeof(unsigned int)) != hipSuccess ||
-        hipMalloc(&c->d_slots, kNumSlots * kSlotStride * sizeof(unsigned long long)) != hipSuccess ||
-        hipMalloc(&c->d_params, 64 * sizeof(int)) != hipSuccess ||
-        hipMalloc(&c->d_sk_part, kSkPartBytes) != hipSuccess ||
-        hipHostMalloc(&c->h_params, 64 * sizeof(int), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc(&c->h_token, 64 * sizeof(int), hipHostMallocMapped) != hipSuccess) {
+    // one device allocation (the counters, slots and params, zeroed below, first) and one pinned
+    // one: each allocation is ~40-100 us of a context's creation
+    const size_t cnt = align256(kNumCounters * sizeof(unsigned int)),
+                 slots = align256(kNumSlots * kSlotStride * sizeof(unsigned long long)),
+                 params = align256(64 * sizeof(int));
+    zeroed = cnt + slots + params;
+    if (hipMalloc(&c->arena, zeroed + align256(kSkPartBytes) + kAttnPrefillPartBytes) != hipSuccess ||
+        hipHostMalloc(&c->h_params, 128 * sizeof(int), hipHostMallocMapped) != hipSuccess) {
       rc = IE_ERR_OOM;
       break;
     }
+    char* const base = static_cast<char*>(c->arena);
+    c->d_counters = reinterpret_cast<unsigned int*>(base);
+    c->d_slots = reinterpret_cast<unsigned long long*>(base + cnt);
+    c->d_params = reinterpret_cast<int*>(base + cnt + slots);
+    c->d_sk_part = reinterpret_cast<float*>(base + zeroed);
+    c->d_attn_part = reinterpret_cast<float*>(base + zeroed + align256(kSkPartBytes));
+    c->h_token = c->h_params + 64;
     if (hipHostGetDevicePointer(reinterpret_cast<void**>(&c->h_token_dev), c->h_token, 0) !=
         hipSuccess) {
       rc = IE_ERR_HIP;
@@ -345,10 +355,7 @@ int ie_context_create(ie_context** out, int device, void* stream) {
       rc = IE_ERR_HIP;
       break;
     }
-    if (hipMemset(c->d_counters, 0, kNumCounters * sizeof(unsigned int)) != hipSuccess ||
-        hipMemset(c->d_slots, 0, kNumSlots * kSlotStride * sizeof(unsigned long long)) != hipSuccess ||
-        hipMemset(c->d_params, 0, 64 * sizeof(int)) != hipSuccess ||
-        hipDeviceSynchronize() != hipSuccess) {
+    if (hipMemset(c->arena, 0, zeroed) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
       rc = IE_ERR_HIP;
       break;
     }
@@ -369,12 +376,8 @@ int ie_context_destroy(ie_context* c) {
   if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
   for (auto& bg : c->bgraph)
     if (bg.exec) (void)hipGraphExecDestroy(bg.exec);
-  (void)hipFree(c->d_counters);
-  (void)hipFree(c->d_slots);
-  (void)hipFree(c->d_params);
-  (void)hipFree(c->d_sk_part);
+  (void)hipFree(c->arena);
   if (c->h_params) (void)hipHostFree(c->h_params);
-  if (c->h_token) (void)hipHostFree(c->h_token);
   if (c->capture) (void)hipStreamDestroy(c->capture);
   if (c->gemm_ws) (void)hipFree(c->gemm_ws);
   delete c;
@@ -648,7 +651,8 @@ int prefill_layer(Context* c, hipStream_t st, const ie_model_weights& W, int l, 
                              data_buffer + (size_t)(S - 1) * kHidden, dw.attn1, dw, kvl, nullptr,
                              start_pos + S, block_table, n_pages);
   }
-  AttnPrefillParams a{qrot, kvl, vpl, attn_buffer, S, start_pos, block_table, n_pages};
+  AttnPrefillParams a{qrot, kvl, vpl, attn_buffer, S, start_pos, block_table, n_pages,
+                      c->d_attn_part};
   IE_TRY(launch_attn_prefill(a, st));
   GemmParams o{};
   o.x = attn_buffer;
@@ -1308,7 +1312,7 @@ int ie_attn_prefill_core(ie_context* c, int seq_len, int start_pos, const ie_bf1
                          const ie_bf16* d_k, const ie_bf16* d_v, ie_bf16* d_out) {
   CTX_OK(c);
   IE_REQUIRE(d_q && d_k && d_v && d_out, "attn_prefill_core: null pointer");
-  AttnPrefillParams a{d_q, d_k, d_v, d_out, seq_len, start_pos};
+  AttnPrefillParams a{d_q, d_k, d_v, d_out, seq_len, start_pos, nullptr, 0, c->d_attn_part};
   return launch_attn_prefill(a, c->stream);
 }
 
@@ -1321,7 +1325,7 @@ int ie_attn_prefill_core_paged(ie_context* c, int seq_len, int start_pos, const 
              "attn_prefill_core_paged: n_pages %d, layer %d", n_pages, layer);
   const uint16_t* kl = static_cast<const uint16_t*>(kv_pages) + (size_t)layer * kPageLayer;
   AttnPrefillParams a{d_q, kl, kl + (size_t)kKVHeads * kPageHead, d_out, seq_len, start_pos,
-                      block_table, n_pages};
+                      block_table, n_pages, c->d_attn_part};
   return launch_attn_prefill(a, c->stream);
 }
 
@@ -1438,7 +1442,8 @@ int ie_attn(ie_context* c, const float* d_rope_cos, const float* d_rope_sin, int
   IE_TRY(launch_qkv_rope_scatter(S, 0, qkv, d_rope_cos, d_rope_sin, qrot, kvl,
                                  kvl + (size_t)kKVHeads * kKVPlane, nullptr, 0, st));
   uint16_t* att = qkv;  // the projection is dead once scattered
-  AttnPrefillParams a{qrot, kvl, kvl + (size_t)kKVHeads * kKVPlane, att, S, 0};
+  AttnPrefillParams a{qrot, kvl, kvl + (size_t)kKVHeads * kKVPlane, att, S, 0, nullptr, 0,
+                      c->d_attn_part};
   IE_TRY(launch_attn_prefill(a, st));
   GemmParams o{};
   o.x = att;

@@ -242,11 +242,12 @@ struct Context {
   int device = 0;
   hipStream_t stream = nullptr;    // nullptr = the legacy default stream
   hipStream_t capture = nullptr;   // private stream the decode graph is captured on
+  void* arena = nullptr;           // the device allocation behind the d_ pointers below
   unsigned int* d_counters = nullptr;       // self-resetting last-block counters
   unsigned long long* d_slots = nullptr;    // 64-bit reduction slots (argmax)
   int* d_params = nullptr;                  // device copy of per-step scalars
   int* h_params = nullptr;                  // pinned staging for d_params
-  int* h_token = nullptr;                   // pinned, mapped token read-back
+  int* h_token = nullptr;                   // pinned, mapped token read-back (after h_params)
   int* h_token_dev = nullptr;               // device address of h_token (the argmax writes it)
   int next_seq = -1;                        // d_params[0] as the last decode step left it
   bool use_graph = true;
@@ -263,6 +264,8 @@ struct Context {
   unsigned long long bgraph_tick = 0;
   // the skinny GEMM's K-half partials (kSkPartBytes) for launches outside the batched step
   float* d_sk_part = nullptr;
+  // the prefill attention's key-split partials (kAttnPrefillPartBytes)
+  float* d_attn_part = nullptr;
   // split-K partials of the op-level GEMM entry (allocated on first use)
   float* gemm_ws = nullptr;
   size_t gemm_ws_bytes = 0;

@@ -92,7 +92,9 @@ __device__ __forceinline__ void issue_tile8(u32x4_t* stage, __amdgpu_buffer_rsrc
 // MFMA's B operand: contraction slot 8 G + r <-> key 32 ks2 + 4 G + r, slot 8 G + 4 + r <->
 // key 32 ks2 + 16 + 4 G + r.  (Measured and not kept: rescaling o only when some lane's max
 // grew by 2^8, behind a wave-uniform branch -- no faster.)
-template <bool MASK, int QI>
+// SPLIT: a row may have no key in any tile so far (its split lies past it): its max stays -inf and
+// its weights are 0 (the exponent's offset is then taken from a finite stand-in).
+template <bool MASK, int QI, bool SPLIT>
 __device__ __forceinline__ void softmax_tile(f32x4_t (&s)[QI][4], float (&m)[QI],
                                              float (&alpha)[QI], f32x4_t (&o)[QI][8],
                                              bf16x8_t (&pb)[QI][2], int key0, int q0, int nkeys,
@@ -115,7 +117,7 @@ __device__ __forceinline__ void softmax_tile(f32x4_t (&s)[QI][4], float (&m)[QI]
     // a query row whose keys in this tile are all masked keeps mn = m (finite after its first
     // tile, which always holds key 0)
     const float mn = fmaxf(m[qi], mt);
-    const float nb = -mn * c;
+    const float nb = -(SPLIT ? fmaxf(mn, -3.0e38f) : mn) * c;
     alpha[qi] = __builtin_amdgcn_exp2f(fmaf(m[qi], c, nb));  // m = -inf: 0
     m[qi] = mn;
 #pragma unroll
@@ -138,7 +140,12 @@ __device__ __forceinline__ void softmax_tile(f32x4_t (&s)[QI][4], float (&m)[QI]
 // QI: 16-row query blocks per wave (1 or 2); SUB: row blocks per workgroup (1: 4 waves, 2: 8
 // waves, the two halves of the workgroup's rows).  A wave whose rows end before the
 // workgroup's last tile skips that tile's work but still passes its barrier.
-template <bool PAGED, int QI, int SUB>
+// SPLIT (few query rows over many keys): the key tiles of a query block are cut into p.splits
+// runs, a workgroup each, so that the chip is full; each writes its rows' unnormalised (o, m, l)
+// in fp32, and flash_merge_kernel combines them.  200 rows at position 30000 (98.7 GFLOP): 443 us
+// unsplit, 133-138 split, 0.72 PF -- then bound as the unsplit kernel on a full chip, by the
+// softmax's issue beside the MFMAs.
+template <bool PAGED, int QI, int SUB, bool SPLIT>
 __global__ __launch_bounds__(256 * SUB, (QI == 2 && SUB == 2) ? 1 : 2) void flash_prefill_kernel(
     AttnPrefillParams p) {
   __shared__ u32x4_t lds0[2 * TC];  // ring stage 0: [K | V][key][16 chunks], 32 KiB
@@ -150,21 +157,32 @@ __global__ __launch_bounds__(256 * SUB, (QI == 2 && SUB == 2) ? 1 : 2) void flas
   const int nqb = (p.S + BQ - 1) / BQ;
   // workgroup b -> (query block, kv head): the first half of the grid takes the longest causal
   // extents in descending order, the second half the shortest in ascending order
+  // (SPLIT: the query blocks of one run of keys are neighbours on one XCD, whose L2 then holds the
+  // run for all of them: workgroup ids go round the 8 XCDs, kv head by kv head)
   const int i = blockIdx.x / kKVHeads, g = blockIdx.x % kKVHeads;
   const int half = (nqb + 1) / 2;
-  const int qb = i < half ? nqb - 1 - i : i - half;
+  const int qb = SPLIT ? i % nqb : i < half ? nqb - 1 - i : i - half;
+  const int split = SPLIT ? i / nqb : 0;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wv = __builtin_amdgcn_readfirstlane(wave);
   const int fr = lane & 15, G = lane >> 4;
   const int h = g * kGQA + (wv & 3);
   const int row0 = qb * BQ;
   const int rows = min(BQ, p.S - row0);
-  const int nkeys = p.start_pos + row0 + rows;
-  const int ntiles = (nkeys + BKEY - 1) / BKEY;
+  int nkeys = p.start_pos + row0 + rows;
+  int ntiles = (nkeys + BKEY - 1) / BKEY, t0 = 0;
+  if constexpr (SPLIT) {
+    // this split's run of tiles; keys past it read as absent (an empty run still writes l = 0)
+    const int tps = (ntiles + p.splits - 1) / p.splits;
+    t0 = min(ntiles, split * tps);
+    ntiles = min(ntiles, t0 + tps);
+    nkeys = min(nkeys, ntiles * BKEY);
+  }
   // this wave's rows (with SUB = 2 the second half may be empty in the last block)
   const int wrow0 = row0 + (wv >> 2) * BW;
   const int wrows = min(BW, p.S - wrow0);
-  const int wtiles = wrows > 0 ? (p.start_pos + wrow0 + wrows + BKEY - 1) / BKEY : 0;
+  int wtiles = wrows > 0 ? (p.start_pos + wrow0 + wrows + BKEY - 1) / BKEY : 0;
+  if constexpr (SPLIT) wtiles = min(wtiles, ntiles);
 
   const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(p.k + (size_t)g * kKVPlane), 0, nkeys * kRowBytes, kBufferFlags);
@@ -217,11 +235,11 @@ __global__ __launch_bounds__(256 * SUB, (QI == 2 && SUB == 2) ? 1 : 2) void flas
   // Paged KV: tile t's buffers are its page's rows; the page id of tile t+1 is loaded (a vector
   // load, so the loop's vmcnt wait covers it) while tile t is multiplied.
   constexpr bool paged = PAGED;
-  int pg_next = paged ? p.block_table[0] : 0;
+  int pg_next = paged ? p.block_table[SPLIT ? min(t0, max(0, ntiles - 1)) : 0] : 0;
   auto tile_rsrc = [&](int t, int page, __amdgpu_buffer_rsrc_t& tk, __amdgpu_buffer_rsrc_t& tv) {
     const bool ok = page >= 0 && page < p.n_pages;
     const size_t base = (size_t)(ok ? page : 0) * kPageElems + (size_t)g * kPageHead;
-    const int bytes = ok ? min(BKEY, nkeys - t * BKEY) * kRowBytes : 0;
+    const int bytes = ok ? max(0, min(BKEY, nkeys - t * BKEY)) * kRowBytes : 0;
     tk = __builtin_amdgcn_make_buffer_rsrc((void*)(p.k + base), 0, bytes, kBufferFlags);
     tv = __builtin_amdgcn_make_buffer_rsrc((void*)(p.v + base), 0, bytes, kBufferFlags);
   };
@@ -234,11 +252,11 @@ __global__ __launch_bounds__(256 * SUB, (QI == 2 && SUB == 2) ? 1 : 2) void flas
   };
   if constexpr (paged) {
     __amdgpu_buffer_rsrc_t tk, tv;
-    tile_rsrc(0, __builtin_amdgcn_readfirstlane(pg_next), tk, tv);
+    tile_rsrc(t0, __builtin_amdgcn_readfirstlane(pg_next), tk, tv);
     issue(lds0, tk, tv, 0);
-    pg_next = p.block_table[min(1, ntiles - 1)];
+    pg_next = p.block_table[min(t0 + 1, ntiles - 1)];
   } else {
-    issue(lds0, krs, vrs, 0);
+    issue(lds0, krs, vrs, (uint32_t)(t0 * BKEY * kRowBytes));
   }
 
   auto step = [&](int t, const u32x4_t* cur, u32x4_t* nxt) {
@@ -276,9 +294,9 @@ __global__ __launch_bounds__(256 * SUB, (QI == 2 && SUB == 2) ? 1 : 2) void flas
     // ---- online softmax; causal masking only on the tiles that reach past the wave's first query
     bf16x8_t pb[QI][2];
     if (key0 + BKEY - 1 <= p.start_pos + wrow0)
-      softmax_tile<false, QI>(s, m, alpha, o, pb, key0, p.start_pos + wrow0 + fr, nkeys, G);
+      softmax_tile<false, QI, SPLIT>(s, m, alpha, o, pb, key0, p.start_pos + wrow0 + fr, nkeys, G);
     else
-      softmax_tile<true, QI>(s, m, alpha, o, pb, key0, p.start_pos + wrow0 + fr, nkeys, G);
+      softmax_tile<true, QI, SPLIT>(s, m, alpha, o, pb, key0, p.start_pos + wrow0 + fr, nkeys, G);
 #pragma unroll
     for (int qi = 0; qi < QI; ++qi) {
       lsum[qi][0] *= alpha[qi];
@@ -304,9 +322,25 @@ __global__ __launch_bounds__(256 * SUB, (QI == 2 && SUB == 2) ? 1 : 2) void flas
       }
     }
   };
-  for (int t = 0; t < ntiles; t += 2) {
+  for (int t = t0; t < ntiles; t += 2) {
     step(t, lds0, lds1);
     if (t + 1 < ntiles) step(t + 1, lds1, lds0);
+  }
+
+  if constexpr (SPLIT) {
+    // this split's partial of its rows, [split][row][head][128] and [split][row][head](m, l)
+#pragma unroll
+    for (int qi = 0; qi < QI; ++qi) {
+      if (16 * qi + fr >= wrows) continue;
+      const size_t slot = ((size_t)split * p.S + wrow0 + 16 * qi + fr) * kQHeads + h;
+      float* dst = p.part + slot * kHeadDim + 4 * G;
+#pragma unroll
+      for (int db = 0; db < 8; ++db) *reinterpret_cast<f32x4_t*>(dst + 16 * db) = o[qi][db];
+      if (G == 0)
+        *reinterpret_cast<float2*>(p.part + (size_t)p.splits * p.S * kQHeads * kHeadDim + 2 * slot) =
+            make_float2(m[qi], lsum[qi][0]);
+    }
+    return;
   }
 
   // ---- o[qi][db][r] = O[q = wrow0 + 16 qi + fr][d = 16 db + 4 G + r] (unnormalised)
@@ -325,14 +359,80 @@ __global__ __launch_bounds__(256 * SUB, (QI == 2 && SUB == 2) ? 1 : 2) void flas
   }
 }
 
-template <int QI, int SUB>
+// Combines the p.splits partials of each (row, q head): 32 lanes each, 4 dims a lane.  A split
+// without keys for the row (l = 0) is passed over.
+__global__ __launch_bounds__(256) void flash_merge_kernel(AttnPrefillParams p) {
+  constexpr float c = 0.08838834764831845f * 1.4426950408889634f;
+  const int item = blockIdx.x * 8 + (threadIdx.x >> 5), d = (threadIdx.x & 31) * 4;
+  const size_t rows = (size_t)p.S * kQHeads;  // (S * 32 is a multiple of 8: no partial group)
+  const float2* ml = reinterpret_cast<const float2*>(p.part + p.splits * rows * kHeadDim);
+  // the splits in groups of 8, a group's loads in flight together (indices clamped to the last
+  // split); the running (M, L, o) is rescaled per group
+  float M = -INFINITY, L = 0.f;
+  f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < p.splits; s0 += 8) {
+    float2 v[8];
+    f32x4_t po[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const size_t slot = min(s0 + u, p.splits - 1) * rows + item;
+      v[u] = ml[slot];
+      po[u] = *reinterpret_cast<const f32x4_t*>(p.part + slot * kHeadDim + d);
+    }
+    float mn = M;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) mn = fmaxf(mn, v[u].x);
+    const float a = L == 0.f ? 0.f : __builtin_amdgcn_exp2f((M - mn) * c);
+    L *= a;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] *= a;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (s0 + u >= p.splits || v[u].y == 0.f) continue;
+      const float w = __builtin_amdgcn_exp2f((v[u].x - mn) * c);
+      L = fmaf(v[u].y, w, L);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = fmaf(po[u][e], w, o[e]);
+    }
+    M = mn;
+  }
+  const float inv = 1.0f / L;
+  const u32x2_t w = {pack_bf2(o[0] * inv, o[1] * inv), pack_bf2(o[2] * inv, o[3] * inv)};
+  *reinterpret_cast<u32x2_t*>(p.out + (size_t)item * kHeadDim + d) = w;
+}
+
+template <int QI, int SUB, bool SPLIT = false>
 void launch_form(const AttnPrefillParams& p, hipStream_t st) {
   const int bq = 16 * QI * SUB;
-  const dim3 grid(((p.S + bq - 1) / bq) * kKVHeads), block(256 * SUB);
+  const dim3 grid(((p.S + bq - 1) / bq) * kKVHeads * (SPLIT ? p.splits : 1)), block(256 * SUB);
   if (p.block_table)
-    hipLaunchKernelGGL((flash_prefill_kernel<true, QI, SUB>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((flash_prefill_kernel<true, QI, SUB, SPLIT>), grid, block, 0, st, p);
   else
-    hipLaunchKernelGGL((flash_prefill_kernel<false, QI, SUB>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((flash_prefill_kernel<false, QI, SUB, SPLIT>), grid, block, 0, st, p);
+  if constexpr (SPLIT)
+    hipLaunchKernelGGL(flash_merge_kernel, dim3(p.S * kQHeads / 8), dim3(256), 0, st, p);
+}
+
+// Key splits for S rows that see up to nkeys keys (1: none).  Without a split the time is the
+// longest row block's walk over its key tiles however few CUs that keeps busy: 200 rows at
+// position 30000 took 521 us on 104 workgroups, 135 in 9 splits (504 workgroups); 32 rows at 2500
+// 48 -> 17, 700 at 8000 186 -> 130.  The model, in tiles: workgroups per CU (the second costs 0.85
+// of the first) x a split's tiles + 2, plus the merge kernel's launch (4) and its partials (0.5 per
+// 64 rows and split); a split has to save 15% of it.  Within 3% of the best split count on average
+// over 1-1300 rows at 500-60000 keys; from about 1000 rows on few keys the row blocks fill the chip
+// and it answers 1.
+int attn_key_splits(int S, int nkeys) {
+  const int wgs = (S + 31) / 32 * kKVHeads, tiles = (nkeys + BKEY - 1) / BKEY;
+  const auto cost = [&](int s) {
+    const int per_cu = (wgs * s + 255) / 256;
+    return (per_cu == 1 ? 1.0 : 0.85 * per_cu) * ((double)tiles / s + 2) +
+           (s > 1 ? 4 + 0.5 / 64 * s * S : 0);
+  };
+  int best = 1;
+  double best_cost = 0.85 * cost(1);
+  for (int s = 2; s <= 32 && 2 * s <= tiles && s * S <= kAttnPrefillPartRows; ++s)
+    if (cost(s) < best_cost) best = s, best_cost = cost(s);
+  return best;
 }
 
 }  // namespace
@@ -347,7 +447,14 @@ int launch_attn_prefill(const AttnPrefillParams& p, hipStream_t st) {
   // row): measured at S = 512 / 1024 / 1536 / 2048 / 2560 / 4096, 10.8 / 20.2 / 36.2 / 55.3 /
   // 81.6 / 179.6 us, 13.3 / 23.3 / 34.1 / 45.1 / 70.3 / 161.3 us and 15.2 / 26.0 / 38.0 / 48.2 /
   // 65.9 / 148.0 us
-  if (p.S < 1280)
+  // Few rows over many keys: the 8-wave form over key splits (ahead of the split 16- and 32-row
+  // 4-wave forms from 64 rows on, 2% behind the 16-row one below).
+  const int splits = p.part ? attn_key_splits(p.S, p.start_pos + p.S) : 1;
+  if (splits > 1) {
+    AttnPrefillParams q = p;
+    q.splits = splits;
+    launch_form<1, 2, true>(q, st);
+  } else if (p.S < 1280)
     launch_form<1, 1>(p, st);
   else if (p.S < 2560)
     launch_form<1, 2>(p, st);

@@ -58,3 +58,38 @@ def test_attn_prefill_core(hip, ctx, S, start_pos):
     want = reference(q, k, v, start_pos)
     assert_close(out.float().view(S, 32, 128).cpu().numpy(), want.cpu().numpy(),
                  what=f"attn prefill core S={S} start={start_pos}")
+
+
+# key splits (few rows over many keys): runs that end inside a row block's masked tiles (33 rows
+# at 1990), a run of one ragged tile, an empty last run (16 tiles in 7 runs of 3), one row, rows
+# that do not fill a 16-row block, and the 4096 rows x splits limit (1300 x 3)
+@pytest.mark.parametrize("S,start_pos", [(1, 1000), (1, 8191), (16, 1000), (33, 1990),
+                                         (64, 4001), (200, 7992), (700, 7000), (1300, 6800)])
+def test_attn_prefill_core_key_splits(hip, ctx, S, start_pos):
+    say(f"attn_prefill_core key splits S={S} start_pos={start_pos}")
+    g = torch.Generator(device="cuda").manual_seed(2000 + S + start_pos)
+    q = (2 * torch.randn(S, 32, 128, generator=g, device="cuda")).to(torch.bfloat16)
+    k = torch.full((8, CTX, 128), 3.0e4, dtype=torch.bfloat16, device="cuda")
+    v = torch.full_like(k, 3.0e4)   # rows past the context: must not be read
+    n = start_pos + S
+    k[:, :n] = torch.randn(8, n, 128, generator=g, device="cuda").to(torch.bfloat16)
+    v[:, :n] = torch.randn(8, n, 128, generator=g, device="cuda").to(torch.bfloat16)
+    out = torch.full((S + 1, 32 * 128), 7.0, dtype=torch.bfloat16, device="cuda")
+    hip.check(hip.lib.ie_attn_prefill_core(ctx.handle, S, start_pos, P(q), P(k), P(v), P(out)))
+    # the same keys in shuffled pages
+    npg = (n + 63) // 64
+    pool = torch.full((npg, 32, 2, 8, 64, 128), 3.0e4, dtype=torch.bfloat16, device="cuda")
+    order = torch.randperm(npg, generator=g, device="cuda")
+    for kv, plane in ((k, 0), (v, 1)):
+        rows = torch.full((8, npg * 64, 128), 3.0e4, dtype=torch.bfloat16, device="cuda")
+        rows[:, :n] = kv[:, :n]
+        pool[order, 3, plane] = rows.view(8, npg, 64, 128).transpose(0, 1).contiguous()
+    paged = torch.empty(S, 32 * 128, dtype=torch.bfloat16, device="cuda")
+    hip.check(hip.lib.ie_attn_prefill_core_paged(ctx.handle, S, start_pos, P(q), P(pool), npg,
+                                                 P(order.to(torch.int32)), 3, P(paged)))
+    torch.cuda.synchronize()
+    want = reference(q, k, v, start_pos)
+    assert_close(out[:S].float().view(S, 32, 128).cpu().numpy(), want.cpu().numpy(),
+                 what=f"attn key splits S={S} start={start_pos}")
+    assert torch.equal(out[:S], paged)
+    assert bool((out[S] == 7.0).all())
