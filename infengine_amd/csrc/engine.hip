@@ -323,17 +323,13 @@ int ie_context_create(ie_context** out, int device, void* stream) {
   size_t zeroed = 0;
   do {
     c->stream = stream_of(stream);
-    if (hipStreamCreateWithFlags(&c->capture, hipStreamNonBlocking) != hipSuccess) {
-      rc = IE_ERR_HIP;
-      break;
-    }
     // one device allocation (the counters, slots and params, zeroed below, first) and one pinned
     // one: each allocation is ~40-100 us of a context's creation
     const size_t cnt = align256(kNumCounters * sizeof(unsigned int)),
                  slots = align256(kNumSlots * kSlotStride * sizeof(unsigned long long)),
                  params = align256(64 * sizeof(int));
     zeroed = cnt + slots + params;
-    if (hipMalloc(&c->arena, zeroed + align256(kSkPartBytes) + kAttnPrefillPartBytes) != hipSuccess ||
+    if (hipMalloc(&c->arena, zeroed + kSkPartBytes) != hipSuccess ||
         hipHostMalloc(&c->h_params, 128 * sizeof(int), hipHostMallocMapped) != hipSuccess) {
       rc = IE_ERR_OOM;
       break;
@@ -343,7 +339,6 @@ int ie_context_create(ie_context** out, int device, void* stream) {
     c->d_slots = reinterpret_cast<unsigned long long*>(base + cnt);
     c->d_params = reinterpret_cast<int*>(base + cnt + slots);
     c->d_sk_part = reinterpret_cast<float*>(base + zeroed);
-    c->d_attn_part = reinterpret_cast<float*>(base + zeroed + align256(kSkPartBytes));
     c->h_token = c->h_params + 64;
     if (hipHostGetDevicePointer(reinterpret_cast<void**>(&c->h_token_dev), c->h_token, 0) !=
         hipSuccess) {
@@ -380,6 +375,7 @@ int ie_context_destroy(ie_context* c) {
   if (c->h_params) (void)hipHostFree(c->h_params);
   if (c->capture) (void)hipStreamDestroy(c->capture);
   if (c->gemm_ws) (void)hipFree(c->gemm_ws);
+  if (c->attn_part) (void)hipFree(c->attn_part);
   delete c;
   return IE_OK;
 }
@@ -464,6 +460,7 @@ int decode_step_impl(Context* c, const ie_model_weights* weights, int seq_len, i
       // captured on the private stream (capture is not allowed on the legacy
       // default stream), replayed on the context's stream
       hipGraph_t g = nullptr;
+      if (!c->capture) IE_CHECK_HIP(hipStreamCreateWithFlags(&c->capture, hipStreamNonBlocking));
       IE_CHECK_HIP(hipStreamBeginCapture(c->capture, hipStreamCaptureModeThreadLocal));
       const int rc = enqueue_decode(c, c->capture, *weights, seq_len, tokenid_buff, data_buffer,
                                     attn_buffer, output_distr, output_token, workspace, kv_cache,
@@ -582,6 +579,38 @@ void skinny_split(Context* c, int epi, GemmParams& g, float* part) {
   g.sk_cnt = c->d_counters + kCntSkinny;
 }
 
+// Room for the attention's key-split partials: the attention workspace past q/k/v and the
+// rotated q (the split-K partials there are dead once q/k/v are reduced).
+void attn_part_room(AttnPrefillParams& a, char* wsb, int S) {
+  a.part = reinterpret_cast<float*>(wsb + prefill_attn_bytes(S));
+  const size_t rows = (ie_attn_workspace_size(S) - prefill_attn_bytes(S)) / (kAttnPrefillPartRow * sizeof(float));
+  a.part_rows = (int)std::min<size_t>(rows, kAttnPrefillPartRows);
+}
+
+// The op-level entries have no workspace: a context-owned scratch, grown on first use.  A call
+// recorded into a graph by the caller cannot allocate: without a large enough scratch it runs
+// unsplit.
+int attn_part_scratch(Context* c, AttnPrefillParams& a) {
+  if (a.S < 1 || a.start_pos < 0) return IE_OK;  // (the launcher refuses them)
+  const int splits = attn_prefill_splits(a.S, a.start_pos + a.S, kAttnPrefillPartRows);
+  const int rows = splits > 1 ? splits * a.S : 0;
+  if (rows > c->attn_part_rows) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    // (the legacy default stream cannot be captured)
+    if (c->stream) IE_CHECK_HIP(hipStreamIsCapturing(c->stream, &cap));
+    if (cap != hipStreamCaptureStatusNone) return IE_OK;
+    IE_CHECK_HIP(hipStreamSynchronize(c->stream));
+    if (c->attn_part) IE_CHECK_HIP(hipFree(c->attn_part));
+    c->attn_part = nullptr;
+    c->attn_part_rows = 0;
+    IE_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&c->attn_part), rows * kAttnPrefillPartRow * sizeof(float)));
+    c->attn_part_rows = rows;
+  }
+  a.part = c->attn_part;
+  a.part_rows = c->attn_part_rows;
+  return IE_OK;
+}
+
 // aux_ready: aux_buffer already holds this layer's input RMSNorm of data_buffer (written by
 // the previous layer's down-projection reduction).  next_norm_w: the next layer's input norm
 // weight, or nullptr; *aux_next is set when this layer left that norm in aux_buffer (the down
@@ -651,8 +680,8 @@ int prefill_layer(Context* c, hipStream_t st, const ie_model_weights& W, int l, 
                              data_buffer + (size_t)(S - 1) * kHidden, dw.attn1, dw, kvl, nullptr,
                              start_pos + S, block_table, n_pages);
   }
-  AttnPrefillParams a{qrot, kvl, vpl, attn_buffer, S, start_pos, block_table, n_pages,
-                      c->d_attn_part};
+  AttnPrefillParams a{qrot, kvl, vpl, attn_buffer, S, start_pos, block_table, n_pages};
+  attn_part_room(a, wsb, S);
   IE_TRY(launch_attn_prefill(a, st));
   GemmParams o{};
   o.x = attn_buffer;
@@ -994,6 +1023,7 @@ int batched_step(ie_context* c, const ie_model_weights* weights, int batch, cons
         slot->exec = nullptr;
       }
       hipGraph_t g = nullptr;
+      if (!c->capture) IE_CHECK_HIP(hipStreamCreateWithFlags(&c->capture, hipStreamNonBlocking));
       IE_CHECK_HIP(hipStreamBeginCapture(c->capture, hipStreamCaptureModeThreadLocal));
       const int rc = enqueue_batched(c, c->capture, *weights, batch, len_class, tokenid_buffs,
                                      tokens_stride, data_buffer, attn_buffer, output_distr,
@@ -1312,7 +1342,8 @@ int ie_attn_prefill_core(ie_context* c, int seq_len, int start_pos, const ie_bf1
                          const ie_bf16* d_k, const ie_bf16* d_v, ie_bf16* d_out) {
   CTX_OK(c);
   IE_REQUIRE(d_q && d_k && d_v && d_out, "attn_prefill_core: null pointer");
-  AttnPrefillParams a{d_q, d_k, d_v, d_out, seq_len, start_pos, nullptr, 0, c->d_attn_part};
+  AttnPrefillParams a{d_q, d_k, d_v, d_out, seq_len, start_pos};
+  IE_TRY(attn_part_scratch(c, a));
   return launch_attn_prefill(a, c->stream);
 }
 
@@ -1325,7 +1356,8 @@ int ie_attn_prefill_core_paged(ie_context* c, int seq_len, int start_pos, const 
              "attn_prefill_core_paged: n_pages %d, layer %d", n_pages, layer);
   const uint16_t* kl = static_cast<const uint16_t*>(kv_pages) + (size_t)layer * kPageLayer;
   AttnPrefillParams a{d_q, kl, kl + (size_t)kKVHeads * kPageHead, d_out, seq_len, start_pos,
-                      block_table, n_pages, c->d_attn_part};
+                      block_table, n_pages};
+  IE_TRY(attn_part_scratch(c, a));
   return launch_attn_prefill(a, c->stream);
 }
 
@@ -1442,8 +1474,8 @@ int ie_attn(ie_context* c, const float* d_rope_cos, const float* d_rope_sin, int
   IE_TRY(launch_qkv_rope_scatter(S, 0, qkv, d_rope_cos, d_rope_sin, qrot, kvl,
                                  kvl + (size_t)kKVHeads * kKVPlane, nullptr, 0, st));
   uint16_t* att = qkv;  // the projection is dead once scattered
-  AttnPrefillParams a{qrot, kvl, kvl + (size_t)kKVHeads * kKVPlane, att, S, 0, nullptr, 0,
-                      c->d_attn_part};
+  AttnPrefillParams a{qrot, kvl, kvl + (size_t)kKVHeads * kKVPlane, att, S, 0};
+  attn_part_room(a, wsb, S);
   IE_TRY(launch_attn_prefill(a, st));
   GemmParams o{};
   o.x = att;

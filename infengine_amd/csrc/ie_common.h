@@ -241,7 +241,7 @@ constexpr double kSynthStd = 37837.22627754049;
 struct Context {
   int device = 0;
   hipStream_t stream = nullptr;    // nullptr = the legacy default stream
-  hipStream_t capture = nullptr;   // private stream the decode graph is captured on
+  hipStream_t capture = nullptr;   // private stream the graphs are captured on (made for the first)
   void* arena = nullptr;           // the device allocation behind the d_ pointers below
   unsigned int* d_counters = nullptr;       // self-resetting last-block counters
   unsigned long long* d_slots = nullptr;    // 64-bit reduction slots (argmax)
@@ -264,8 +264,9 @@ struct Context {
   unsigned long long bgraph_tick = 0;
   // the skinny GEMM's K-half partials (kSkPartBytes) for launches outside the batched step
   float* d_sk_part = nullptr;
-  // the prefill attention's key-split partials (kAttnPrefillPartBytes)
-  float* d_attn_part = nullptr;
+  // key-split partials of the op-level prefill attention entries (allocated on first use)
+  float* attn_part = nullptr;
+  int attn_part_rows = 0;
   // split-K partials of the op-level GEMM entry (allocated on first use)
   float* gemm_ws = nullptr;
   size_t gemm_ws_bytes = 0;

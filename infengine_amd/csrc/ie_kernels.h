@@ -253,14 +253,16 @@ struct AttnPrefillParams {
   int start_pos;       // absolute position of q row 0 (keys 0..start_pos+S-1)
   const int* block_table = nullptr;  // paged KV: page of each 64-key block; k / v = the layer's
   int n_pages = 0;                   // head-0 K / V planes in page 0 (ids outside: empty)
-  float* part = nullptr;             // kAttnPrefillPartBytes for the key splits' partials
+  float* part = nullptr;             // room for the key splits' partials: part_rows rows x
+  int part_rows = 0;                 // splits of kAttnPrefillPartRow floats (0: no splits)
   int splits = 1;                    // set by the launcher
 };
-// Rows x key splits of a prefill attention with few rows over many keys (launch_attn_prefill);
-// each takes 128 + 2 floats per q head.
+// Prefill attention with few rows over many keys: fp32 partials per row and key split (128 + 2
+// floats per q head), at most kAttnPrefillPartRows of them.
 constexpr int kAttnPrefillPartRows = 4096;
-constexpr size_t kAttnPrefillPartBytes =
-    (size_t)kAttnPrefillPartRows * kQHeads * (kHeadDim + 2) * sizeof(float);
+constexpr size_t kAttnPrefillPartRow = (size_t)kQHeads * (kHeadDim + 2);
+// The key splits (1: none) for S rows over nkeys keys with room for part_rows partial rows.
+int attn_prefill_splits(int S, int nkeys, int part_rows);
 int launch_attn_prefill(const AttnPrefillParams& p, hipStream_t st);
 
 }  // namespace ie

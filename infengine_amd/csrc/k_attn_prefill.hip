@@ -29,6 +29,8 @@
 // bounds), so the masked tail never multiplies garbage.  Workgroups are issued longest causal
 // extent first, paired so that the two a CU holds sum to about the mean.  Output rows are
 // [s][h][d] (the attn_permute.cu:15-31 layout), bf16.
+#include <algorithm>
+
 #include "ie_kernels.h"
 
 namespace ie {
@@ -413,7 +415,9 @@ void launch_form(const AttnPrefillParams& p, hipStream_t st) {
     hipLaunchKernelGGL(flash_merge_kernel, dim3(p.S * kQHeads / 8), dim3(256), 0, st, p);
 }
 
-// Key splits for S rows that see up to nkeys keys (1: none).  Without a split the time is the
+}  // namespace
+
+// Without a split the time is the
 // longest row block's walk over its key tiles however few CUs that keeps busy: 200 rows at
 // position 30000 took 521 us on 104 workgroups, 135 in 9 splits (504 workgroups); 32 rows at 2500
 // 48 -> 17, 700 at 8000 186 -> 130.  The model, in tiles: workgroups per CU (the second costs 0.85
@@ -421,7 +425,7 @@ void launch_form(const AttnPrefillParams& p, hipStream_t st) {
 // 64 rows and split); a split has to save 15% of it.  Within 3% of the best split count on average
 // over 1-1300 rows at 500-60000 keys; from about 1000 rows on few keys the row blocks fill the chip
 // and it answers 1.
-int attn_key_splits(int S, int nkeys) {
+int attn_prefill_splits(int S, int nkeys, int part_rows) {
   const int wgs = (S + 31) / 32 * kKVHeads, tiles = (nkeys + BKEY - 1) / BKEY;
   const auto cost = [&](int s) {
     const int per_cu = (wgs * s + 255) / 256;
@@ -430,12 +434,10 @@ int attn_key_splits(int S, int nkeys) {
   };
   int best = 1;
   double best_cost = 0.85 * cost(1);
-  for (int s = 2; s <= 32 && 2 * s <= tiles && s * S <= kAttnPrefillPartRows; ++s)
+  for (int s = 2; s <= 32 && 2 * s <= tiles && s * S <= std::min(part_rows, kAttnPrefillPartRows); ++s)
     if (cost(s) < best_cost) best = s, best_cost = cost(s);
   return best;
 }
-
-}  // namespace
 
 int launch_attn_prefill(const AttnPrefillParams& p, hipStream_t st) {
   // the reference-layout planes hold kMaxCtx rows; pages reach kMaxLongCtx positions
@@ -449,7 +451,7 @@ int launch_attn_prefill(const AttnPrefillParams& p, hipStream_t st) {
   // 65.9 / 148.0 us
   // Few rows over many keys: the 8-wave form over key splits (ahead of the split 16- and 32-row
   // 4-wave forms from 64 rows on, 2% behind the 16-row one below).
-  const int splits = p.part ? attn_key_splits(p.S, p.start_pos + p.S) : 1;
+  const int splits = attn_prefill_splits(p.S, p.start_pos + p.S, p.part ? p.part_rows : 0);
   if (splits > 1) {
     AttnPrefillParams q = p;
     q.splits = splits;

@@ -10,11 +10,11 @@
 //            against all X rows; K split into fp32 partial planes summed by a split reduction
 //            (RoPE + K/V write, residual + RMSNorm, SwiGLU or bf16), or unsplit with the
 //            epilogue in the kernel.
-//   to 1024  gemm_wide_kernel (128-row X tiles, direct-to-LDS rings) split over K, with the
-//            same reductions, where the best tiling is one round that leaves half the chip idle.
-//   beyond   launch_tiled: the ping-pong gemm_pp_kernel / gemm_pp_dual_kernel on 256 x 256,
-//            256 x 128 and 192 x 256 tiles, chosen by rounds of 256 tiles; the 128 x 128
-//            gemm_kernel described next takes what the larger tiles do not fit.
+//   beyond   launch_tiled: the ping-pong gemm_pp_kernel on the tile shape (128 or 256 W rows by
+//            128 - 256 X rows; 192 for the fused QKV) and K split that a fitted cost model
+//            picks (plan_tiles), or gemm_pp_dual_kernel; gemm_wide_kernel (direct-to-LDS ring) is
+//            the same products' A/B form, and the 128 x 128 gemm_kernel described next takes
+//            operands off 16 bytes.
 //
 // Tile: 128 W-rows x 128 X-rows x 64 k per workgroup of 4 waves; each wave owns
 // a 64 x 64 block as 4 x 4 v_mfma_f32_16x16x32_bf16 tiles.  The MFMA computes
@@ -51,7 +51,6 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 constexpr int BM = 128;  // X rows per tile
 constexpr int BN = 128;  // W rows per tile
 constexpr int BK = 64;
-constexpr int kWideMinRows = 128;  // smallest M the wide-tile kernels are considered for
 
 template <int EPI>
 __device__ __forceinline__ const uint16_t* w_row(const GemmParams& p, int ntile, int r) {
@@ -204,16 +203,13 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams p, int m_tiles) {
 }
 
 // ---------------------------------------------------------------------------
-// Wide-tile kernel for M >= 128 (prefill): 256 (or 192) W rows x 128 (or 256) X rows x 64 k
-// per workgroup; each wave owns 128 (96) W rows x 64 X rows as 4 (3) x 2 tiles of
-// v_mfma_f32_32x32x16_bf16 (128 fp32 accumulators per lane).  The 256 x 128 tile runs 8 waves
-// as two k-groups (each takes two of a k-step's four k16 sub-steps for the whole tile, and the
-// groups' sums are added through LDS at the end): two waves per SIMD where one tile's worth
-// of 128 x 64 blocks would leave one.
+// DMA-ring kernel (ie_tune_gemm_schedule 0 and 1): 256 W rows x 256 X rows x 64 k per workgroup
+// of 8 waves; each wave owns 128 W rows x 64 X rows as 4 x 2 tiles of
+// v_mfma_f32_32x32x16_bf16 (128 fp32 accumulators per lane).
 //
 // Operands reach LDS by direct-to-LDS buffer loads (buffer_load_dwordx4 ... lds:
-// lane i of a wave writes 16 bytes at LDS base + 16 i), through a 3-stage ring
-// of 48 KiB stages, so the loads for k-step kt+2 are in flight while k-step kt
+// lane i of a wave writes 16 bytes at LDS base + 16 i), through a 2-stage ring
+// of 64 KiB stages, so the loads for k-step kt+1 are in flight while k-step kt
 // is multiplied.  Each load covers 8 tile rows through its own buffer descriptor
 // (base = the group's first row, size = the rows left in its matrix), so rows
 // past the end of a matrix read as zero, and the k offset is a scalar operand.
@@ -225,9 +221,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams p, int m_tiles) {
 // 16-byte bank groups for both a 64-bank and a 128-bank LDS.
 //
 // The loads are counted by vmcnt; the compiler does not track them, so every
-// k-step starts with an explicit "s_waitcnt vmcnt(N); s_barrier": N = the loads
-// of the one younger stage still allowed in flight (12 per wave), 0 on the last
-// step.  No other vector-memory instruction is issued inside the loop.
+// k-step's last sub-step starts with an explicit "s_waitcnt vmcnt(0); s_barrier".
+// No other vector-memory instruction is issued inside the loop.
 namespace wide {
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
@@ -235,23 +230,16 @@ typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int kBufferFlags = 0x00020000;  // buffer descriptor word 3 (raw 32-bit access)
 
-// Tile geometry: BN (256 or 192) W rows x BM (128 or 256) X rows x BK (32 or 64) k, in a
-// ring of STAGES LDS stages.  Every wave owns BN / 2 W rows x 64 X rows (NI = BN / 64 blocks
-// of 32 W rows), so a workgroup has NW = 2 * BM / 64 waves (4 or 8).
-template <int BM_, int BK_, int STAGES_, int BN_ = 256, int KG_ = 1>
+// Tile geometry: BN W rows x BM X rows x BK k, in a ring of STAGES LDS stages.  Every wave owns
+// BN / 2 W rows x 64 X rows (NI = BN / 64 blocks of 32 W rows).
 struct Cfg {
-  static constexpr int BN = BN_;
+  static constexpr int BN = 256, BM = 256, BK = 64, STAGES = 2;
   static constexpr int WTN = BN / 2;                 // W rows per wave
   static constexpr int NI = WTN / 32;                // 32-row MFMA blocks per wave
   static constexpr int NT = 2 * NI;                  // MFMAs per k16 sub-step
-  static constexpr int BM = BM_;
-  static constexpr int BK = BK_;
-  static constexpr int STAGES = STAGES_;
   static constexpr int WM = BM / 64;                 // waves along X
-  static constexpr int NW = 2 * WM;                  // waves per k-group (one tile's worth)
-  static constexpr int KG = KG_;                     // k-groups: waves splitting each k-step
-  static constexpr int NWT = NW * KG;                // waves per workgroup
-  static constexpr int THREADS = 64 * NWT;
+  static constexpr int NW = 2 * WM;                  // waves
+  static constexpr int THREADS = 64 * NW;
   static constexpr int CPR = BK / 8;                 // 16-byte chunks per tile row
   static constexpr int RPL = 64 / CPR;               // tile rows per wave-wide load
   static constexpr int W_CHUNKS = BN * CPR;
@@ -261,21 +249,12 @@ struct Cfg {
   static constexpr int X_LOADS = X_CHUNKS / THREADS;
   static constexpr int LOADS = W_LOADS + X_LOADS;
   static constexpr int KSUB = BK / 16;               // MFMA k16 sub-steps per stage
-  static constexpr int KSUBW = KSUB / KG;            // sub-steps per wave per k-step
-  // With a ring of 3 or more stages a stage's loads are spread over a wave's KSUBW sub-steps (the
-  // last of k-step kt and the first KSUBW-1 of k-step kt+1) instead of all issued in one.
-  static constexpr bool SPREAD = STAGES >= 3;
-  static_assert(BK == 32 || BK == 64, "BK");
-  static_assert(BN == 256 || BN == 192, "BN");
-  static_assert(KSUBW % 2 == 0, "fragment double buffer alternates within a k-step");
+  static_assert(KSUB % 2 == 0, "fragment double buffer alternates within a k-step");
   static_assert(W_CHUNKS % THREADS == 0 && X_CHUNKS % THREADS == 0, "loads per thread");
   static_assert(STAGES * STAGE * 16 <= 160 * 1024, "LDS");
   // Chunk slot s of row r holds global chunk s ^ swz(r): the 16 (or 32) consecutive rows one
   // ds_read_b128 phase touches fall in distinct 16-byte bank groups (64- or 128-bank LDS).
-  static __device__ __forceinline__ int swz(int r) {
-    if constexpr (CPR == 8) return ((r >> 1) & 7) ^ ((r >> 4) & 1);
-    else return ((r >> 2) & 3) ^ ((r >> 4) & 1);
-  }
+  static __device__ __forceinline__ int swz(int r) { return ((r >> 1) & 7) ^ ((r >> 4) & 1); }
 };
 
 // Buffer descriptor for the `rows` W rows starting at tile-local row r (all in one matrix).
@@ -332,27 +311,25 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t x_group(const GemmParams& p, i
 // Direct-to-LDS loads of k-step kt into ring slot `stage`.  (Plain device functions, not
 // lambdas: a lambda around the amdgcn builtin inside a kernel template stops the host pass
 // from emitting the kernel's launch stub.)
-template <class C>
+using C = Cfg;
 __device__ __forceinline__ void issue_load(u32x4_t* lds, const __amdgpu_buffer_rsrc_t* rsrc,
                                            const uint32_t* voff, int wv, int kt, int stage, int j) {
   const bool is_w = j < C::W_LOADS;
-  const int g = wv + C::NWT * (is_w ? j : j - C::W_LOADS);
+  const int g = wv + C::NW * (is_w ? j : j - C::W_LOADS);
   u32x4_t* dst = &lds[stage * C::STAGE + (is_w ? 0 : C::W_CHUNKS) + g * 64];
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc[j], (lds_void*)dst, 16, voff[j],
                                            (uint32_t)(kt * C::BK * 2), 0, 0);
 }
 
-template <class C>
 __device__ __forceinline__ void issue_stage(u32x4_t* lds, const __amdgpu_buffer_rsrc_t* rsrc,
                                             const uint32_t* voff, int wv, int kt, int stage) {
 #pragma unroll
-  for (int j = 0; j < C::LOADS; ++j) issue_load<C>(lds, rsrc, voff, wv, kt, stage, j);
+  for (int j = 0; j < C::LOADS; ++j) issue_load(lds, rsrc, voff, wv, kt, stage, j);
 }
 
 // Operand fragment n (0..NI+1) of a k16 sub-step, in the order the sub-step's MFMAs first use
 // them: X0 W0 X1 W1 W2 (W3).  Lane l supplies tile row base + l%32 at k chunk ch (2*kk + l/32,
 // swizzled).
-template <class C>
 __device__ __forceinline__ void read_frag(const u32x4_t* src, int a_row, int b_row, int ch, int n,
                                           bf16x8_t* af, bf16x8_t* bfr) {
   if (n == 0 || n == 2) {
@@ -373,34 +350,23 @@ __device__ __forceinline__ void store16(uint16_t* dst, uint2 lo, uint2 hi, bool 
   }
 }
 
-// Wait until at most n stages of loads (n * loads per stage) are in flight and this wave's
-// LDS reads have returned, then barrier: after it the stage is visible to every wave and no
-// wave still reads the ring slot the next loads overwrite.
-template <int LOADS, int N>
-__device__ __forceinline__ void wait_stage_n(int n) {
-  if constexpr (N < 0) {
-    return;
-  } else {
-    if (n == N) {
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N * LOADS) : "memory");
-      return;
-    }
-    wait_stage_n<LOADS, N - 1>(n);
-  }
+// Wait until every load in flight has landed and this wave's LDS reads have returned, then
+// barrier: after it the stage is visible to every wave and no wave still reads the ring slot the
+// next loads overwrite.
+__device__ __forceinline__ void wait_stage() {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 // Logical tile of workgroup b.  Workgroups are dealt round-robin to the 8 XCDs, so each XCD
 // is handed a contiguous range of W tiles (n_tiles / 8); inside it the range is swept in
-// groups of MAPG W tiles x all X tiles, X-tile-major within a group, so the 32 tiles an XCD
-// runs at once share W rows and X rows in its L2.
-template <int MAPG>
+// one W tile x all X tiles at a time, so the 32 tiles an XCD runs at once share W rows and X rows
+// in its L2.
 __device__ __forceinline__ void tile_of(int b, int nb, int m_tiles, int& mtile, int& ntile) {
   const int n_tiles = nb / m_tiles;
-  if (nb % 8 == 0 && n_tiles % (8 * MAPG) == 0) {
+  if (nb % 8 == 0 && n_tiles % 8 == 0) {
     const int x = b % 8, local = b / 8;
-    const int grp = local / (MAPG * m_tiles), within = local % (MAPG * m_tiles);
-    ntile = x * (n_tiles / 8) + grp * MAPG + within % MAPG;
-    mtile = within / MAPG;
+    ntile = x * (n_tiles / 8) + local / m_tiles;
+    mtile = local % m_tiles;
   } else {
     const int t = (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;
     mtile = t % m_tiles;
@@ -408,76 +374,48 @@ __device__ __forceinline__ void tile_of(int b, int nb, int m_tiles, int& mtile, 
   }
 }
 
-// One k-step on ring slot kt % STAGES, as 4 (BK 64) or 2 (BK 32) MFMA sub-steps of k16 (with
-// KG = 2 k-groups a wave runs the KSUBW = KSUB / 2 sub-steps from kk0 = its group's half).  The
-// fragments of the next sub-step are read one after each MFMA of the current one, so that their
-// issue hides under the MFMAs (the scheduling fences keep this order: left alone the scheduler
-// groups the reads and moves each just before its use).  The last sub-step waits for stage
-// kt+1 and reads its first fragments, so no k-step starts on an LDS latency.
-// Loads: with NEW the last sub-step refills slot kt % STAGES (free once every wave has passed
-// that sub-step's barrier) with stage kt+STAGES -- all of it, or with SPREAD its first share;
-// with REST (SPREAD) sub-step kk < KSUBW-1 issues share kk+1 of stage kt-1+STAGES.  Loads are
-// issued in stage order either way, so the wait for stage kt+1 allows exactly the younger
-// stages issued so far: min(STAGES-2, KT-2-kt) of them.
-template <class C, bool NEW, bool REST>
+// One k-step on ring slot kt % STAGES, as 4 MFMA sub-steps of k16.  The fragments of the next
+// sub-step are read one after each MFMA of the current one, so that their issue hides under the
+// MFMAs (the scheduling fences keep this order: left alone the scheduler groups the reads and
+// moves each just before its use).  The last sub-step waits for stage kt+1 and reads its first
+// fragments, so no k-step starts on an LDS latency; with NEW it refills slot kt % STAGES (free
+// once every wave has passed that sub-step's barrier) with stage kt+STAGES.
+template <bool NEW>
 __device__ __forceinline__ void k_step(f32x16_t (&acc)[C::NI][2], bf16x8_t (&af)[2][C::NI],
                                        bf16x8_t (&bfr)[2][2], u32x4_t* lds,
                                        const __amdgpu_buffer_rsrc_t* rsrc, const uint32_t* voff,
-                                       int wv, int a_row, int b_row, int fh, int fs, int kk0,
-                                       int kt, int KT) {
+                                       int wv, int a_row, int b_row, int fh, int fs, int kt, int KT) {
   const u32x4_t* st = &lds[(kt % C::STAGES) * C::STAGE];
   const u32x4_t* nst = &lds[((kt + 1) % C::STAGES) * C::STAGE];
 #pragma unroll
-  for (int kk = 0; kk < C::KSUBW; ++kk) {
+  for (int kk = 0; kk < C::KSUB; ++kk) {
     const int cur = kk & 1;
-    const bool last = kk + 1 == C::KSUBW;
+    const bool last = kk + 1 == C::KSUB;
     const bool rd = !last || kt + 1 < KT;
-    // stage kt+1 must have landed; the younger stages issued so far may stay in flight
-    if (last && rd)
-      wait_stage_n<C::LOADS, C::STAGES - 2>(NEW ? C::STAGES - 2 : min(C::STAGES - 2, KT - 2 - kt));
+    if (last && rd) wait_stage();
     const u32x4_t* src = last ? nst : st;
-    const int ch = (2 * (kk0 + (last ? 0 : kk + 1)) + fh) ^ fs;
-    // loads of this sub-step: share `sh` of stage `ls` into ring slot `slot`
-    const bool issue = last ? NEW : (C::SPREAD && REST);
-    const int sh = !C::SPREAD ? 0 : last ? 0 : kk + 1;
-    const int ls = last ? kt + C::STAGES : kt - 1 + C::STAGES;
-    const int slot = ls % C::STAGES;
+    const int ch = (2 * (last ? 0 : kk + 1) + fh) ^ fs;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < C::NT; ++t) {
       acc[t / 2][t % 2] =
           __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cur][t / 2], bfr[cur][t % 2], acc[t / 2][t % 2], 0, 0, 0);
-      if (rd && t < C::NI + 2) read_frag<C>(src, a_row, b_row, ch, t, af[cur ^ 1], bfr[cur ^ 1]);
-      if (issue) {
-        constexpr int SHARES = C::SPREAD ? C::KSUBW : 1;
-        constexpr int PER = (C::LOADS + SHARES - 1) / SHARES;  // loads per share (last may be short)
+      if (rd && t < C::NI + 2) read_frag(src, a_row, b_row, ch, t, af[cur ^ 1], bfr[cur ^ 1]);
+      if (last && NEW) {
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-          const int j = sh * PER + i;
-          if (j < C::LOADS && i * C::NT / PER == t) issue_load<C>(lds, rsrc, voff, wv, ls, slot, j);
-        }
+        for (int j = 0; j < C::LOADS; ++j)
+          if (j * C::NT / C::LOADS == t)
+            issue_load(lds, rsrc, voff, wv, kt + C::STAGES, kt % C::STAGES, j);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
 
-// Output-tile swizzle: 8-byte unit u of row r (of `upr` units) sits at slot swz_out(u, r).  The
-// 32 rows one write instruction touches land in distinct 8-byte bank pairs: within a 32-unit
-// group u ^ (r % 32) is a permutation of the rows; in the 16-unit tail of a 48-unit row the rows'
-// alternating 16-unit offset (48 r mod 32) supplies the fifth bit.
-template <int UPR>
-__device__ __forceinline__ int swz_out(int u, int r) {
-  if constexpr (UPR == 48) {
-    if (u >= 32) return 32 + ((u - 32) ^ ((r & 14) | ((r >> 4) & 1)));
-  }
-  return u ^ (r & 31);
-}
+// Output-tile swizzle: 8-byte unit u of row r (32 or 64 units a row) sits at slot
+// u ^ (r % 32): the 32 rows one write instruction touches land in distinct 8-byte bank pairs.
+__device__ __forceinline__ int swz_out(int u, int r) { return u ^ (r & 31); }
 
-// The epilogue of a 256- or 192-row W tile: wave (wn, wm) of k-group kg holds accumulator element
-// 4*g + q of tile (i, j) = W row wn*WTN + 32*i + 8*g + 4*(lane/32) + q, X row m0 + wm*64 + 32*j +
-// lane%32 (k-group 0 holds the sums).  fp32 results go straight to global memory; bf16 ones are
-// staged through the LDS ring as a [BM][OUTN] tile and stored as whole row segments.
 // Copy-out of a bf16 output tile staged in LDS as [BM][UPR] 8-byte units (unit u of row r at
 // swz(u, r)): 16 bytes (8 columns) per thread, consecutive threads along a row; the residual
 // epilogue adds the tile to y.
@@ -512,17 +450,17 @@ __device__ __forceinline__ void tile_copy_out(const GemmParams& p, const uint2* 
   }
 }
 
-// Copy-out of the prefill QKV + RoPE tile staged in LDS as [256][48] 8-byte units: unit u < 24
+// Copy-out of the prefill QKV + RoPE tile staged in LDS as [BM][48] 8-byte units: unit u < 24
 // holds the first halves of pairs 96 ntile + 4u .. +3 (pair P: head P / 64, dims P % 64 and
 // P % 64 + 64), unit 24 + u their second halves.  Each thread takes 4 pairs of one row: RoPE at
 // position start_pos + m on q and k (the scatter kernel's pairing and roundings, on the same
 // bf16 values), q to y [M][32][128], k and v to this layer's cache planes (or pages).
-template <int THREADS, class SW>
+template <int THREADS, int BM, class SW>
 __device__ __forceinline__ void rope_copy_out(const GemmParams& p, const uint2* ot, int m0,
                                               int ntile, int tid, SW swz) {
   constexpr int UPR = 48, QUADS = 24;
 #pragma unroll 4
-  for (int it = tid; it < 256 * QUADS; it += THREADS) {
+  for (int it = tid; it < BM * QUADS; it += THREADS) {
     const int r = it / QUADS, u = it % QUADS;
     const int m = m0 + r;
     if (m >= p.M) continue;
@@ -566,20 +504,21 @@ __device__ __forceinline__ void rope_copy_out(const GemmParams& p, const uint2* 
   }
 }
 
-template <int UPR>
 struct WideOutSwz {
-  __device__ __forceinline__ int operator()(int u, int r) const { return swz_out<UPR>(u, r); }
+  __device__ __forceinline__ int operator()(int u, int r) const { return swz_out(u, r); }
 };
 
-template <class C, int EPI>
+// The epilogue of the ring kernel's tile: wave (wn, wm) holds accumulator element 4*g + q of tile
+// (i, j) = W row wn*WTN + 32*i + 8*g + 4*(lane/32) + q, X row m0 + wm*64 + 32*j + lane%32.  fp32
+// results go straight to global memory; bf16 ones are staged through the LDS ring as a [BM][OUTN]
+// tile and stored as whole row segments.
+template <int EPI>
 __device__ __forceinline__ void wide_epilogue(const GemmParams& p, f32x16_t (&acc)[C::NI][2],
                                               u32x4_t* lds, uint16_t* y, float* yf, int m0,
-                                              int ntile, int kg, int wn, int wm, int lane,
-                                              int tid) {
+                                              int ntile, int wn, int wm, int lane, int tid) {
   constexpr int BM = C::BM, BN = C::BN, STAGES = C::STAGES;
   const int fr = lane & 31, fh = lane >> 5;
   if constexpr (EPI == kGemmF32) {
-    if (kg != 0) return;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int m = m0 + wm * 64 + j * 32 + fr;
@@ -607,7 +546,6 @@ __device__ __forceinline__ void wide_epilogue(const GemmParams& p, f32x16_t (&ac
     __syncthreads();  // every wave is done reading the ring
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      if (kg != 0) break;
       const int r = wm * 64 + j * 32 + fr;
       if constexpr (EPI == kGemmSwiglu) {
 #pragma unroll
@@ -627,7 +565,7 @@ __device__ __forceinline__ void wide_epilogue(const GemmParams& p, f32x16_t (&ac
               o[q] = pack_bf2(v[0], v[1]);
             }
             const int u = (2 * wn + i / 2) * 8 + 2 * g + fh;
-            ot[r * UPR + swz_out<UPR>(u, r)] = make_uint2(o[0], o[1]);
+            ot[r * UPR + swz_out(u, r)] = make_uint2(o[0], o[1]);
           }
       } else {
 #pragma unroll
@@ -635,41 +573,36 @@ __device__ __forceinline__ void wide_epilogue(const GemmParams& p, f32x16_t (&ac
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
             const int u = wn * (C::WTN / 4) + i * 8 + 2 * g + fh;
-            ot[r * UPR + swz_out<UPR>(u, r)] = make_uint2(pack_bf2(acc[i][j][4 * g], acc[i][j][4 * g + 1]),
+            ot[r * UPR + swz_out(u, r)] = make_uint2(pack_bf2(acc[i][j][4 * g], acc[i][j][4 * g + 1]),
                                                 pack_bf2(acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]));
           }
       }
     }
     __syncthreads();
-    tile_copy_out<C::THREADS, BM, UPR, EPI>(p, ot, y, m0, ntile * OUTN, tid, WideOutSwz<UPR>{});
+    tile_copy_out<C::THREADS, BM, UPR, EPI>(p, ot, y, m0, ntile * OUTN, tid, WideOutSwz{});
   }
 }
 
-template <int EPI, int BM, int BK, int STAGES, int MAPG, int BN, int KG>
-__global__ __launch_bounds__(2 * BM * KG) __attribute__((amdgpu_waves_per_eu(BM * KG / 128, BM * KG / 128)))
+template <int EPI>
+__global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_wide_kernel(GemmParams p, int m_tiles) {
-  using C = Cfg<BM, BK, STAGES, BN, KG>;
-  static_assert(C::THREADS == 2 * BM * KG, "launch bounds");
-  static_assert(EPI != kGemmSwiglu || BN == 256, "SwiGLU tiles are 256 W rows");
+  constexpr int BM = C::BM, BK = C::BK, STAGES = C::STAGES;
+  static_assert(C::THREADS == 512, "two waves per SIMD");
   __shared__ u32x4_t lds[STAGES * C::STAGE];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // wave = kg * NW + wt: k-group kg runs sub-steps kk0 .. kk0+KSUBW-1 of every k-step for the
-  // 128 x 64 block wt of the tile; with KG = 2 the groups' sums are added at the end
-  const int kg = wave / C::NW, wt = wave % C::NW;
-  const int wn = wt / C::WM, wm = wt % C::WM;
-  const int kk0 = __builtin_amdgcn_readfirstlane(kg * C::KSUBW);
+  const int wn = wave / C::WM, wm = wave % C::WM;
   // split K: workgroup b takes k-steps [split * KT, (split + 1) * KT) of tile b % tiles and
   // writes its fp32 partial product to partial plane `split` of yf
   const int nsplit = max(1, p.k_splits);
   const int nb = gridDim.x / nsplit, split = blockIdx.x / nb;
   int mtile, ntile;
-  tile_of<MAPG>(blockIdx.x - split * nb, nb, m_tiles, mtile, ntile);
+  tile_of(blockIdx.x - split * nb, nb, m_tiles, mtile, ntile);
   const int m0 = mtile * BM;
   const int KT = p.K / BK / nsplit;
   const int k0 = split * KT * BK;
 
-  // load j of this wave covers tile rows RPL*g .. RPL*g+RPL-1 with g = wave + NWT*j;
+  // load j of this wave covers tile rows RPL*g .. RPL*g+RPL-1 with g = wave + NW*j;
   // lane i fills LDS slot (row RPL*g + i/CPR, chunk i%CPR) from global chunk (i%CPR) ^ swz(row)
   const int wv = __builtin_amdgcn_readfirstlane(wave);
   __amdgpu_buffer_rsrc_t rsrc[C::LOADS];
@@ -677,7 +610,7 @@ void gemm_wide_kernel(GemmParams p, int m_tiles) {
 #pragma unroll
   for (int j = 0; j < C::LOADS; ++j) {
     const bool is_w = j < C::W_LOADS;
-    const int g = wv + C::NWT * (is_w ? j : j - C::W_LOADS);
+    const int g = wv + C::NW * (is_w ? j : j - C::W_LOADS);
     rsrc[j] = is_w ? w_group<EPI, C::BN>(p, ntile, g * C::RPL, k0) : x_group(p, m0, g * C::RPL, k0);
     const int rl = lane / C::CPR, c = (lane % C::CPR) ^ C::swz(g * C::RPL + rl);
     voff[j] = (uint32_t)((rl * p.K + c * 8) * 2);
@@ -701,60 +634,23 @@ void gemm_wide_kernel(GemmParams p, int m_tiles) {
   float* const yf = p.yf + (size_t)split * p.M * p.ldy;
   asm volatile("" ::"s"(y), "s"(yf), "s"(p.ldy), "s"(p.M), "s"(p.N));
 
-#pragma unroll
-  for (int s0 = 0; s0 < STAGES - 1; ++s0)
-    if (s0 < KT) issue_stage<C>(lds, rsrc, voff, wv, s0, s0);
-  // stage 0 landed; stage STAGES-1 goes to the last ring slot, which no wave reads yet
-  wait_stage_n<C::LOADS, STAGES - 2>(min(STAGES - 2, KT - 1));
-  if (STAGES - 1 < KT) issue_stage<C>(lds, rsrc, voff, wv, STAGES - 1, STAGES - 1);
+  issue_stage(lds, rsrc, voff, wv, 0, 0);
+  wait_stage();  // stage 0 landed; stage 1 goes to the slot no wave reads yet
+  if (STAGES - 1 < KT) issue_stage(lds, rsrc, voff, wv, 1, 1);
   bf16x8_t af[2][C::NI], bfr[2][2];
 #pragma unroll
-  for (int n = 0; n < C::NI + 2; ++n) read_frag<C>(lds, a_row, b_row, (2 * kk0 + fh) ^ fs, n, af[0], bfr[0]);
+  for (int n = 0; n < C::NI + 2; ++n) read_frag(lds, a_row, b_row, fh ^ fs, n, af[0], bfr[0]);
   int kt = 0;
-  // stage STAGES-1 was issued whole above, so k-step 0 issues no remaining shares
-  if (STAGES < KT) {
-    k_step<C, true, false>(acc, af, bfr, lds, rsrc, voff, wv, a_row, b_row, fh, fs, kk0, kt, KT);
-    ++kt;
-  }
   for (; kt + STAGES < KT; ++kt)
-    k_step<C, true, true>(acc, af, bfr, lds, rsrc, voff, wv, a_row, b_row, fh, fs, kk0, kt, KT);
-  if (C::SPREAD && kt >= 1 && kt < KT) {  // the shares of stage KT-1 still to issue
-    k_step<C, false, true>(acc, af, bfr, lds, rsrc, voff, wv, a_row, b_row, fh, fs, kk0, kt, KT);
-    ++kt;
-  }
+    k_step<true>(acc, af, bfr, lds, rsrc, voff, wv, a_row, b_row, fh, fs, kt, KT);
   for (; kt < KT; ++kt)
-    k_step<C, false, false>(acc, af, bfr, lds, rsrc, voff, wv, a_row, b_row, fh, fs, kk0, kt, KT);
+    k_step<false>(acc, af, bfr, lds, rsrc, voff, wv, a_row, b_row, fh, fs, kt, KT);
 
-  if constexpr (C::KG == 2) {
-    // k-group 1 hands its sums to k-group 0 through the ring: block wt's 128 fp32 per lane,
-    // lane-contiguous (conflict-free)
-    static_assert(C::NW * C::NI * 2 * 16 * 64 * 4 <= STAGES * C::STAGE * 16, "reduction fits the ring");
-    float* red = reinterpret_cast<float*>(lds) + (size_t)wt * (C::NI * 2 * 16 * 64) + lane;
-    __syncthreads();  // every wave is done reading the ring
-    if (kg == 1) {
-#pragma unroll
-      for (int i = 0; i < C::NI; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) red[((i * 2 + j) * 16 + e) * 64] = acc[i][j][e];
-    }
-    __syncthreads();
-    if (kg == 0) {
-#pragma unroll
-      for (int i = 0; i < C::NI; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc[i][j][e] += red[((i * 2 + j) * 16 + e) * 64];
-    }
-  }
-
-  wide_epilogue<C, EPI>(p, acc, lds, y, yf, m0, ntile, kg, wn, wm, lane, tid);
+  wide_epilogue<EPI>(p, acc, lds, y, yf, m0, ntile, wn, wm, lane, tid);
 }
 
 // ---------------------------------------------------------------------------
-// Ping-pong kernel for the 256 x 256 (or 192 W x 256 X) tile on v_mfma_f32_16x16x32_bf16.
+// Ping-pong kernel on v_mfma_f32_16x16x32_bf16, described for its 256 x 256 tile.
 //
 // The part runs these GEMMs power-limited: the same kernels on all-zero operands run 25-35%
 // faster, and on random data a stream of 32x32x16 MFMAs alone (no LDS reads, loads or
@@ -790,17 +686,17 @@ void gemm_wide_kernel(GemmParams p, int m_tiles) {
 // offsets are base ^ (ks << 6) plus immediates of 2048 bytes per block.
 namespace pp {
 
-// Tile: BN W rows x BM X rows x 64 k per stage.  BM = 256 (KG = 1): the two wave groups split the
-// W rows.  BM = 128 (KG = 2): each group owns the whole tile and multiplies one k32 half of every
-// stage, and group 1's sums are added to group 0's through LDS at the end.
-template <int BN_, int BM_, int NW_ = 3>
+// Tile: BN W rows x BM X rows x 64 k per stage.  The two wave groups split the W rows, and the 4
+// waves of a group are 4 / WX along W by WX along X.
+template <int BN_, int BM_, int NW_ = 3, int WX_ = 4>
 struct PC {
   static constexpr int BN = BN_, BM = BM_, BK = 64;
-  static constexpr int KG = BM == 256 ? 1 : 2;
-  static constexpr int KS = 2 / KG;            // k32 sub-steps a wave multiplies per stage
-  static constexpr int WTN = BN / 2;           // W rows per wave
-  static constexpr int NA = WTN / 16;          // 16-row W blocks per wave (8 or 6)
-  static constexpr int NB = 4;                 // 16-row X blocks per wave (64 X rows)
+  static constexpr int WX = WX_;               // waves of a group along X
+  static constexpr int KS = 2;                 // k32 sub-steps per stage
+  static constexpr int WTN = BN / 2 * WX / 4;  // W rows per wave
+  static constexpr int WTM = BM / WX;          // X rows per wave
+  static constexpr int NA = WTN / 16;          // 16-row W blocks per wave
+  static constexpr int NB = WTM / 16;          // 16-row X blocks per wave
   static constexpr int CPR = 8;                // 16-byte chunks per tile row
   static constexpr int W_CHUNKS = BN * CPR;    // one stage's W half
   static constexpr int X_CHUNKS = BM * CPR;    // one stage's X half
@@ -814,7 +710,7 @@ struct PC {
   static constexpr int NX = (NW * W_CHUNKS + 3 * X_CHUNKS) * 16 <= 160 * 1024 ? 3 : 2;
   static constexpr int X_BASE = NW * W_CHUNKS;  // chunk offset of X slot 0
   static constexpr int TOTAL = NW * W_CHUNKS + NX * X_CHUNKS;
-  static_assert(BM == 256 || (BM == 128 && BN == 256), "tile shapes");
+  static_assert(WTN % 16 == 0 && WTM % 16 == 0 && BM % 32 == 0 && BN % 32 == 0, "tile shapes");
   static_assert(NW == 3 || NW == 4, "W ring depth");
   static_assert(TOTAL * 16 <= 160 * 1024, "LDS");
   static __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
@@ -826,10 +722,10 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // first chunk plus the wave's first 8-row group).
 template <int NL>
 __device__ __forceinline__ void issue(u32x4_t* lds, const __amdgpu_buffer_rsrc_t* rs,
-                                      const uint32_t* vo, int base, int kt) {
+                                      uint32_t vo, int base, int kt) {
 #pragma unroll
   for (int j = 0; j < NL; ++j)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs[j], (lds_void*)&lds[base + 256 * j], 16, vo[j],
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs[j], (lds_void*)&lds[base + 256 * j], 16, vo,
                                              (uint32_t)(kt * 128), 0, 0);
 }
 
@@ -859,7 +755,7 @@ __device__ __forceinline__ void read(const u32x4_t* lds, uint32_t sa, uint32_t s
 template <class C, int NL, bool DMA>
 __device__ __forceinline__ void compute(f32x4_t (&acc)[C::NA][C::NB], const bf16x8_t (&fa)[C::KS][C::NA],
                                         const bf16x8_t (&fb)[C::KS][C::NB], u32x4_t* lds,
-                                        const __amdgpu_buffer_rsrc_t* rs, const uint32_t* vo,
+                                        const __amdgpu_buffer_rsrc_t* rs, uint32_t vo,
                                         int base, int kt) {
   asm volatile("s_setprio 2" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
@@ -872,7 +768,7 @@ __device__ __forceinline__ void compute(f32x4_t (&acc)[C::NA][C::NB], const bf16
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[ks][i], fb[ks][j], acc[i][j], 0, 0, 0);
         const int n = (ks * C::NA + i) * C::NB + j;
         if (DMA && n < NL)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs[n], (lds_void*)&lds[base + 256 * n], 16, vo[n],
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs[n], (lds_void*)&lds[base + 256 * n], 16, vo,
                                                    (uint32_t)(kt * 128), 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -894,40 +790,40 @@ struct OutSwz {
   }
 };
 
-// Tile b of the nb tiles of p (the LDS ring: at least PC<BN, BM, NWR>::TOTAL chunks).
-template <int EPI, int BN, int BM, int NWR>
-__device__ __forceinline__ void pp_tile(const GemmParams& p, int m_tiles, int b, int nb,
+// Tile b of the nb tiles of p (the LDS ring: at least C::TOTAL chunks).  kGemmF32: k-steps
+// split KT .. of the tile's K (KT = K / 64 / k_splits), its fp32 sums to partial plane `split`.
+template <int EPI, class C>
+__device__ __forceinline__ void pp_tile(const GemmParams& p, int m_tiles, int b, int nb, int split,
                                         u32x4_t* lds) {
-  using C = PC<BN, BM, NWR>;
+  constexpr int BN = C::BN, BM = C::BM;
   constexpr int NA = C::NA, NB = C::NB, WL = C::WL, XL = C::XL, PL = C::PL, KS = C::KS;
-  static_assert(EPI == kGemmBf16 || EPI == kGemmResid || EPI == kGemmSwiglu || EPI == kGemmQkvRope,
-                "bf16 epilogues");
-  static_assert(EPI != kGemmSwiglu || BN == 256, "SwiGLU tiles are 256 W rows");
-  static_assert(EPI != kGemmQkvRope || (BN == 192 && BM == 256), "QKV + RoPE: 192 x 256 tiles");
+  static_assert(EPI != kGemmSwiglu || C::WTN % 64 == 0, "SwiGLU waves hold [32 gate | 32 up] rows");
+  static_assert(EPI != kGemmQkvRope || BN == 192, "QKV + RoPE: 192 W rows");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wv >> 2, gw = wv & 3;
-  // the wave's output block: W rows wn * WTN .., X rows wm * 64 ..; with KG = 2 its k32 half grp
-  const int wn = C::KG == 1 ? grp : gw >> 1, wm = C::KG == 1 ? gw : gw & 1;
+  // the wave's output block: W rows wn * WTN .., X rows wm * WTM ..
+  const int wn = grp * (4 / C::WX) + gw / C::WX, wm = gw % C::WX;
   int mtile, ntile;
-  tile_of<1>(b, nb, m_tiles, mtile, ntile);
+  tile_of(b, nb, m_tiles, mtile, ntile);
   const int m0 = mtile * BM;
-  const int KT = p.K / 64;
+  const int KT = EPI == kGemmF32 ? p.K / 64 / p.k_splits : p.K / 64;
+  const int k0 = EPI == kGemmF32 ? split * KT * 64 : 0;
 
   // this wave's share of a stage: 8-row groups gw + 4 j of its half (W or X); lane i fills LDS
-  // slot (row 8 g + i / 8, chunk i % 8) from global chunk (i % 8) ^ swz(row)
+  // slot (row 8 g + i / 8, chunk i % 8) from global chunk (i % 8) ^ swz(row), the same for every
+  // j (rows 32 apart)
   __amdgpu_buffer_rsrc_t rs[PL];
-  uint32_t vo[PL];
 #pragma unroll
   for (int j = 0; j < PL; ++j) {
     const int g = gw + 4 * j;
-    rs[j] = grp == 0 ? w_group<EPI, BN>(p, ntile, min(g, BN / 8 - 1) * 8) : x_group(p, m0, g * 8);
-    const int rl = lane / 8, c = (lane % 8) ^ C::swz(g * 8 + rl);
-    vo[j] = (uint32_t)((rl * p.K + c * 8) * 2);
+    rs[j] = grp == 0 ? w_group<EPI, BN>(p, ntile, min(g, BN / 8 - 1) * 8, k0)
+                     : x_group(p, m0, g * 8, k0);
   }
+  const int rl = lane / 8;
+  const uint32_t vo = (uint32_t)((rl * p.K + ((lane % 8) ^ C::swz(gw * 8 + rl)) * 8) * 2);
   const int dst0 = (grp == 0 ? 0 : C::X_BASE) + gw * 64;  // the wave's first row group, slot 0
-  const int slot_chunks = grp == 0 ? C::W_CHUNKS : C::X_CHUNKS;
 
   f32x4_t acc[NA][NB];
 #pragma unroll
@@ -938,13 +834,14 @@ __device__ __forceinline__ void pp_tile(const GemmParams& p, int m_tiles, int b,
   // fragment byte offsets within a stage (ks = 0, block 0): lane l reads row base + l % 16 at
   // chunk (l / 16) ^ swz(row)
   const int fr = lane & 15, fq = lane >> 4;
-  const uint32_t chunk0 = (uint32_t)((fq ^ C::swz(fr)) * 16) ^ (C::KG == 2 ? (uint32_t)(grp << 6) : 0u);
+  const uint32_t chunk0 = (uint32_t)((fq ^ C::swz(fr)) * 16);
   const uint32_t aA = (uint32_t)((wn * C::WTN + fr) * C::CPR * 16) + chunk0;
-  const uint32_t aB = (uint32_t)((wm * 64 + fr) * C::CPR * 16) + chunk0;
+  const uint32_t aB = (uint32_t)((wm * C::WTM + fr) * C::CPR * 16) + chunk0;
   bf16x8_t fa[KS][NA], fb[KS][NB];
 
   uint16_t* const y = p.y;
-  asm volatile("" ::"s"(y), "s"(p.ldy), "s"(p.M), "s"(p.N));
+  float* const yf = p.yf + (size_t)split * p.M * p.ldy;
+  asm volatile("" ::"s"(y), "s"(yf), "s"(p.ldy), "s"(p.M), "s"(p.N));
 
   // stage k's W half lives in W slot k % NW, its X half in X slot k % NX.  The wait that ends
   // phase 2k+1 leaves in flight only this wave's loads of stages issued after k+1.
@@ -1008,33 +905,22 @@ __device__ __forceinline__ void pp_tile(const GemmParams& p, int m_tiles, int b,
       sx = sx + 1 == NX ? 0 : sx + 1;
     }
   }
-  (void)slot_chunks;
 
-  // ---- epilogue: acc[i][j][r] = D[W row wn*WTN + 16 i + 4 (lane/16) + r][X row wm*64 + 16 j +
-  //      lane%16]; staged in the ring as [256][OUTN] bf16 (8-byte units), then stored as rows
-  if constexpr (C::KG == 2) {
-    // group 1 hands its sums to group 0 through the ring, half the W blocks at a time (a lane's
-    // 16-byte accumulators lane-contiguous: conflict-free)
-    constexpr int HALF = NA / 2 * NB;
-    static_assert(4 * HALF * 64 * 16 <= C::TOTAL * 16, "reduction fits the ring");
-    f32x4_t* red = reinterpret_cast<f32x4_t*>(lds) + (size_t)gw * HALF * 64 + lane;
+  // ---- epilogue: acc[i][j][r] = D[W row wn*WTN + 16 i + 4 (lane/16) + r][X row wm*WTM + 16 j +
+  //      lane%16]; staged in the ring as [BM][OUTN] bf16 (8-byte units), then stored as rows
+  if constexpr (EPI == kGemmF32) {
+    // a lane's 4 columns of one row; 4 lanes and the next block's 4 make a line
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      __syncthreads();  // the ring (or the previous half) is free
-      if (grp == 1) {
+    for (int j = 0; j < NB; ++j) {
+      const int m = m0 + wm * C::WTM + 16 * j + fr;
 #pragma unroll
-        for (int i = 0; i < NA / 2; ++i)
-#pragma unroll
-          for (int j = 0; j < NB; ++j) red[(i * NB + j) * 64] = acc[h * NA / 2 + i][j];
-      }
-      __syncthreads();
-      if (grp == 0) {
-#pragma unroll
-        for (int i = 0; i < NA / 2; ++i)
-#pragma unroll
-          for (int j = 0; j < NB; ++j) acc[h * NA / 2 + i][j] += red[(i * NB + j) * 64];
+      for (int i = 0; i < NA; ++i) {
+        const int n = ntile * BN + wn * C::WTN + 16 * i + 4 * fq;
+        if (m < p.M && n < p.N)
+          *reinterpret_cast<f32x4_t*>(yf + (size_t)m * p.ldy + n) = acc[i][j];
       }
     }
+    return;
   }
   constexpr int OUTN = (EPI == kGemmSwiglu) ? BN / 2 : BN;
   constexpr int UPR = OUTN / 4;
@@ -1044,8 +930,7 @@ __device__ __forceinline__ void pp_tile(const GemmParams& p, int m_tiles, int b,
   __syncthreads();  // every wave is done reading the ring
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
-    if (C::KG == 2 && grp != 0) break;
-    const int r = wm * 64 + 16 * j + fr;
+    const int r = wm * C::WTM + 16 * j + fr;
     if constexpr (EPI == kGemmSwiglu) {
       // W rows of the wave: [32 gate | 32 up] x 2, so block i (gate) pairs with i + 2 (up)
 #pragma unroll
@@ -1076,30 +961,34 @@ __device__ __forceinline__ void pp_tile(const GemmParams& p, int m_tiles, int b,
     }
   }
   __syncthreads();
-  if constexpr (EPI == kGemmQkvRope) rope_copy_out<512>(p, ot, m0, ntile, tid, swz);
+  if constexpr (EPI == kGemmQkvRope) rope_copy_out<512, BM>(p, ot, m0, ntile, tid, swz);
   else tile_copy_out<512, BM, UPR, EPI>(p, ot, y, m0, ntile * OUTN, tid, swz);
 }
 
-template <int EPI, int BN, int BM, int NWR>
+template <int EPI, int BN, int BM, int NWR, int WX>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_pp_kernel(GemmParams p, int m_tiles) {
-  __shared__ u32x4_t lds[PC<BN, BM, NWR>::TOTAL];
-  pp_tile<EPI, BN, BM, NWR>(p, m_tiles, blockIdx.x, gridDim.x, lds);
+  using C = PC<BN, BM, NWR, WX>;
+  __shared__ u32x4_t lds[C::TOTAL];
+  const int nb = EPI == kGemmF32 ? gridDim.x / p.k_splits : gridDim.x;
+  const int split = EPI == kGemmF32 ? blockIdx.x / nb : 0;
+  pp_tile<EPI, C>(p, m_tiles, blockIdx.x - split * nb, nb, split, lds);
 }
 
-// Two column ranges of one product in one launch: workgroups 0 .. nb1-1 take the BM1-row X
-// tiles of p1, the rest the BM2-row tiles of p2 (gate/up at S = 2048: three rounds of 256 x 256
+// Two column ranges of one product in one launch: workgroups 0 .. nb1-1 take 256 x 256 tiles of
+// p1, the rest 256 x 128 tiles of p2 (gate/up at S = 2048: three rounds of 256 x 256
 // tiles, then the last 2048 columns as 256 x 128 tiles, each starting on a CU as soon as the CU's
 // third big tile ends instead of after a kernel boundary).
-template <int EPI, int BN, int BM1, int BM2>
+template <int EPI>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_pp_dual_kernel(GemmParams p1, int m_tiles1, int nb1, GemmParams p2, int m_tiles2) {
-  constexpr int T1 = PC<BN, BM1, 3>::TOTAL, T2 = PC<BN, BM2, 3>::TOTAL;
-  __shared__ u32x4_t lds[T1 > T2 ? T1 : T2];
+  using C1 = PC<256, 256, 3, 2>;
+  using C2 = PC<256, 128, 3, 2>;
+  __shared__ u32x4_t lds[C1::TOTAL > C2::TOTAL ? C1::TOTAL : C2::TOTAL];
   if ((int)blockIdx.x < nb1)
-    pp_tile<EPI, BN, BM1, 3>(p1, m_tiles1, blockIdx.x, nb1, lds);
+    pp_tile<EPI, C1>(p1, m_tiles1, blockIdx.x, nb1, 0, lds);
   else
-    pp_tile<EPI, BN, BM2, 3>(p2, m_tiles2, blockIdx.x - nb1, gridDim.x - nb1, lds);
+    pp_tile<EPI, C2>(p2, m_tiles2, blockIdx.x - nb1, gridDim.x - nb1, 0, lds);
 }
 
 }  // namespace pp
@@ -1304,26 +1193,28 @@ __global__ __launch_bounds__(WR * 4) void gemm_mid_kernel(GemmParams p, int n_ti
 
 }  // namespace wide
 
-template <int EPI, int BM = 128, int BK = 64, int STAGES = 3, int MAPG = 1, int WBN = 256, int KG = 1>
+template <int EPI>
 int launch_wide(const GemmParams& p, hipStream_t st) {
-  const int m_tiles = (p.M + BM - 1) / BM;
-  const int n_tiles = (EPI == kGemmSwiglu) ? (p.N + 127) / 128 : (p.N + WBN - 1) / WBN;
+  const int m_tiles = (p.M + wide::C::BM - 1) / wide::C::BM;
+  const int n_tiles = (EPI == kGemmSwiglu) ? (p.N + 127) / 128 : (p.N + wide::C::BN - 1) / wide::C::BN;
   const long long blocks = (long long)m_tiles * n_tiles * std::max(1, p.k_splits);
   IE_REQUIRE(blocks <= 0x7fffffff, "gemm: too many tiles");
-  hipLaunchKernelGGL((wide::gemm_wide_kernel<EPI, BM, BK, STAGES, MAPG, WBN, KG>), dim3((unsigned)blocks),
-                     dim3(wide::Cfg<BM, BK, STAGES, WBN, KG>::THREADS), 0, st, p, m_tiles);
+  hipLaunchKernelGGL((wide::gemm_wide_kernel<EPI>), dim3((unsigned)blocks), dim3(wide::C::THREADS),
+                     0, st, p, m_tiles);
   IE_CHECK_LAUNCH();
   return IE_OK;
 }
 
-template <int EPI, int WBN, int XBM = 256, int NW = 3>
+template <int EPI, int WBN, int XBM = 256, int NW = 3, int WX = 4>
 int launch_pp(const GemmParams& p, hipStream_t st) {
   const int m_tiles = (p.M + XBM - 1) / XBM;
   const int n_tiles = (EPI == kGemmSwiglu) ? (p.N + WBN / 2 - 1) / (WBN / 2) : (p.N + WBN - 1) / WBN;
-  const long long blocks = (long long)m_tiles * n_tiles;
-  IE_REQUIRE(blocks <= 0x7fffffff && p.k_splits <= 1, "gemm: ping-pong tiles");
-  hipLaunchKernelGGL((wide::pp::gemm_pp_kernel<EPI, WBN, XBM, NW>), dim3((unsigned)blocks), dim3(512), 0,
-                     st, p, m_tiles);
+  const long long blocks = (long long)m_tiles * n_tiles * (EPI == kGemmF32 ? p.k_splits : 1);
+  IE_REQUIRE(blocks <= 0x7fffffff && (EPI == kGemmF32 ? p.k_splits >= 1 && p.K / 64 % p.k_splits == 0
+                                                      : p.k_splits <= 1),
+             "gemm: ping-pong tiles");
+  hipLaunchKernelGGL((wide::pp::gemm_pp_kernel<EPI, WBN, XBM, NW, WX>), dim3((unsigned)blocks),
+                     dim3(512), 0, st, p, m_tiles);
   IE_CHECK_LAUNCH();
   return IE_OK;
 }
@@ -1336,7 +1227,7 @@ int launch_pp_dual(const GemmParams& head, const GemmParams& tail, hipStream_t s
   const long long b1 = (long long)m1 * n1, b2 = (long long)m2 * n2;
   IE_REQUIRE(b1 + b2 <= 0x7fffffff && head.k_splits <= 1 && tail.k_splits <= 1,
              "gemm: ping-pong tiles");
-  hipLaunchKernelGGL((wide::pp::gemm_pp_dual_kernel<EPI, 256, 256, 128>), dim3((unsigned)(b1 + b2)),
+  hipLaunchKernelGGL((wide::pp::gemm_pp_dual_kernel<EPI>), dim3((unsigned)(b1 + b2)),
                      dim3(512), 0, st, head, m1, (int)b1, tail, m2);
   IE_CHECK_LAUNCH();
   return IE_OK;
@@ -1354,96 +1245,115 @@ int launch_e(const GemmParams& p, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------------------
-// Tile shape by a cost model: time = rounds of workgroups over the 256 CUs x the time of one
-// tile at the measured per-CU rate of that shape (256x256 and 192x256: 1085, 256x128: 900,
-// 128x128: 750 TFLOP/s over the chip at full occupancy).  Big tiles win when they fill the
-// chip; at small S the 128 x 128 tile keeps more CUs busy.  192 W rows x 256 X rows gives
-// exactly 256 tiles for the QKV projection at S = 2048 (N = 6144).
-enum { kTileSmall, kTileWide, kTileBig, kTileBig192, kTileKinds };
+// Tile shapes of the ping-pong kernel: W rows x X rows, waves of a group along X, and the time of
+// one 64-k step of one tile in us (below).  SwiGLU needs waves of whole [32 gate | 32 up] groups;
+// 192 W rows are 96 RoPE pairs (the fused QKV epilogue).
+struct TileKind {
+  int bn, bm, wx;
+  double step;
+};
+constexpr TileKind kTiles[] = {
+    {128, 128, 4, 0.535}, {128, 160, 2, 0.606}, {128, 192, 4, 0.661}, {128, 224, 2, 0.742},
+    {128, 256, 4, 0.828}, {256, 160, 2, 0.995}, {256, 192, 2, 1.127}, {256, 224, 2, 1.277},
+    {256, 256, 2, 1.431}, {192, 128, 4, 0.738}, {192, 192, 4, 0.921}, {192, 256, 4, 1.135},
+};
+constexpr int kTileKinds = sizeof(kTiles) / sizeof(kTiles[0]);
+constexpr int kTileBig = 8, kTileRope0 = 9, kTileRopeBig = 11;
+constexpr double kStep256x128 = 0.85;  // the dual launch's tail tile
 
-// Kernel of the bf16 wide tiles: 0 = the DMA-ring wide kernels; 1 = the ping-pong kernel for
-// the 256-row X tiles; 2 (default) = the ping-pong kernel for those and for the 128-row X tiles;
-// 3 = as 2 with 4 W ring slots (2 X slots) on the 256 x 128 and 192 x 256 tiles.
-// Outputs are bit-identical across all (same per-accumulator MFMA order).
+// Kernel of the tiles past 128 rows: 0 = the DMA-ring kernel; 1 = the ping-pong kernel for the
+// 256-row X tiles; 2 (default) = the ping-pong kernel; 3 = as 2 with 4 W ring slots (2 X slots) on
+// the 192 x 256 tiles.  Outputs are bit-identical across all: the same K splits, and the same MFMA
+// order in every accumulator whatever the tile.
 int g_gemm_schedule = 2;
 
-struct TileKind {
-  int tm, tn, tn_swiglu;  // X rows, output columns (plain / SwiGLU) per tile
-  double unit;            // relative time of one tile
-};
-constexpr TileKind kTiles[kTileKinds] = {
-    {128, 128, 64, 128.0 * 128 / 750.0},
-    {128, 256, 128, 256.0 * 128 / 900.0},
-    {256, 256, 128, 256.0 * 256 / 1085.0},
-    {256, 192, 0, 192.0 * 256 / 1085.0},
+// A product's tile shape and K splits by the least modelled time.
+struct TilePlan {
+  int kind = -1, splits = 1;
+  double us = 1e30;
 };
 
-bool tile_ok(int kind, int epi, const GemmParams& p) {
-  if (kind == kTileSmall) return true;
-  if (p.M < kWideMinRows) return false;
-  if (kind == kTileWide) return true;
-  if (epi == kGemmF32) return false;
-  return kind == kTileBig || epi != kGemmSwiglu;
+// QKV projection as a product of its own or fused: its unsplit tiles are the 192-row ones, so that
+// both forms take the same plan (and give the same bits).
+bool rope_product(int epi, const GemmParams& p) {
+  return epi == kGemmQkvRope || (epi == kGemmBf16 && p.n0 < p.N);
 }
 
-long long tile_count(int kind, int epi, int M, int N) {
-  const TileKind& t = kTiles[kind];
-  const int tn = epi == kGemmSwiglu ? t.tn_swiglu : t.tn;
-  return (long long)((M + t.tm - 1) / t.tm) * ((N + tn - 1) / tn);
+// Time of one tile with kt k-steps, `wgs` workgroups in the launch (or of one round of it).
+double tile_us(int bn, int bm, double step, double kt, double wgs) {
+  const double idle = wgs < 256 ? 1 - wgs / 256 : 0;
+  return kt * step * (1 - 0.28 * idle) + 3.95 + 4.18 * bn * bm / 65536;
 }
 
-double tile_cost(int kind, int epi, int M, int N) {
-  return (double)((tile_count(kind, epi, M, N) + 255) / 256) * kTiles[kind].unit;
+// Model (us), fitted to 78 measured shapes (the four layer products at 130 .. 6000 rows, weights
+// from HBM, 16 tile shapes x their K splits; 6% rms, and the shape it picks is 1% off the best
+// measured one on average, 12% at most):
+//   launch 1.4 + rounds x (k-steps x step + 3.95 + 4.18 x tile / 64 Ki)
+// a step 28% faster on an empty chip than on a full one; past one round 0.71 of the time goes
+// with whole rounds, 0.29 with the tiles; K splits add 3.2 + 0.245 per MB of fp32 partials; the
+// weights stream at 3.5 TB/s at best beside the products.  What follows an unsplit residual product
+// as a launch of its own (the RMSNorm, which the split reduction runs) counts too.
+// Before, tiles were 256 x 256, 256 x 128 or 192 x 256 (and 128 x 128 with an older kernel), K
+// split up to 1024 rows only: 640 rows 201 -> 134 us (gate/up), 117 -> 77 (down), 1200 rows down
+// 189 -> 125, 6000 rows down 661 -> 551.
+TilePlan plan_tiles(int epi, const GemmParams& p) {
+  const bool sw = epi == kGemmSwiglu, rope = rope_product(epi, p);
+  const int kt = p.K / 64;
+  const bool can_split = p.split_ws && !sw && epi != kGemmF32 && p.N % 8 == 0 && p.ldy % 8 == 0;
+  const double plane = (double)p.M * p.N * 4;
+  const double weights = (double)p.N * p.K * (sw ? 4 : 2) / 3.5e6;
+  TilePlan best;
+  for (int k = 0; k < kTileKinds; ++k) {
+    const TileKind& t = kTiles[k];
+    if (sw && (t.bn / 2 * t.wx / 4) % 64 != 0) continue;
+    if (!rope && t.bn == 192) continue;
+    const long long tiles =
+        (long long)((p.M + t.bm - 1) / t.bm) * ((p.N + (sw ? t.bn / 2 : t.bn) - 1) / (sw ? t.bn / 2 : t.bn));
+    for (int s = 1; s <= 16; ++s) {
+      if (s > 1 && (!can_split || kt % s != 0 || tiles * s > 512 || t.bn == 192 ||
+                    s * plane > (double)p.split_ws_bytes))
+        continue;
+      if (s == 1 && rope && t.bn != 192) continue;
+      const double wgs = (double)tiles * s;
+      const double rounds = wgs <= 256 ? 1 : 0.71 * ((tiles * s + 255) / 256) + 0.29 * wgs / 256;
+      double us = std::max(rounds * tile_us(t.bn, t.bm, t.step, (double)kt / s, wgs), weights) + 1.4;
+      if (s > 1) us += 3.2 + 0.245e-6 * s * plane;
+      else if (epi == kGemmResid) us += 2 + 0.0021 * p.M;
+      if (us < best.us) best = {k, s, us};
+    }
+  }
+  return best;
 }
 
-int launch_kind(int kind, int epi, const GemmParams& p, hipStream_t st) {
-  if (g_gemm_schedule == 3 && kind == kTileWide && epi != kGemmF32) {
-    switch (epi) {
-      case kGemmBf16: return launch_pp<kGemmBf16, 256, 128, 4>(p, st);
-      case kGemmResid: return launch_pp<kGemmResid, 256, 128, 4>(p, st);
-      case kGemmSwiglu: return launch_pp<kGemmSwiglu, 256, 128, 4>(p, st);
+// The plan's product by the schedule's kernel (kGemmF32: p.k_splits partial planes).
+template <int EPI>
+int launch_kind(int kind, const GemmParams& p, hipStream_t st) {
+  if (g_gemm_schedule == 0 || (g_gemm_schedule == 1 && kTiles[kind].bm != 256)) {
+    if constexpr (EPI != kGemmQkvRope) return launch_wide<EPI>(p, st);
+  }
+  constexpr bool sw = EPI == kGemmSwiglu;
+  if constexpr (EPI == kGemmBf16 || EPI == kGemmQkvRope) {
+    switch (kind) {
+      case kTileRope0: return launch_pp<EPI, 192, 128>(p, st);
+      case kTileRope0 + 1: return launch_pp<EPI, 192, 192>(p, st);
+      case kTileRopeBig:
+        return g_gemm_schedule == 3 ? launch_pp<EPI, 192, 256, 4>(p, st) : launch_pp<EPI, 192, 256>(p, st);
     }
   }
-  if (g_gemm_schedule == 3 && kind == kTileBig192) {
-    switch (epi) {
-      case kGemmBf16: return launch_pp<kGemmBf16, 192, 256, 4>(p, st);
-      case kGemmResid: return launch_pp<kGemmResid, 192, 256, 4>(p, st);
+  if constexpr (EPI != kGemmQkvRope) {
+    switch (kind) {
+      case 0: return launch_pp<EPI, 128, 128>(p, st);
+      case 1: if constexpr (!sw) return launch_pp<EPI, 128, 160, 3, 2>(p, st); break;
+      case 2: return launch_pp<EPI, 128, 192>(p, st);
+      case 3: if constexpr (!sw) return launch_pp<EPI, 128, 224, 3, 2>(p, st); break;
+      case 4: return launch_pp<EPI, 128, 256>(p, st);
+      case 5: return launch_pp<EPI, 256, 160, 3, 2>(p, st);
+      case 6: return launch_pp<EPI, 256, 192, 3, 2>(p, st);
+      case 7: return launch_pp<EPI, 256, 224, 3, 2>(p, st);
+      case kTileBig: return launch_pp<EPI, 256, 256, 3, 2>(p, st);
     }
   }
-  if (g_gemm_schedule >= 2 && kind == kTileWide && epi != kGemmF32) {
-    switch (epi) {
-      case kGemmBf16: return launch_pp<kGemmBf16, 256, 128>(p, st);
-      case kGemmResid: return launch_pp<kGemmResid, 256, 128>(p, st);
-      case kGemmSwiglu: return launch_pp<kGemmSwiglu, 256, 128>(p, st);
-    }
-  }
-  switch (kind * 4 + epi) {
-    case kTileSmall * 4 + kGemmBf16: return launch_e<kGemmBf16>(p, st);
-    case kTileSmall * 4 + kGemmResid: return launch_e<kGemmResid>(p, st);
-    case kTileSmall * 4 + kGemmF32: return launch_e<kGemmF32>(p, st);
-    case kTileSmall * 4 + kGemmSwiglu: return launch_e<kGemmSwiglu>(p, st);
-    case kTileWide * 4 + kGemmBf16: return launch_wide<kGemmBf16, 128, 64, 3, 1, 256, 2>(p, st);
-    case kTileWide * 4 + kGemmResid: return launch_wide<kGemmResid, 128, 64, 3, 1, 256, 2>(p, st);
-    case kTileWide * 4 + kGemmF32: return launch_wide<kGemmF32, 128, 64, 3, 1, 256, 2>(p, st);
-    case kTileWide * 4 + kGemmSwiglu: return launch_wide<kGemmSwiglu, 128, 64, 3, 1, 256, 2>(p, st);
-  }
-  if (g_gemm_schedule >= 1) {
-    switch (kind * 4 + epi) {
-      case kTileBig * 4 + kGemmBf16: return launch_pp<kGemmBf16, 256>(p, st);
-      case kTileBig * 4 + kGemmResid: return launch_pp<kGemmResid, 256>(p, st);
-      case kTileBig * 4 + kGemmSwiglu: return launch_pp<kGemmSwiglu, 256>(p, st);
-      case kTileBig192 * 4 + kGemmBf16: return launch_pp<kGemmBf16, 192>(p, st);
-      case kTileBig192 * 4 + kGemmResid: return launch_pp<kGemmResid, 192>(p, st);
-    }
-  }
-  switch (kind * 4 + epi) {
-    case kTileBig * 4 + kGemmBf16: return launch_wide<kGemmBf16, 256, 64, 2>(p, st);
-    case kTileBig * 4 + kGemmResid: return launch_wide<kGemmResid, 256, 64, 2>(p, st);
-    case kTileBig * 4 + kGemmSwiglu: return launch_wide<kGemmSwiglu, 256, 64, 2>(p, st);
-    case kTileBig192 * 4 + kGemmBf16: return launch_wide<kGemmBf16, 256, 64, 2, 1, 192>(p, st);
-    case kTileBig192 * 4 + kGemmResid: return launch_wide<kGemmResid, 256, 64, 2, 1, 192>(p, st);
-  }
-  set_error("gemm: bad epilogue %d", epi);
+  set_error("gemm: tile kind %d for epilogue %d", kind, EPI);
   return IE_ERR_INVALID_ARG;
 }
 
@@ -1477,54 +1387,21 @@ GemmParams column_tail(int epi, const GemmParams& p, int c) {
   return q;
 }
 
-// Cheapest tile shape; with `split`, a partial last round of that shape may instead be run as
-// a second launch over the remaining output columns with the shape that fills the chip for
-// them (gate/up at S = 2048: 3 rounds of 256 x 256 tiles, then the last 2048 columns as one
-// round of 256 x 128 tiles, in place of a half-empty fourth round).
-// Cheapest tile shape for p.
-int best_kind(int epi, const GemmParams& p) {
-  int best = kTileSmall;
-  double best_cost = tile_cost(kTileSmall, epi, p.M, p.N);
-  for (int k = kTileWide; k < kTileKinds; ++k) {
-    if (!tile_ok(k, epi, p)) continue;
-    const double c = tile_cost(k, epi, p.M, p.N);
-    if (c < best_cost) best = k, best_cost = c;
-  }
-  return best;
-}
-
-int launch_tiled(int epi, const GemmParams& p, hipStream_t st, bool split) {
-  const int best = best_kind(epi, p);
-  const double best_cost = tile_cost(best, epi, p.M, p.N);
-  if (split) {
-    const TileKind& t = kTiles[best];
-    const int tn = epi == kGemmSwiglu ? t.tn_swiglu : t.tn;
-    const int m_tiles = (p.M + t.tm - 1) / t.tm;
-    const long long tiles = tile_count(best, epi, p.M, p.N);
-    if (tiles > 256 && tiles % 256 != 0 && 256 % m_tiles == 0) {
-      const int c = (int)(tiles / 256 * 256 / m_tiles) * tn;  // columns of the full rounds
-      const GemmParams tail = column_tail(epi, p, c);
-      double tail_cost = 1e30;
-      for (int k = kTileSmall; k < kTileKinds; ++k)
-        if (tile_ok(k, epi, tail)) tail_cost = std::min(tail_cost, tile_cost(k, epi, tail.M, tail.N));
-      if ((double)(tiles / 256) * t.unit + tail_cost < best_cost) {
-        GemmParams head = p;
-        head.N = c;
-        // 256 x 256 then 256 x 128 ping-pong tiles: one launch
-        if (g_gemm_schedule >= 2 && best == kTileBig && best_kind(epi, tail) == kTileWide) {
-          switch (epi) {
-            case kGemmBf16: return launch_pp_dual<kGemmBf16>(head, tail, st);
-            case kGemmResid: return launch_pp_dual<kGemmResid>(head, tail, st);
-            case kGemmSwiglu: return launch_pp_dual<kGemmSwiglu>(head, tail, st);
-          }
-        }
-        const int rc = launch_kind(best, epi, head, st);
-        if (rc != IE_OK) return rc;
-        return launch_tiled(epi, tail, st, false);
-      }
-    }
-  }
-  return launch_kind(best, epi, p, st);
+// The columns past the full rounds of 256 x 256 tiles as 256 x 128 tiles of the same launch, when
+// that beats the plan (gate/up at S = 2048: 3 rounds, then the last 2048 columns as one round of the
+// smaller tiles, in place of a half-empty fourth round): those columns' count, else 0.
+int dual_tail(int epi, const GemmParams& p, double plan_us) {
+  const int tn = epi == kGemmSwiglu ? 128 : 256, m_tiles = (p.M + 255) / 256;
+  const long long tiles = (long long)m_tiles * ((p.N + tn - 1) / tn);
+  if (g_gemm_schedule < 2 || tiles <= 256 || tiles % 256 == 0 || 256 % m_tiles != 0) return 0;
+  const int head = (int)(tiles / 256 * 256 / m_tiles) * tn;
+  if (head >= p.N) return 0;
+  const double kt = p.K / 64;
+  const long long tail = (long long)((p.M + 127) / 128) * ((p.N - head + tn - 1) / tn);
+  const double us = 1.4 + (double)(tiles / 256) * tile_us(256, 256, kTiles[kTileBig].step, kt, 256) +
+                    (double)((tail + 255) / 256) * tile_us(256, 128, kStep256x128, kt, 256) +
+                    (epi == kGemmResid ? 2 + 0.0021 * p.M : 0);
+  return us < plan_us ? p.N - head : 0;
 }
 
 // Sum of the split planes of 8 consecutive partials.
@@ -1695,11 +1572,6 @@ __global__ __launch_bounds__(256) void split_reduce_rope_kernel(const float* par
   }
 }
 
-// Split K when the best tiling is a single round that leaves at least half the chip idle, or
-// one of 128 x 128 tiles: the wide kernel's tiles times the largest K split that divides the
-// k-steps, fits one round of 256 workgroups and whose partials fit p.split_ws (at least 2),
-// fp32 partials into p.split_ws, then the reduction.  Returns
-// IE_OK after launching, 1 when split K does not apply.
 // The reduction of a split product: p.split_ws holds `splits` fp32 planes of M x NP (NP = 2N
 // for SwiGLU: gate then up), y = epilogue(sum) -- RoPE and the K/V scatter, residual + RMSNorm
 // (p.rn_out), residual, SwiGLU or bf16.
@@ -1729,43 +1601,50 @@ int launch_split_reduce(int epi, const GemmParams& p, int splits, hipStream_t st
   return IE_OK;
 }
 
-int launch_split(int epi, const GemmParams& p, hipStream_t st) {
-  // (below kWideMinRows too: a 128-row tile half empty still beats a few 128 x 128 tiles)
-  if (!p.split_ws || epi == kGemmF32 || p.M > kSplitMaxRows || p.N % 8 != 0 || p.ldy % 8 != 0)
-    return 1;
-  const bool sw = epi == kGemmSwiglu;
-  const bool rope = epi == kGemmQkvRope;
-  const int te = rope ? kGemmBf16 : epi;  // the tiling of the plain product
-  if (sw && p.N % 16 != 0) return 1;
-  int best = kTileSmall;
-  for (int k = kTileWide; k < kTileKinds; ++k)
-    if (tile_ok(k, te, p) && tile_cost(k, te, p.M, p.N) < tile_cost(best, te, p.M, p.N)) best = k;
-  // a single round that leaves half the chip idle, or one of 128 x 128 tiles (the older,
-  // slower kernel)
-  const long long best_tiles = tile_count(best, te, p.M, p.N);
-  if (best_tiles > 256 || (best_tiles > 128 && best != kTileSmall)) return 1;
-  // SwiGLU: one fp32 product over the gate rows then the up rows (2N columns)
-  const int NP = sw ? 2 * p.N : p.N;
-  const long long tiles = tile_count(kTileWide, kGemmF32, p.M, NP);
-  const int kt = p.K / 64;
-  const size_t plane = (size_t)p.M * NP * sizeof(float);
-  int splits = 1;
-  for (int s = 2; s <= 16; ++s)
-    if (kt % s == 0 && tiles * s <= 256 && (size_t)s * plane <= (size_t)p.split_ws_bytes) splits = s;
-  if (splits < 2) return 1;
-  GemmParams q = p;
-  q.yf = p.split_ws;
-  q.ldy = NP;
-  q.k_splits = splits;
-  if (sw) {
-    q.N = NP;
-    q.n0 = p.N;  // rows [0, N) of w0 (gate), then [N, 2N) of w1 (up)
-    q.n1 = p.N;
-    q.w2 = p.w1;
+// The tiled product of any M: the plan's tiles, K split into fp32 planes summed by the reduction
+// that applies the epilogue, or unsplit.  p's operands 16-byte aligned.
+int launch_tiled(int epi, const GemmParams& p, hipStream_t st) {
+  const TilePlan plan = plan_tiles(epi, p);
+  IE_REQUIRE(plan.kind >= 0, "gemm: no tile shape for epilogue %d", epi);
+  if (plan.splits > 1) {
+    GemmParams q = p;
+    q.yf = p.split_ws;
+    q.ldy = p.N;
+    q.k_splits = plan.splits;
+    IE_TRY(launch_kind<kGemmF32>(plan.kind, q, st));
+    return launch_split_reduce(epi, p, plan.splits, st);
   }
-  const int rc = launch_wide<kGemmF32, 128, 64, 3, 1, 256, 2>(q, st);
-  if (rc != IE_OK) return rc;
-  return launch_split_reduce(epi, p, splits, st);
+  if (epi == kGemmBf16 || epi == kGemmResid || epi == kGemmSwiglu) {
+    const int tail = rope_product(epi, p) ? 0 : dual_tail(epi, p, plan.us);
+    if (tail > 0) {
+      GemmParams head = p;
+      head.N = p.N - tail;
+      const GemmParams rest = column_tail(epi, p, head.N);
+      switch (epi) {
+        case kGemmBf16: return launch_pp_dual<kGemmBf16>(head, rest, st);
+        case kGemmResid: return launch_pp_dual<kGemmResid>(head, rest, st);
+        default: return launch_pp_dual<kGemmSwiglu>(head, rest, st);
+      }
+    }
+  }
+  GemmParams q = p;
+  q.k_splits = 1;
+  switch (epi) {
+    case kGemmBf16: return launch_kind<kGemmBf16>(plan.kind, q, st);
+    case kGemmResid: return launch_kind<kGemmResid>(plan.kind, q, st);
+    case kGemmF32: return launch_kind<kGemmF32>(plan.kind, q, st);
+    case kGemmSwiglu: return launch_kind<kGemmSwiglu>(plan.kind, q, st);
+    case kGemmQkvRope: return launch_kind<kGemmQkvRope>(plan.kind, q, st);
+  }
+  set_error("gemm: bad epilogue %d", epi);
+  return IE_ERR_INVALID_ARG;
+}
+
+// Direct-to-LDS loads move 16 bytes: the bases (rows are K x 2 bytes apart, K a multiple of 64)
+// must be 16-byte aligned; other operands take the register-staged 128 x 128 kernel.
+bool operands_aligned(const GemmParams& p) {
+  const auto a16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
+  return a16(p.x) && a16(p.w0) && a16(p.w1) && a16(p.w2) && a16(p.yf);
 }
 
 // Medium M (16 < M <= 128, K a multiple of 64): the 64-W-row streaming kernel, with its fp32
@@ -1858,9 +1737,15 @@ int launch_gemm(int epi, const GemmParams& p, hipStream_t st) {
   IE_REQUIRE(p.k_splits <= 1, "gemm: k_splits is the launcher's");
   IE_REQUIRE(!p.rn_out || (epi == kGemmResid && p.N == kHidden && p.rn_w),
              "gemm: the fused RMSNorm output follows a residual product of %d columns", kHidden);
-  const int rc = launch_split(epi, p, st);
-  if (rc != 1) return rc;
-  return launch_tiled(epi, p, st, true);
+  if (!operands_aligned(p)) {
+    switch (epi) {
+      case kGemmBf16: return launch_e<kGemmBf16>(p, st);
+      case kGemmResid: return launch_e<kGemmResid>(p, st);
+      case kGemmF32: return launch_e<kGemmF32>(p, st);
+      default: return launch_e<kGemmSwiglu>(p, st);
+    }
+  }
+  return launch_tiled(epi, p, st);
 }
 
 }  // namespace ie
@@ -1878,19 +1763,8 @@ int launch_qkv_rope_prefill(const GemmParams& p, hipStream_t st) {
     if (rc != 1) return rc;
   }
   if (gemm_skinny_mb_fits(kGemmBf16, p)) return 1;
-  // up to kSplitMaxRows rows: K split with the RoPE / scatter reduction where the bf16 product
-  // would split
-  if (p.M <= kSplitMaxRows) return launch_split(kGemmQkvRope, p, st);
-  // above: the bf16 product's own choice (launch_gemm): the 192 x 256 tile in whole rounds
-  int best = kTileSmall;
-  for (int k = kTileWide; k < kTileKinds; ++k)
-    if (tile_ok(k, kGemmBf16, p) &&
-        tile_cost(k, kGemmBf16, p.M, p.N) < tile_cost(best, kGemmBf16, p.M, p.N))
-      best = k;
-  const long long tiles = tile_count(kTileBig192, kGemmBf16, p.M, p.N);
-  if (best != kTileBig192 || (tiles > 256 && tiles % 256 != 0)) return 1;
-  if (g_gemm_schedule == 3) return launch_pp<kGemmQkvRope, 192, 256, 4>(p, st);
-  return launch_pp<kGemmQkvRope, 192, 256>(p, st);
+  if (!operands_aligned(p)) return 1;
+  return launch_tiled(kGemmQkvRope, p, st);
 }
 
 }  // namespace ie

@@ -361,3 +361,29 @@ def test_batched_generate_512_then_256_config5(hip, model, oracle_model, noise_f
         check_token(th[b], want[b], got[b], noise_floor)
         assert_bf16_close(gkv[b][0, :, :, last], kvo[b][0, :, :, last],
                           what=f"row {b} layer-0 kv row {last}", outlier_frac=2e-3)
+
+
+@pytest.mark.parametrize("S", [130, 200, 300, 777, 930, 1100, 1537, 2100])
+def test_prefill_layer_schedules_equal(hip, ctx, model, S):
+    """One prefill layer past 128 rows: QKV with RoPE and the K/V write in the product's epilogue
+    (192-row tiles of 128, 192 and 256 X rows) or in the split reduction, against schedule 0's
+    product + scatter kernel over the same K splits: K/V rows and output rows bit for bit."""
+    from infengine_amd.engine import kv_cache_size, workspace_size
+    g = torch.Generator(device="cuda").manual_seed(S)
+    x0 = torch.empty(S, 4096, dtype=torch.bfloat16, device="cuda").normal_(0.0, 1.0, generator=g)
+    ws = torch.empty(workspace_size(S), dtype=torch.uint8, device="cuda")
+    outs = []
+    try:
+        for sched in (2, 0):
+            say(f"prefill layer S={S}, gemm schedule {sched}")
+            hip.check(hip.lib.ie_tune_gemm_schedule(sched))
+            kv = torch.zeros(kv_cache_size() // 2, dtype=torch.bfloat16, device="cuda")
+            x, aux, attn = x0.clone(), torch.empty_like(x0), torch.empty_like(x0)
+            hip.check(hip.lib.ie_decoder_layer_prefill(ctx.handle, model.ref(), 3, S, _ptr(x), _ptr(aux),
+                                                       _ptr(attn), _ptr(ws), _ptr(kv)))
+            torch.cuda.synchronize()
+            outs.append((x, kv.view(32, 2, 8, 8192, 128)[3, :, :, :S + 1].clone()))
+    finally:
+        hip.check(hip.lib.ie_tune_gemm_schedule(2))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    assert bool(outs[0][1][:, :, :S].any()) and not bool(outs[0][1][:, :, S].any())

@@ -388,6 +388,73 @@ def test_gemm_schedules_bit_identical(hip, ctx, epi, m, k, n):
     assert np.isfinite(orc.bf16_to_f32(outs[2])).all() and outs[2][[0, m // 2, m - 1]].any()
 
 
+# Every tile shape of the prefill GEMM past 128 rows at the first, last or a middle row count that
+# picks it, K split (planes of 2-8) and not, ragged columns (n = 1000, 4104; n = 4100 never
+# splits), one and three k-steps, and bases off 16 bytes (the register-staged kernel).
+@pytest.mark.parametrize("epi,m,k,n", [
+    ("resid", 130, 4096, 4096), ("resid", 192, 4096, 4096), ("resid", 257, 4096, 4096),
+    ("resid", 385, 4096, 4104), ("resid", 512, 4096, 4096), ("resid", 929, 4096, 4096),
+    ("resid", 1100, 4096, 4100), ("resid", 1284, 4096, 4096), ("resid", 1600, 4096, 4096),
+    ("resid", 2575, 4096, 4096), ("resid", 300, 14336, 4096), ("resid", 700, 14336, 4096),
+    ("resid", 800, 14336, 4096), ("resid", 901, 14336, 4096), ("resid", 3100, 14336, 4096),
+    ("bf16", 161, 4096, 1000), ("bf16", 1030, 192, 4096), ("bf16", 200, 64, 4096),
+    ("f32", 129, 4096, 4096), ("f32", 1025, 192, 4100), ("f32", 2100, 4096, 4096),
+    ("swiglu", 129, 4096, 14336), ("swiglu", 256, 4096, 14336), ("swiglu", 257, 4096, 14336),
+    ("swiglu", 384, 4096, 14336), ("swiglu", 385, 4096, 14336), ("swiglu", 449, 4096, 14340),
+    ("swiglu", 2100, 256, 1000)])
+def test_gemm_tile_shapes(hip, ctx, epi, m, k, n):
+    """Products past 128 rows against torch in float32 on every row (|y - y_ref| <= 2 bf16 steps of
+    the value, as in assert_bf16_close), nothing written past the last row, and the same bits from
+    the DMA-ring kernel (schedule 0) over the same K splits."""
+    say(f"gemm tile shapes {epi} m={m} k={k} n={n}")
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    def draw(*shape, std=1.0):
+        return torch.empty(shape, dtype=torch.bfloat16, device="cuda").normal_(0.0, std, generator=g)
+    x, w0, w1, y0 = draw(m, k), draw(n, k, std=0.02), draw(n, k, std=0.02), draw(m + 1, n)
+    dt = torch.float32 if epi == "f32" else torch.bfloat16
+    outs = []
+    try:
+        for sched in (2, 0):
+            hip.check(hip.lib.ie_tune_gemm_schedule(sched))
+            y = y0.to(dt, copy=True)
+            hip.check(hip.lib.ie_gemm_ex(ctx.handle, GEMM_EPI[epi], m, k, n, P(x), P(w0), P(w1), P(y)))
+            sync()
+            outs.append(y)
+    finally:
+        hip.check(hip.lib.ie_tune_gemm_schedule(2))
+    assert torch.equal(outs[0], outs[1])
+    assert torch.equal(outs[0][m], y0[m].to(dt))
+    acc = x.float() @ w0.float().t()
+    got = outs[0][:m].float().cpu().numpy()
+    if epi == "f32":
+        assert_close(got, acc.cpu().numpy(), tol=1e-4, what="tile shapes f32")
+        return
+    want = acc.bfloat16()
+    if epi == "resid":
+        want = (y0[:m].float() + want.float()).bfloat16()
+    elif epi == "swiglu":
+        up = (x.float() @ w1.float().t()).bfloat16().float()
+        want = (torch.nn.functional.silu(want.float()) * up).bfloat16()
+    want = want.view(torch.int16)
+    assert_close(got, orc.bf16_to_f32(host(want)), what=f"tile shapes {epi}")
+    assert_bf16_close(host(outs[0][:m].view(torch.int16)), host(want), ulps=4 if epi == "swiglu" else 2,
+                      what=f"tile shapes {epi}", outlier_frac=1e-3 if epi == "resid" else 0.0)
+
+
+def test_gemm_unaligned_operands(hip, ctx):
+    """X and W bases off 16 bytes (8): the register-staged kernel, the aligned call's values."""
+    m, k, n = 300, 256, 512
+    say(f"gemm unaligned operands m={m} k={k} n={n}")
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.empty(m * k + 4, dtype=torch.bfloat16, device="cuda").normal_(0.0, 1.0, generator=g)
+    w = torch.empty(n * k + 4, dtype=torch.bfloat16, device="cuda").normal_(0.0, 0.02, generator=g)
+    y = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    hip.check(hip.lib.ie_gemm_bf16(ctx.handle, m, k, n, P(x[4:]), P(w[4:]), P(y)))
+    sync()
+    want = (x[4:].view(m, k).float() @ w[4:].view(n, k).float().t()).bfloat16()
+    assert_bf16_close(host(y.view(torch.int16)), host(want.view(torch.int16)), ulps=2, what="unaligned")
+
+
 # The skinny kernel at M <= 16: the fp32 epilogue's 32-row tiles (K = 4096 / 14336) with the
 # last partial round in K halves (n = 8224: 257 tiles, one split; the lm_head's 128256 columns:
 # 4008 tiles, 168 split) or none (n = 4100: 129 tiles, the last with 4 rows), and the bf16 /
