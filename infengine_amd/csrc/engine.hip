@@ -323,6 +323,10 @@ int ie_context_create(ie_context** out, int device, void* stream) {
   size_t zeroed = 0;
   do {
     c->stream = stream_of(stream);
+    if (hipStreamCreateWithFlags(&c->capture, hipStreamNonBlocking) != hipSuccess) {
+      rc = IE_ERR_HIP;
+      break;
+    }
     // one device allocation (the counters, slots and params, zeroed below, first) and one pinned
     // one: each allocation is ~40-100 us of a context's creation
     const size_t cnt = align256(kNumCounters * sizeof(unsigned int)),
@@ -460,7 +464,6 @@ int decode_step_impl(Context* c, const ie_model_weights* weights, int seq_len, i
       // captured on the private stream (capture is not allowed on the legacy
       // default stream), replayed on the context's stream
       hipGraph_t g = nullptr;
-      if (!c->capture) IE_CHECK_HIP(hipStreamCreateWithFlags(&c->capture, hipStreamNonBlocking));
       IE_CHECK_HIP(hipStreamBeginCapture(c->capture, hipStreamCaptureModeThreadLocal));
       const int rc = enqueue_decode(c, c->capture, *weights, seq_len, tokenid_buff, data_buffer,
                                     attn_buffer, output_distr, output_token, workspace, kv_cache,
@@ -1023,7 +1026,6 @@ int batched_step(ie_context* c, const ie_model_weights* weights, int batch, cons
         slot->exec = nullptr;
       }
       hipGraph_t g = nullptr;
-      if (!c->capture) IE_CHECK_HIP(hipStreamCreateWithFlags(&c->capture, hipStreamNonBlocking));
       IE_CHECK_HIP(hipStreamBeginCapture(c->capture, hipStreamCaptureModeThreadLocal));
       const int rc = enqueue_batched(c, c->capture, *weights, batch, len_class, tokenid_buffs,
                                      tokens_stride, data_buffer, attn_buffer, output_distr,

@@ -241,7 +241,7 @@ constexpr double kSynthStd = 37837.22627754049;
 struct Context {
   int device = 0;
   hipStream_t stream = nullptr;    // nullptr = the legacy default stream
-  hipStream_t capture = nullptr;   // private stream the graphs are captured on (made for the first)
+  hipStream_t capture = nullptr;   // private stream the graphs are captured on
   void* arena = nullptr;           // the device allocation behind the d_ pointers below
   unsigned int* d_counters = nullptr;       // self-resetting last-block counters
   unsigned long long* d_slots = nullptr;    // 64-bit reduction slots (argmax)
