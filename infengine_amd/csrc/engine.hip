@@ -1544,7 +1544,8 @@ int ie_sample_argmax_rows(ie_context* c, int rows, int vocab, const float* d_log
 }
 
 size_t ie_top_p_workspace_size(int rows, int vocab) {
-  return top_p_workspace_bytes(rows < 1 ? 1 : rows, vocab < 1 ? 1 : vocab);
+  (void)vocab;
+  return top_p_workspace_bytes(rows < 1 ? 1 : rows);
 }
 
 int ie_sample_top_p(ie_context* c, int rows, int vocab, const float* d_logits, float temperature,
@@ -1555,7 +1556,7 @@ int ie_sample_top_p(ie_context* c, int rows, int vocab, const float* d_logits, f
                       static_cast<float*>(workspace), c->stream);
 }
 
-// No allocation: the exponentials go to the library's static per-device scratch
+// No allocation: the rows' state goes to the library's static per-device scratch
 // (top_p_scratch), resolved when a context was created on this device.  Calls that overlap on
 // one GPU share that scratch and race.
 int ie_sample_top_p_noalloc(ie_context* c, int rows, int vocab, const float* d_logits,
@@ -1564,11 +1565,10 @@ int ie_sample_top_p_noalloc(ie_context* c, int rows, int vocab, const float* d_l
   CTX_OK(c);
   IE_REQUIRE(d_logits && d_output, "sample_top_p_noalloc: null pointer");
   IE_REQUIRE(rows >= 1 && vocab >= 1, "sample_top_p_noalloc: rows=%d vocab=%d", rows, vocab);
-  IE_REQUIRE(rows <= kTopPNoallocRows && (size_t)rows * (size_t)vocab <= kTopPScratchFloats &&
-                 top_p_workspace_bytes(rows, vocab) <= kTopPScratchBytes,
+  IE_REQUIRE(rows <= kTopPNoallocRows && (size_t)rows * (size_t)vocab <= kTopPNoallocFloats,
              "sample_top_p_noalloc: rows x vocab = %d x %d exceeds the static scratch (%d rows, "
              "%zu logits; use ie_sample_top_p with a workspace)",
-             rows, vocab, kTopPNoallocRows, kTopPScratchFloats);
+             rows, vocab, kTopPNoallocRows, kTopPNoallocFloats);
   float* ws = top_p_scratch(c->device);
   IE_REQUIRE(ws != nullptr, "sample_top_p_noalloc: scratch of device %d not initialised",
              c->device);

@@ -13,7 +13,7 @@
 // <= 1-p, keep >= 1 token): token i is kept iff the probability mass of tokens
 // with a strictly larger scaled logit is < p.  Masses are exp(l/T - max) in
 // fixed point (2^-40 units, uint64), so every sum is exact and order-free:
-//   1. max of l/T; e_i = expf(l_i/T - max) cached in the workspace; Z = sum q_i
+//   1. max of l/T; e_i = expf(l_i/T - max); Z = sum q_i
 //   2. the cut key kappa with mass(key > kappa) < target <= mass(key >= kappa): the positive
 //      masses binned by distance to the max locate its bin, then a radix select (4 x 8-bit
 //      digits of the order-preserving key of l_i/T) over that bin's tokens
@@ -21,6 +21,8 @@
 //      uniform of (seed, row, step)
 //   4. the sampled token is the smallest id whose kept prefix mass exceeds t
 //      (inverse CDF in token-id order), found with a block-wide exclusive scan.
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #include "ie_kernels.h"
@@ -122,44 +124,62 @@ __device__ __forceinline__ T wave_sum_u64(T v) {
   return v;
 }
 
+// Inclusive scan over the wave's lanes.
+template <typename T>
+__device__ __forceinline__ T wave_scan(T v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const T w = __shfl_up(v, o, 64);
+    if (lane >= o) v += w;
+  }
+  return v;
+}
+
 // Tokens with a positive fixed-point mass lie within 28 nats of the largest scaled logit
 // (exp(-27.8) * 2^40 < 1), and only they can be kept (the cut token has positive mass, and every
 // zero-mass token's key is below its key).  They are binned by their distance d = max - l/T into
 // kTopPBins bins: bin(d) is non-decreasing in d, so every key of a lower bin is strictly larger
 // than every key of a higher one and equal keys share a bin.  The bin where the cumulative mass
 // from the top reaches the target holds the cut; the radix select runs over its tokens only.
+// Tokens of lower bins are kept whole.
 //
-// Each row is split into kTopPChunks chunks, one workgroup each, over six launches (the row's
-// state, histogram and candidates sit in a TopPRow after the exponentials in the workspace):
+// Each row is split into kTopPChunks chunks, one workgroup each (a chunk of the 128256-entry
+// vocabulary is one round of 8 loads in flight a thread), over four launches; the row's state is
+// a TopPRow in the workspace, the masses are recomputed from the logits (a division and an expf a
+// token, cheaper than caching them in memory):
 //   tp_max     chunk maxima of l (the max of l/T is fl(max l / T): division by T > 0 is
 //              monotone); the row's histogram and candidate count are cleared
-//   tp_hist    e = expf(l/T - max) (cached), chunk mass, the chunk's positive masses binned in
+//   tp_hist    chunk mass; the chunk's masses up to the last bin that can hold the cut, binned in
 //              LDS and added to the row's histogram
 //   tp_gather  every workgroup scans the histogram for the cut bin (identical results), then
-//              appends its chunk's tokens of that bin to the candidates
-//   tp_select  one workgroup per row: radix select of the cut key over the candidates (over the
-//              row's tokens of the cut bin when there are more than kTopPCandMax)
-//   tp_kept    chunk masses of the kept tokens
-//   tp_walk    one workgroup per row: t from the kept total, the chunk holding t, then its
-//              token by a scan over the chunk in token-id order
-constexpr int kTopPBins = 2048;
+//              appends its chunk's tokens of that bin to the candidates and sums the mass of its
+//              tokens in lower bins
+//   tp_finish  one workgroup per row: radix select of the cut key over the candidates (over the
+//              row's tokens of the cut bin when there are more than kTopPCandMax), the chunks' kept
+//              masses, t, the chunk holding t, then its token by a scan in token-id order
+// 16 rows of the 128256-entry vocabulary: 30 us, 1 row 23; the six launches that cached
+// the exponentials, used 2048 bins and summed the kept masses over all tokens took 53-57 and 37.
+// 512 bins of 0.055 nats in place of 2048: the device-scope additions of the histograms (the
+// largest part, 700 thousand a call at 16 rows) fall to a quarter, and a cut bin of a row whose
+// scaled logits spread over more than ~0.3 nats still fits the candidate list.
+constexpr int kTopPBins = 512;
 constexpr float kTopPBinScale = kTopPBins / 28.0f;
 constexpr int kTopPChunks = 64;
 constexpr int kTopPChunkThreads = 256;
-constexpr int kTopPCandMax = 8192;
+constexpr int kTopPCandMax = 10240;
+constexpr int kTopPCandLds = 4096;  // candidates that tp_finish keeps in LDS
 
 struct TopPRow {
   unsigned long long hist[kTopPBins];
   unsigned long long zpart[kTopPChunks];
-  unsigned long long kpart[kTopPChunks];
+  unsigned long long klow[kTopPChunks];  // mass of the chunk's tokens in bins below the cut bin
   float pmax[kTopPChunks];
   unsigned int ncand;
   int bcut;
-  uint32_t kappa;
-  unsigned int pad;
   unsigned long long above, target;
   uint32_t cand_key[kTopPCandMax];
-  unsigned long long cand_q[kTopPCandMax];
+  unsigned long long cand_q[kTopPCandMax];  // mass (41 bits) | chunk << 48
 };
 
 __device__ __forceinline__ int top_p_bin(float d) {
@@ -170,15 +190,10 @@ __device__ __forceinline__ int tp_chunk_len(int vocab) {
   return (vocab + kTopPChunks - 1) / kTopPChunks;
 }
 
-// Block-wide sum / max for kTopPChunkThreads threads (red: 4 entries).
-__device__ __forceinline__ unsigned long long tp_block_sum(unsigned long long v,
-                                                           unsigned long long* red) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  v = wave_sum_u64(v);
-  __syncthreads();
-  if (lane == 0) red[wave] = v;
-  __syncthreads();
-  return (red[0] + red[1]) + (red[2] + red[3]);
+// 8 logits of chunk [beg, end) from i on, 256 apart (past the end: the chunk's last one).
+__device__ __forceinline__ void tp_load8(const float* L, int i, int end, float (&v)[8]) {
+#pragma unroll
+  for (int u = 0; u < 8; ++u) v[u] = L[min(i + u * kTopPChunkThreads, end - 1)];
 }
 
 // One 256-bin digit step of the radix select (wave 0): the highest digit whose cumulative mass
@@ -193,12 +208,7 @@ __device__ __forceinline__ void top_p_digit(const unsigned long long* hist, unsi
     hb[j] = hist[255 - 4 * lane - j];
     loc += hb[j];
   }
-  unsigned long long inc = loc;  // inclusive scan over lanes
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const unsigned long long v = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += v;
-  }
+  const unsigned long long inc = wave_scan(loc);
   const unsigned long long exc = inc - loc;
   const unsigned long long hit = __ballot(inc >= t_rem);
   const int first = hit ? __ffsll((long long)hit) - 1 : 63;
@@ -226,100 +236,89 @@ __global__ __launch_bounds__(kTopPChunkThreads) void tp_max_kernel(const float* 
   TopPRow& R = rows[row];
   const float* L = logits + (size_t)row * vocab;
   const int cl = tp_chunk_len(vocab), beg = c * cl, end = min(vocab, beg + cl);
-  for (int b = c * (kTopPBins / kTopPChunks) + tid; b < (c + 1) * (kTopPBins / kTopPChunks);
-       b += kTopPChunkThreads)
-    R.hist[b] = 0;
+  if (tid < kTopPBins / kTopPChunks) R.hist[c * (kTopPBins / kTopPChunks) + tid] = 0;
   if (c == 0 && tid == 0) R.ncand = 0;
   float m = -INFINITY;
-  for (int i = beg + tid; i < end; i += kTopPChunkThreads) m = fmaxf(m, L[i]);
+  for (int i = beg + tid; i < end; i += 8 * kTopPChunkThreads) {
+    float v[8];
+    tp_load8(L, i, end, v);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) m = fmaxf(m, v[u]);
+  }
   m = wave_max(m);
   if (lane == 0) redf[wave] = m;
   __syncthreads();
   if (tid == 0) R.pmax[c] = fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
 }
 
+static_assert(kTopPChunks == 64, "one chunk a lane");
+
 __device__ __forceinline__ float tp_row_max(const TopPRow& R, float temperature) {
-  float m = R.pmax[0];
-  for (int c = 1; c < kTopPChunks; ++c) m = fmaxf(m, R.pmax[c]);
-  return m / temperature;
+  return wave_max(R.pmax[threadIdx.x & 63]) / temperature;
 }
 
 __global__ __launch_bounds__(kTopPChunkThreads) void tp_hist_kernel(const float* logits, int vocab,
-                                                                    float temperature, TopPRow* rows,
-                                                                    float* ws) {
+                                                                    float temperature, int last_bin,
+                                                                    TopPRow* rows) {
   __shared__ unsigned long long hist[kTopPBins];
   __shared__ unsigned long long red[4];
-  const int c = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+  const int c = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   TopPRow& R = rows[row];
   const float* L = logits + (size_t)row * vocab;
-  float* E = ws + (size_t)row * vocab;
   const int cl = tp_chunk_len(vocab), beg = c * cl, end = min(vocab, beg + cl);
-  const float mx = tp_row_max(R, temperature);
   for (int b = tid; b < kTopPBins; b += kTopPChunkThreads) hist[b] = 0;
+  const float mx = tp_row_max(R, temperature);
   __syncthreads();
   unsigned long long z = 0;
-  for (int i = beg + tid; i < end; i += kTopPChunkThreads) {
-    const float sv = L[i] / temperature;
-    const float e = expf(sv - mx);
-    E[i] = e;
-    const unsigned long long q = fix_mass(e);
-    z += q;
-    if (q) atomicAdd(&hist[top_p_bin(mx - sv)], q);
+  for (int i = beg + tid; i < end; i += 8 * kTopPChunkThreads) {
+    float v[8];
+    tp_load8(L, i, end, v);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (i + u * kTopPChunkThreads >= end) continue;
+      const float sv = v[u] / temperature;
+      const unsigned long long q = fix_mass(expf(sv - mx));
+      z += q;
+      const int b = top_p_bin(mx - sv);
+      if (q && b <= last_bin) atomicAdd(&hist[b], q);
+    }
   }
-  z = tp_block_sum(z, red);
-  if (tid == 0) R.zpart[c] = z;
-  for (int b = tid; b < kTopPBins; b += kTopPChunkThreads)
+  z = wave_sum_u64(z);
+  if (lane == 0) red[wave] = z;
+  __syncthreads();
+  if (tid == 0) R.zpart[c] = (red[0] + red[1]) + (red[2] + red[3]);
+  for (int b = tid; b <= last_bin; b += kTopPChunkThreads)
     if (hist[b]) atomicAdd(&R.hist[b], hist[b]);
 }
 
 __global__ __launch_bounds__(kTopPChunkThreads) void tp_gather_kernel(const float* logits, int vocab,
                                                                       float temperature, float top_p,
-                                                                      TopPRow* rows, const float* ws) {
+                                                                      TopPRow* rows) {
+  static_assert(kTopPBins == 2 * kTopPChunkThreads, "two bins a thread");
   __shared__ unsigned long long red[4];
+  __shared__ unsigned int cnt[4], s_base;
   __shared__ int s_bin;
   __shared__ unsigned long long s_above;
   const int c = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   TopPRow& R = rows[row];
   const float* L = logits + (size_t)row * vocab;
-  const float* E = ws + (size_t)row * vocab;
   const int cl = tp_chunk_len(vocab), beg = c * cl, end = min(vocab, beg + cl);
+  const unsigned long long z = wave_sum_u64(R.zpart[lane]);
   const float mx = tp_row_max(R, temperature);
-  unsigned long long z = 0;
-  for (int j = 0; j < kTopPChunks; ++j) z += R.zpart[j];
   unsigned long long target = (unsigned long long)((double)z * (double)top_p);
   if (target < 1) target = 1;
-  // the cut bin: thread t owns bins 8 t .. 8 t + 7 (ascending distance), block inclusive scan
-  unsigned long long hb[8], loc = 0;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    hb[j] = R.hist[8 * tid + j];
-    loc += hb[j];
-  }
-  unsigned long long inc = loc;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const unsigned long long v = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += v;
-  }
+  // the cut bin: thread t owns bins 2t, 2t + 1 (ascending distance), block inclusive scan
+  const unsigned long long h0 = R.hist[2 * tid], h1 = R.hist[2 * tid + 1];
+  unsigned long long inc = wave_scan(h0 + h1);
   if (lane == 63) red[wave] = inc;
-  if (tid == 0) s_bin = -1;
+  if (tid == 0) s_bin = -1, s_above = 0;
   __syncthreads();
-  unsigned long long wb = 0;
-  for (int w = 0; w < wave; ++w) wb += red[w];
-  inc += wb;
-  const unsigned long long exc = inc - loc;
+  for (int w = 0; w < wave; ++w) inc += red[w];
+  const unsigned long long exc = inc - (h0 + h1);
   if (exc < target && inc >= target) {  // exactly one thread
-    unsigned long long cum = exc;
-    int bin = 8 * tid + 7;
-    for (int j = 0; j < 8; ++j) {
-      if (cum + hb[j] >= target) {
-        bin = 8 * tid + j;
-        break;
-      }
-      cum += hb[j];
-    }
-    s_bin = bin;
-    s_above = cum;
+    const bool first = exc + h0 >= target;
+    s_bin = first ? 2 * tid : 2 * tid + 1;
+    s_above = first ? exc : exc + h0;
   }
   __syncthreads();
   const int bcut = s_bin;
@@ -328,51 +327,98 @@ __global__ __launch_bounds__(kTopPChunkThreads) void tp_gather_kernel(const floa
     R.above = s_above;
     R.target = target;
   }
-  for (int i = beg + tid; i < end; i += kTopPChunkThreads) {
-    const float sv = L[i] / temperature;
-    if (top_p_bin(mx - sv) != bcut) continue;
-    const unsigned long long q = fix_mass(E[i]);
-    if (!q) continue;
-    const unsigned int slot = atomicAdd(&R.ncand, 1u);
-    if (slot < (unsigned)kTopPCandMax) {
-      R.cand_key[slot] = order_key(sv);
-      R.cand_q[slot] = q;
+  unsigned long long low = 0;
+  // (beg and end are the workgroup's: every thread runs every round and its barriers)
+  for (int i0 = beg; i0 < end; i0 += 8 * kTopPChunkThreads) {
+    const int i = i0 + tid;
+    float v[8];
+    tp_load8(L, i, end, v);
+    unsigned int hits = 0;
+    unsigned long long q[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float sv = v[u] / temperature;
+      const int b = top_p_bin(mx - sv);
+      const bool in = i + u * kTopPChunkThreads < end;
+      q[u] = fix_mass(expf(sv - mx));
+      if (in && b < bcut) low += q[u];
+      if (in && b == bcut && q[u]) hits |= 1u << u;
     }
+    // this round's candidates take consecutive slots: one device-scope addition a workgroup
+    const unsigned int n = __popc(hits), ninc = wave_scan(n);
+    if (lane == 63) cnt[wave] = ninc;
+    __syncthreads();
+    if (tid == 0) {
+      const unsigned int all = (cnt[0] + cnt[1]) + (cnt[2] + cnt[3]);
+      s_base = all ? atomicAdd(&R.ncand, all) : 0;
+    }
+    __syncthreads();
+    unsigned int slot = s_base + ninc - n;
+    for (int w = 0; w < wave; ++w) slot += cnt[w];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (!(hits >> u & 1)) continue;
+      if (slot < (unsigned)kTopPCandMax) {
+        R.cand_key[slot] = order_key(v[u] / temperature);
+        R.cand_q[slot] = q[u] | (unsigned long long)c << 48;
+      }
+      ++slot;
+    }
+    __syncthreads();  // cnt and s_base are reused
   }
+  low = wave_sum_u64(low);
+  if (lane == 0) red[wave] = low;
+  __syncthreads();
+  if (tid == 0) R.klow[c] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-__global__ __launch_bounds__(kTopPThreads) void tp_select_kernel(const float* logits, int vocab,
-                                                                 float temperature, TopPRow* rows,
-                                                                 const float* ws) {
+__global__ __launch_bounds__(kTopPThreads) void tp_finish_kernel(const float* logits, int vocab,
+                                                                 float temperature, uint64_t seed,
+                                                                 uint64_t step, TopPRow* rows,
+                                                                 int* out) {
   __shared__ unsigned long long hist[256];
-  __shared__ int s_bin;
-  __shared__ unsigned long long s_above;
-  const int row = blockIdx.x, tid = threadIdx.x, wave = tid >> 6;
+  __shared__ uint32_t ck[kTopPCandLds];
+  __shared__ unsigned long long cq[kTopPCandLds];
+  __shared__ unsigned long long kpart[kTopPChunks];
+  __shared__ unsigned long long red[kTopPThreads / 64];
+  __shared__ int s_bin, s_chunk, s_tok;
+  __shared__ unsigned long long s_above, s_t;
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   TopPRow& R = rows[row];
   const float* L = logits + (size_t)row * vocab;
-  const float* E = ws + (size_t)row * vocab;
+  const int cl = tp_chunk_len(vocab);
   const int ncand = (int)R.ncand, bcut = R.bcut;
-  const bool listed = ncand <= kTopPCandMax;
+  const bool listed = ncand <= kTopPCandMax, in_lds = ncand <= kTopPCandLds;
   const float mx = tp_row_max(R, temperature);
-  uint32_t prefix = 0, mask = 0;
   unsigned long long t_rem = R.target - R.above;
-  for (int shift = 24; shift >= 0; shift -= 8) {
-    if (tid < 256) hist[tid] = 0;
-    __syncthreads();
+  if (tid < kTopPChunks) kpart[tid] = R.klow[tid];
+  if (tid == 0) s_tok = -1;
+  if (in_lds)
+    for (int j = tid; j < ncand; j += kTopPThreads) ck[j] = R.cand_key[j], cq[j] = R.cand_q[j];
+  // f(key, mass, chunk) over the tokens of the cut bin
+  const auto each = [&](auto f) {
     if (listed) {
       for (int j = tid; j < ncand; j += kTopPThreads) {
-        const uint32_t k = R.cand_key[j];
-        if ((k & mask) == prefix) atomicAdd(&hist[(k >> shift) & 255u], R.cand_q[j]);
+        const uint32_t k = in_lds ? ck[j] : R.cand_key[j];
+        const unsigned long long q = in_lds ? cq[j] : R.cand_q[j];
+        f(k, q & 0xFFFFFFFFFFFFull, (int)(q >> 48));
       }
     } else {
       for (int i = tid; i < vocab; i += kTopPThreads) {
         const float sv = L[i] / temperature;
         if (top_p_bin(mx - sv) != bcut) continue;
-        const unsigned long long q = fix_mass(E[i]);
-        const uint32_t k = order_key(sv);
-        if (q && (k & mask) == prefix) atomicAdd(&hist[(k >> shift) & 255u], q);
+        const unsigned long long q = fix_mass(expf(sv - mx));
+        if (q) f(order_key(sv), q, i / cl);
       }
     }
+  };
+  uint32_t prefix = 0, mask = 0;
+  for (int shift = 24; shift >= 0; shift -= 8) {
+    if (tid < 256) hist[tid] = 0;
+    __syncthreads();
+    each([&](uint32_t k, unsigned long long q, int) {
+      if ((k & mask) == prefix) atomicAdd(&hist[(k >> shift) & 255u], q);
+    });
     __syncthreads();
     if (wave == 0) top_p_digit(hist, t_rem, &s_bin, &s_above);
     __syncthreads();
@@ -381,90 +427,61 @@ __global__ __launch_bounds__(kTopPThreads) void tp_select_kernel(const float* lo
     t_rem -= s_above;
     __syncthreads();
   }
-  if (tid == 0) R.kappa = prefix;
-}
-
-__global__ __launch_bounds__(kTopPChunkThreads) void tp_kept_kernel(const float* logits, int vocab,
-                                                                    float temperature, TopPRow* rows,
-                                                                    const float* ws) {
-  __shared__ unsigned long long red[4];
-  const int c = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
-  TopPRow& R = rows[row];
-  const float* L = logits + (size_t)row * vocab;
-  const float* E = ws + (size_t)row * vocab;
-  const int cl = tp_chunk_len(vocab), beg = c * cl, end = min(vocab, beg + cl);
-  const uint32_t kappa = R.kappa;
-  unsigned long long m = 0;
-  for (int i = beg + tid; i < end; i += kTopPChunkThreads)
-    if (order_key(L[i] / temperature) >= kappa) m += fix_mass(E[i]);
-  m = tp_block_sum(m, red);
-  if (tid == 0) R.kpart[c] = m;
-}
-
-__global__ __launch_bounds__(kTopPChunkThreads) void tp_walk_kernel(const float* logits, int vocab,
-                                                                    float temperature, uint64_t seed,
-                                                                    uint64_t step, TopPRow* rows,
-                                                                    const float* ws, int* out) {
-  __shared__ unsigned long long red[4];
-  __shared__ int s_tok;
-  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const TopPRow& R = rows[row];
-  const float* L = logits + (size_t)row * vocab;
-  const float* E = ws + (size_t)row * vocab;
-  const uint32_t kappa = R.kappa;
-  unsigned long long zk = 0;
-  for (int j = 0; j < kTopPChunks; ++j) zk += R.kpart[j];
-  const uint64_t bits = splitmix64(synth_base(seed, 0x70707070ull + (uint64_t)row) + step) >> 40;
-  const unsigned long long t = (zk >> 24) * bits + (((zk & 0xFFFFFFull) * bits) >> 24);
-  // the chunk holding t (kept masses in chunk order = token-id order)
-  int c = 0;
-  unsigned long long cbase = 0;
-  while (c + 1 < kTopPChunks && cbase + R.kpart[c] <= t) cbase += R.kpart[c++];
-  const int cl = tp_chunk_len(vocab), cbeg = c * cl, cend = min(vocab, cbeg + cl);
-  // thread segments of the chunk, exclusive scan of their kept masses, the owner walks
-  const int seg = (cl + kTopPChunkThreads - 1) / kTopPChunkThreads;
-  const int beg = min(cend, cbeg + tid * seg), end = min(cend, beg + seg);
-  unsigned long long mine = 0;
-  for (int i = beg; i < end; ++i)
-    if (order_key(L[i] / temperature) >= kappa) mine += fix_mass(E[i]);
-  unsigned long long inc = mine;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const unsigned long long v = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += v;
-  }
-  if (lane == 63) red[wave] = inc;
-  if (tid == 0) s_tok = -1;
+  const uint32_t kappa = prefix;
+  // the chunks' kept masses: lower bins whole, the cut bin's keys from kappa up
+  each([&](uint32_t k, unsigned long long q, int c) {
+    if (k >= kappa) atomicAdd(&kpart[c], q);
+  });
   __syncthreads();
-  unsigned long long wb = cbase;
-  for (int w = 0; w < wave; ++w) wb += red[w];
-  const unsigned long long exc = wb + inc - mine;
-  if (mine > 0 && exc <= t && t < exc + mine) {
-    unsigned long long cum = exc;
-    for (int i = beg; i < end; ++i) {
-      if (order_key(L[i] / temperature) >= kappa) {
-        cum += fix_mass(E[i]);
-        if (cum > t) {
-          s_tok = i;
-          break;
-        }
-      }
+  // t, and the chunk holding it (kept masses in chunk order = token-id order)
+  if (wave == 0) {
+    const unsigned long long kp = kpart[lane], inc = wave_scan(kp);
+    const unsigned long long zk = __shfl(inc, 63, 64);
+    const uint64_t bits = splitmix64(synth_base(seed, 0x70707070ull + (uint64_t)row) + step) >> 40;
+    const unsigned long long t = (zk >> 24) * bits + (((zk & 0xFFFFFFull) * bits) >> 24);
+    const unsigned long long hit = __ballot(inc > t);
+    const int c = hit ? __ffsll((long long)hit) - 1 : kTopPChunks - 1;
+    if (lane == c) {
+      s_chunk = c;
+      s_t = t - (inc - kp);  // within the chunk
     }
   }
   __syncthreads();
+  // the chunk's tokens in token-id order, kTopPThreads at a time
+  const int cbeg = min(vocab, s_chunk * cl), cend = min(vocab, cbeg + cl);
+  unsigned long long base = 0;
+  for (int i0 = cbeg; i0 < cend; i0 += kTopPThreads) {
+    const int i = i0 + tid;
+    unsigned long long q = 0;
+    if (i < cend) {
+      const float sv = L[i] / temperature;
+      if (order_key(sv) >= kappa) q = fix_mass(expf(sv - mx));
+    }
+    unsigned long long inc = wave_scan(q);
+    if (lane == 63) red[wave] = inc;
+    __syncthreads();
+    unsigned long long all = 0;
+#pragma unroll
+    for (int w = 0; w < kTopPThreads / 64; ++w) {
+      if (w < wave) inc += red[w];
+      all += red[w];
+    }
+    inc += base;
+    if (q && inc - q <= s_t && s_t < inc) s_tok = i;  // exactly one token
+    base += all;
+    __syncthreads();
+  }
   if (tid == 0) out[row] = s_tok;
 }
 
 }  // namespace
 
-static_assert(kTopPScratchBytes >= kTopPScratchFloats * sizeof(float) +
-                                    kTopPNoallocRows * sizeof(TopPRow),
+static_assert(kTopPScratchBytes >= kTopPNoallocRows * sizeof(TopPRow),
               "the static scratch holds the largest no-allocation workspace");
 
 // ---------------------------------------------------------------- no-allocation scratch
-// The top-p sampler's workspace (the [rows][vocab] fp32 exponentials, then a TopPRow per row)
-// for the entry point that takes none: a file-scope device array of kTopPScratchBytes (8 MiB of
-// exponentials for up to kTopPNoallocRows rows of 131072, and their TopPRows), one copy per GPU
+// The top-p sampler's workspace (a TopPRow per row) for the entry point that takes none: a
+// file-scope device array of kTopPScratchBytes (kTopPNoallocRows TopPRows), one copy per GPU
 // for the life of the process.  Host code never passes `scratch` itself to a kernel (on the
 // host the name is only a stand-in, not the device address): top_p_scratch_init looks up each
 // device's address once with hipGetSymbolAddress and the launcher passes that.
@@ -511,10 +528,7 @@ int launch_argmax_rows(int rows, int vocab, const float* logits, int* out,
   return IE_OK;
 }
 
-size_t top_p_workspace_bytes(int rows, int vocab) {
-  const size_t e = ((size_t)rows * (size_t)vocab * sizeof(float) + 255) & ~(size_t)255;
-  return e + (size_t)rows * sizeof(TopPRow);
-}
+size_t top_p_workspace_bytes(int rows) { return (size_t)rows * sizeof(TopPRow); }
 
 int launch_top_p(int rows, int vocab, const float* logits, float temperature, float top_p,
                  uint64_t seed, uint64_t step, int* out, float* ws, hipStream_t st) {
@@ -523,21 +537,21 @@ int launch_top_p(int rows, int vocab, const float* logits, float temperature, fl
   IE_REQUIRE(temperature > 0.f, "top_p: temperature must be > 0 (got %g)", (double)temperature);
   IE_REQUIRE(top_p > 0.f && top_p <= 1.f, "top_p: top_p must be in (0, 1] (got %g)",
              (double)top_p);
-  TopPRow* R = reinterpret_cast<TopPRow*>(reinterpret_cast<char*>(ws) +
-                                          (top_p_workspace_bytes(rows, vocab) -
-                                           (size_t)rows * sizeof(TopPRow)));
+  TopPRow* R = reinterpret_cast<TopPRow*>(ws);
+  // The last bin that can hold the cut: the largest token alone has mass 1, the tokens past d
+  // nats at most vocab exp(-d), and the cut lies before the point where what is past it falls
+  // below the (1 - p) Z left out (half of it, for the roundings).
+  const double left = 1.0 - (double)top_p;
+  const double d0 = left > 1e-9 ? std::log(2.0 * vocab / left) : 28.0;
+  const int last_bin = (int)std::min<double>(kTopPBins - 1, d0 * kTopPBinScale + 1);
   const dim3 chunks(kTopPChunks, rows);
   hipLaunchKernelGGL(tp_max_kernel, chunks, dim3(kTopPChunkThreads), 0, st, logits, vocab, R);
   hipLaunchKernelGGL(tp_hist_kernel, chunks, dim3(kTopPChunkThreads), 0, st, logits, vocab,
-                     temperature, R, ws);
+                     temperature, last_bin, R);
   hipLaunchKernelGGL(tp_gather_kernel, chunks, dim3(kTopPChunkThreads), 0, st, logits, vocab,
-                     temperature, top_p, R, ws);
-  hipLaunchKernelGGL(tp_select_kernel, dim3(rows), dim3(kTopPThreads), 0, st, logits, vocab,
-                     temperature, R, ws);
-  hipLaunchKernelGGL(tp_kept_kernel, chunks, dim3(kTopPChunkThreads), 0, st, logits, vocab,
-                     temperature, R, ws);
-  hipLaunchKernelGGL(tp_walk_kernel, dim3(rows), dim3(kTopPChunkThreads), 0, st, logits, vocab,
-                     temperature, seed, step, R, ws, out);
+                     temperature, top_p, R);
+  hipLaunchKernelGGL(tp_finish_kernel, dim3(rows), dim3(kTopPThreads), 0, st, logits, vocab,
+                     temperature, seed, step, R, out);
   IE_CHECK_LAUNCH();
   return IE_OK;
 }

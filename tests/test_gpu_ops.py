@@ -836,6 +836,36 @@ def test_top_p_ties_and_flat_rows(hip, ctx):
             assert int(out[r].item()) == want, (r, step, int(out[r].item()), want)
 
 
+# chunks of one token, empty chunks (vocab 7, 65), two rounds a chunk (131072), ragged ones; nearly
+# nothing left out (p = 1: every bin can hold the cut) and nearly everything; spreads that put more
+# candidates in the cut bin than tp_finish keeps in LDS (0.25) and than the list holds (0.1)
+@pytest.mark.parametrize("vocab,temperature,p,std", [(7, 1.0, 0.5, 1.0), (65, 0.7, 0.9, 2.0),
+                                                     (1000, 1.0, 1.0, 3.0), (50001, 0.4, 0.02, 2.0),
+                                                     (131072, 1.2, 0.98, 2.0), (V, 1.0, 0.7, 0.25),
+                                                     (V, 1.0, 0.5, 0.1), (V, 2.0, 1.0, 4.0)])
+def test_top_p_shapes(hip, ctx, vocab, temperature, p, std):
+    """Top-p sampling at the edges of its chunks, bins and candidate list: the oracle's tokens (the
+    masses are exact; a t within 1e-6 of a token's edge may fall on either side, as expf's last
+    bit differs between host and device)."""
+    say(f"top-p vocab={vocab} T={temperature} p={p} std={std}")
+    rng = np.random.default_rng(vocab + int(100 * p))
+    lg = (rng.standard_normal((3, vocab)) * std).astype(np.float32)
+    lg[1, ::3] = -np.inf        # masked tokens
+    lg[2] = lg[2].round(1)      # ties
+    logits = torch.from_numpy(lg).cuda()
+    out = torch.empty(3, dtype=torch.int32, device="cuda")
+    ws = torch.empty(hip.lib.ie_top_p_workspace_size(3, vocab), dtype=torch.uint8, device="cuda")
+    for step in range(3):
+        hip.check(hip.lib.ie_sample_top_p(ctx.handle, 3, vocab, P(logits), temperature, p, 77, step,
+                                          P(out), P(ws)))
+        sync()
+        for r in range(3):
+            want, info = orc.top_p(lg[r], temperature, p, 77, r, step)
+            margin = min(info["t"] - info["lo"], info["hi"] - info["t"]) / info["z_kept"]
+            if margin > 1e-6:
+                assert int(out[r].item()) == want, (r, step, int(out[r].item()), want)
+
+
 @pytest.mark.parametrize("rows", [2, 4, 5, 8, 9, 16, 17, 64])
 def test_final_norm_lm_head_rows(hip, ctx, rows):
     """The head of 2 .. 64 rows, at the edges of its 4-, 8- and 16-row kernels and of the 16-row
