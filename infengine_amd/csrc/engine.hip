@@ -111,34 +111,26 @@ int qkv_rope_gemv(const ie_layer& L, const ie_rope_weights& rope, const uint16_t
 
 // merge: also write the bf16 attention output to `out` (merge kernel); otherwise only the
 // partials are written, for an O projection that merges them.  max_len: host-known bound on
-// the context lengths; beyond kAttnFusedMaxCtx the splits go up to kAttnSplits (merge only).
+// the context length; beyond kAttnFusedMaxCtx the splits go up to kAttnSplits (merge only).
 // Paged KV (block_table set): kvl is the layer's base inside page 0, n_pages the pool size.
 int attn_decode(const uint16_t* q, uint16_t* kvl, uint16_t* out, const DecodeWs& w,
-                const int* d_seq_len, int seq_len, int max_len, int batch, long long cache_stride,
-                bool merge, hipStream_t st, const int* block_table = nullptr, int table_stride = 0,
-                int n_pages = 0, bool batched = false) {
+                const int* d_seq_len, int seq_len, int max_len, bool merge, hipStream_t st,
+                const int* block_table = nullptr, int n_pages = 0) {
   AttnDecodeParams a{};
   a.q = q;
   a.k_cache = kvl;
   a.v_cache = kvl + (size_t)kKVHeads * (block_table ? kPageHead : kKVPlane);
-  a.cache_batch_stride = cache_stride;
   a.block_table = block_table;
-  a.table_stride = table_stride;
   a.n_pages = n_pages;
   a.out = out;
   a.part_o = w.part_o;
   a.part_ml = w.part_ml;
   a.d_seq_len = d_seq_len;
   a.seq_len = seq_len;
-  // batched step: 16 x 8 (sequence, kv head) workgroups already fill the chip, so up to
-  // kAttnDirectMaxCtx one split per pair writes the output (no merge launch).  At every batch
-  // size, so that a sequence's results do not depend on how many others share its step.
-  a.max_splits = (batched && merge && max_len <= kAttnDirectMaxCtx) ? 1
-                 : max_len <= kAttnFusedMaxCtx                        ? attn_fused_splits(max_len)
-                                                                     : kAttnSplits;
+  a.max_splits = max_len <= kAttnFusedMaxCtx ? attn_fused_splits(max_len) : kAttnSplits;
   IE_REQUIRE(merge || a.max_splits <= kAttnFusedSplitsLong,
              "attn_decode: contexts past %d need the merge kernel", kAttnFusedMaxCtx);
-  return launch_attn_decode(a, batch, merge, st);
+  return launch_attn_decode(a, merge, st);
 }
 
 int gemv_plain(int K, int epi, const uint16_t* x, const uint16_t* norm_w, const uint16_t* w0,
@@ -171,8 +163,8 @@ int decode_layer_tail(hipStream_t st, const ie_layer& L, const uint16_t* q, uint
                       uint16_t* attn_out, const DecodeWs& w, uint16_t* kvl, const int* d_seq_len,
                       int seq_len, const int* block_table = nullptr, int n_pages = 0) {
   const bool fused = attn_fused(seq_len);
-  IE_TRY(attn_decode(q, kvl, attn_out, w, d_seq_len, seq_len, seq_len, 1, 0, !fused, st,
-                     block_table, 0, n_pages));
+  IE_TRY(attn_decode(q, kvl, attn_out, w, d_seq_len, seq_len, seq_len, !fused, st, block_table,
+                     n_pages));
   if (fused) {
     // O projection + residual, its input merged from the split partials in its prologue
     GemvParams p{};
@@ -854,7 +846,7 @@ namespace {
 // rows' partial sums of squares already in w.ss (from the previous layer's down projection or
 // the prep kernel); with ss_next the down projection leaves those of its output rows there.
 int batched_layer(Context* c, hipStream_t st, const ie_model_weights& W, int l, int batch,
-                  int len_class, ie_bf16* data_buffer, ie_bf16* attn_buffer, const DecodeWs& w,
+                  BatchClass cls, ie_bf16* data_buffer, ie_bf16* attn_buffer, const DecodeWs& w,
                   void* kv_caches, const int* block_table, int table_stride, int n_pages,
                   bool ss_next) {
   const int* d_sl = c->d_params + 1;
@@ -888,8 +880,20 @@ int batched_layer(Context* c, hipStream_t st, const ie_model_weights& W, int l, 
   g.x_norm_w = L.input_layernorm;
   skinny_split(c, kGemmQkvRope, g, w.sk_part);
   IE_TRY(launch_gemm(kGemmQkvRope, g, st));
-  IE_TRY(attn_decode(w.q, kvl, attn_buffer, w, d_sl, 0, len_class, batch, cstride, true, st,
-                     block_table, table_stride, n_pages, true));
+  AttnDecodeParams a{};
+  a.q = w.q;
+  a.k_cache = kvl;
+  a.v_cache = g.v_cache;
+  a.cache_batch_stride = cstride;
+  a.block_table = block_table;
+  a.table_stride = table_stride;
+  a.n_pages = n_pages;
+  a.out = attn_buffer;
+  a.part_o = w.part_o;
+  a.part_ml = w.part_ml;
+  a.d_seq_len = d_sl;
+  a.counters = c->d_counters + kCntAttn;
+  IE_TRY(launch_attn_decode_batched(a, batch, cls.max_len, cls.nt, st));
   GemmParams o{};
   o.x = attn_buffer;
   o.w0 = L.transformer.w_o;
@@ -932,11 +936,9 @@ int batched_layer(Context* c, hipStream_t st, const ie_model_weights& W, int l, 
 }
 
 // The kernels of one batched step on stream st, the sequences' lengths already in
-// d_params[1 .. batch].  len_class bounds the longest context and picks the attention path:
-// kAttnDirectMaxCtx (one split per sequence and kv head, no merge launch), kAttnFusedMaxCtx or
-// beyond (split contexts + the merge kernel).
+// d_params[1 .. batch].
 int enqueue_batched(Context* c, hipStream_t st, const ie_model_weights& W, int batch,
-                    int len_class, int* tokenid_buffs, int tokens_stride, ie_bf16* data_buffer,
+                    BatchClass cls, int* tokenid_buffs, int tokens_stride, ie_bf16* data_buffer,
                     ie_bf16* attn_buffer, float* output_distr, int* output_tokens,
                     void* workspace, void* kv_caches, const int* block_table, int table_stride,
                     int n_pages) {
@@ -950,7 +952,7 @@ int enqueue_batched(Context* c, hipStream_t st, const ie_model_weights& W, int b
   // normalise the rows on their way in, with rmsnorm.cu:61's two roundings
   IE_TRY(launch_rmsnorm_prep(batch, data_buffer, w.ss, st));
   for (int l = 0; l < kLayers; ++l)
-    IE_TRY(batched_layer(c, st, W, l, batch, len_class, data_buffer, attn_buffer, w, kv_caches,
+    IE_TRY(batched_layer(c, st, W, l, batch, cls, data_buffer, attn_buffer, w, kv_caches,
                          block_table, table_stride, n_pages, l + 1 < kLayers));
   // prefill.cu:41-43 / decode.cu:41: final RMSNorm of the rows, then the lm_head product
   IE_TRY(launch_rmsnorm(batch, data_buffer, W.final_norm, w.xn, st));
@@ -994,16 +996,10 @@ int batched_step(ie_context* c, const ie_model_weights* weights, int batch, cons
                "(rope_rows)", b, seq_lens[b], rope_rows(*weights));
   }
   hipStream_t st = c->stream;
-  int max_len = 1;
-  for (int b = 0; b < batch; ++b) {
-    c->h_params[1 + b] = seq_lens[b];
-    max_len = std::max(max_len, seq_lens[b]);
-  }
+  for (int b = 0; b < batch; ++b) c->h_params[1 + b] = seq_lens[b];
   IE_CHECK_HIP(hipMemcpyAsync(c->d_params + 1, c->h_params + 1, batch * sizeof(int),
                               hipMemcpyHostToDevice, st));
-  const int len_class = max_len <= kAttnDirectMaxCtx  ? kAttnDirectMaxCtx
-                        : max_len <= kAttnFusedMaxCtx ? kAttnFusedMaxCtx
-                                                      : cap;
+  const BatchClass cls = batch_class(seq_lens, batch, cap);
   if (c->use_graph) {
     // replayed from a graph captured with the same buffers, batch and attention path (the
     // lengths are read from d_params on the device)
@@ -1013,7 +1009,7 @@ int batched_step(ie_context* c, const ie_model_weights* weights, int batch, cons
                            attn_buffer, output_distr, output_tokens, workspace, kv_caches,
                            block_table, (const void*)(intptr_t)table_stride,
                            (const void*)(intptr_t)n_pages, (const void*)(intptr_t)batch,
-                           (const void*)(intptr_t)len_class, nullptr};
+                           (const void*)(intptr_t)(2 * cls.max_len + (cls.nt ? 1 : 0)), nullptr};
     Context::BatchGraph* slot = nullptr;
     for (auto& bg : c->bgraph)
       if (bg.exec && std::memcmp(bg.key, key, sizeof key) == 0) slot = &bg;
@@ -1027,7 +1023,7 @@ int batched_step(ie_context* c, const ie_model_weights* weights, int batch, cons
       }
       hipGraph_t g = nullptr;
       IE_CHECK_HIP(hipStreamBeginCapture(c->capture, hipStreamCaptureModeThreadLocal));
-      const int rc = enqueue_batched(c, c->capture, *weights, batch, len_class, tokenid_buffs,
+      const int rc = enqueue_batched(c, c->capture, *weights, batch, cls, tokenid_buffs,
                                      tokens_stride, data_buffer, attn_buffer, output_distr,
                                      output_tokens, workspace, kv_caches, block_table,
                                      table_stride, n_pages);
@@ -1045,7 +1041,7 @@ int batched_step(ie_context* c, const ie_model_weights* weights, int batch, cons
     slot->used = ++c->bgraph_tick;
     IE_CHECK_HIP(hipGraphLaunch(slot->exec, st));
   } else {
-    IE_TRY(enqueue_batched(c, st, *weights, batch, len_class, tokenid_buffs, tokens_stride,
+    IE_TRY(enqueue_batched(c, st, *weights, batch, cls, tokenid_buffs, tokens_stride,
                            data_buffer, attn_buffer, output_distr, output_tokens, workspace,
                            kv_caches, block_table, table_stride, n_pages));
   }
@@ -1080,23 +1076,18 @@ int ie_decoder_layer_batched(ie_context* c, const ie_model_weights* weights, int
   IE_REQUIRE(batch >= 1 && batch <= 16, "decoder_layer_batched: batch %d out of [1, 16]", batch);
   IE_REQUIRE(seq_lens && data_buffer && attn_buffer && workspace && kv_caches,
              "decoder_layer_batched: null buffer");
-  int max_len = 1;
   for (int b = 0; b < batch; ++b) {
     IE_REQUIRE(seq_lens[b] >= 1 && seq_lens[b] <= kMaxCtx,
                "decoder_layer_batched: seq_lens[%d]=%d out of [1, %d]", b, seq_lens[b], kMaxCtx);
     c->h_params[1 + b] = seq_lens[b];
-    max_len = std::max(max_len, seq_lens[b]);
   }
   hipStream_t st = c->stream;
   IE_CHECK_HIP(hipMemcpyAsync(c->d_params + 1, c->h_params + 1, batch * sizeof(int),
                               hipMemcpyHostToDevice, st));
-  // the attention path ie_decode_step_batched takes for these lengths
-  const int len_class = max_len <= kAttnDirectMaxCtx  ? kAttnDirectMaxCtx
-                        : max_len <= kAttnFusedMaxCtx ? kAttnFusedMaxCtx
-                                                      : kMaxCtx;
+  const BatchClass cls = batch_class(seq_lens, batch, kMaxCtx);
   const DecodeWs w = decode_ws(workspace, batch);
   IE_TRY(launch_rmsnorm_prep(batch, data_buffer, w.ss, st));
-  IE_TRY(batched_layer(c, st, *weights, layer_idx, batch, len_class, data_buffer, attn_buffer, w,
+  IE_TRY(batched_layer(c, st, *weights, layer_idx, batch, cls, data_buffer, attn_buffer, w,
                        kv_caches, nullptr, 0, 0, false));
   // the lengths' pinned staging is reused by the next call
   IE_CHECK_HIP(hipStreamSynchronize(st));
@@ -1514,7 +1505,7 @@ int ie_decode_attn(ie_context* c, const float* d_rope_cos, const float* d_rope_s
   L.transformer.w_v = const_cast<ie_bf16*>(d_vproj);
   ie_rope_weights rope{const_cast<float*>(d_rope_cos), const_cast<float*>(d_rope_sin)};
   IE_TRY(qkv_rope_gemv(L, rope, d_input, nullptr, w.q, kvl, nullptr, seq_len - 1, st));
-  IE_TRY(attn_decode(w.q, kvl, w.attn1, w, nullptr, seq_len, seq_len, 1, 0, true, st));
+  IE_TRY(attn_decode(w.q, kvl, w.attn1, w, nullptr, seq_len, seq_len, true, st));
   return gemv_plain(kHidden, kEpiBf16, w.attn1, nullptr, d_oproj, nullptr, kHidden / 2, d_output,
                     nullptr, 1, kHidden, st);
 }

@@ -35,7 +35,7 @@ constexpr size_t kPageHead = (size_t)kPagePos * kHeadDim;              // one he
 constexpr size_t kPageLayer = 2 * (size_t)kKVHeads * kPageHead;        // one layer in a page
 constexpr size_t kPageElems = (size_t)kLayers * kPageLayer;            // elements per page
 
-// Decode attention splits the context of each KV head over this many blocks.
+// Decode attention splits the context of each KV head over at most this many blocks.
 constexpr int kAttnSplits = 32;
 constexpr int kAttnTile = 64;
 
@@ -284,7 +284,9 @@ constexpr int kCntArgmax = 0;  // [64][kCntStride] argmax rows
 // kSkTailMax tiles per launch.
 constexpr int kSkTailMax = 256;
 constexpr int kCntSkinny = kCntArgmax + kNumSlots * kCntStride;  // [kSkTailMax][kCntStride]
-constexpr int kNumCounters = kCntSkinny + kSkTailMax * kCntStride;
+// the batched attention's arrival counters, one per (sequence, kv head)
+constexpr int kCntAttn = kCntSkinny + kSkTailMax * kCntStride;  // [16 x 8][kCntStride]
+constexpr int kNumCounters = kCntAttn + 16 * kKVHeads * kCntStride;
 
 inline hipStream_t stream_of(void* s) { return reinterpret_cast<hipStream_t>(s); }
 

@@ -59,8 +59,8 @@ struct AttnDecodeParams {
   float* part_ml;           // [batch][8][splits][4][2]
   const int* d_seq_len;     // [batch] device seq lens, or nullptr
   int seq_len;              // used when d_seq_len == nullptr (batch must be 1)
-  int max_splits;           // splits per kv head cap: kAttnFusedSplits or kAttnSplits (1: the
-                            // kernel writes the normalised bf16 output itself)
+  int max_splits;           // splits per kv head cap (batch 1): kAttnFusedSplits or kAttnSplits
+  unsigned int* counters;   // batched: zeroed arrival counters [batch x 8], kCntStride apart
 };
 // Splits per (sequence, kv head) for a context of ntiles 64-row tiles: four tiles per split
 // (one per wave of the split workgroup) up to the cap.  Device and host must agree on it.
@@ -80,9 +80,30 @@ inline int attn_fused_splits(int max_len) {
   return max_len <= kAttnFusedShortCtx ? kAttnFusedSplits : kAttnFusedSplitsLong;
 }
 constexpr int kAttnFusedMaxCtx = 4096;  // beyond: merge kernel + up to kAttnSplits splits
-constexpr int kAttnDirectMaxCtx = 2048; // batched contexts up to this: one split, output written directly
-// merge = also launch the merge kernel (bf16 output in p.out)
-int launch_attn_decode(const AttnDecodeParams& p, int batch, bool merge, hipStream_t st);
+// Batched steps up to here: a sequence's attention does not depend on what shares its step.
+constexpr int kAttnShortMaxCtx = 2048;
+// What the batched step's kernels take from the host's view of the lengths (a step is captured per
+// class): a bound on the longest (the attention's grid) and whether the sequences' K/V of all
+// layers exceed the 256 MB Infinity Cache (2048 positions of 128 KiB).  Past that nothing of a
+// layer's K/V is left when the next step reads it and the nontemporal policy streams better
+// (per layer: 6 sequences of 2500-20000 66 -> 58 us, 16 of 75-600 13.2 -> 11.7); within it the
+// default policy finds it there (2 of 75-600: 7.5 against 9.4 us).
+struct BatchClass {
+  int max_len;
+  bool nt;
+};
+inline BatchClass batch_class(const int* lens, int batch, int cap) {
+  int longest = 1;
+  long long total = 0;
+  for (int b = 0; b < batch; ++b) longest = lens[b] > longest ? lens[b] : longest, total += lens[b];
+  return {longest <= kAttnShortMaxCtx ? kAttnShortMaxCtx : cap, total > 2048};
+}
+// Batch 1.  merge = also launch the merge kernel (bf16 output in p.out)
+int launch_attn_decode(const AttnDecodeParams& p, bool merge, hipStream_t st);
+// Up to 16 sequences, none longer than max_len (which sizes the grid): bf16 output in p.out.
+// nt: nontemporal K/V loads.
+int launch_attn_decode_batched(const AttnDecodeParams& p, int batch, int max_len, bool nt,
+                               hipStream_t st);
 size_t attn_decode_partials_bytes(int batch);
 
 // ------------------------------------------------------------ elementwise

@@ -25,6 +25,8 @@
 // batched GEMM path and long contexts (max_splits = 32).  A device-scope "last
 // workgroup merges" scheme is not used: its fence (L2 write-back / invalidate on
 // this multi-XCD part) per workgroup cost more than a launch.
+#include <algorithm>
+
 #include "ie_kernels.h"
 
 namespace ie {
@@ -37,7 +39,7 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) short4_t lds_short4;
 
-constexpr int kSplitWaves = 4;
+constexpr int kBatchedWaves = 12, kBatchedTile = 32;
 constexpr int kRowBytes = kHeadDim * 2;
 constexpr int kBufferFlags = 0x00020000;   // buffer descriptor word 3 (raw 32-bit access)
 static_assert(kAttnTile == 64, "tile = 4 x 16-key MFMA blocks");
@@ -50,43 +52,39 @@ static_assert(kAttnSplits <= 64, "the merge gives each split one lane");
 // kSplitWaves waves, the longest context keeps that within 64 tiles per wave.
 static_assert(kMaxLongCtx / kAttnTile <= 64 * kAttnSplits * 4, "page ids per wave exceed a wave");
 
-// Phase 1: split s of (batch b, kv head g) attends its run of tiles (its NW waves take every
-// NW-th tile) and writes the unnormalised partial (m, l, o) of each of the 4 q heads; with one
-// split (max_splits = 1, batched: 12 waves on 32-key tiles) it writes the normalised bf16 output
-// instead.  VREG: one LDS slice per wave, K through it and V staged in registers then written over
-// K (72 KiB per 4-wave workgroup of 64-key tiles, two workgroups per CU: the batched split grid;
-// 120 KiB for the 12-wave form); otherwise K and V each have a slice (136 KiB, one workgroup per
-// CU; 0.7% faster per decode step at batch 1 than K fragments loaded straight into registers).
-// The batched one-split form takes 32-key tiles so that 12 waves (3 per SIMD within the registers)
-// cover a context of 17-24 half tiles in two rounds of half the work: 10.6 against 11.8 us per
-// layer for 8 waves on 64-key tiles at bs = 16, S = 517-564, where one wave's ninth full tile
-// ended each workgroup ~3 us after the others.  The batch-1 split form likewise runs 8 waves on
-// 32-key tiles (the same tiles per split, half the work per wave): 4.85 against 5.07 us at
-// S = 550-610.  Splits are counted in 64-key tiles whatever the tile, as the merge counts them.
-template <bool VREG, int NW, int KT = kAttnTile>
-__global__ __launch_bounds__(NW * 64) void attn_decode_split_kernel(AttnDecodeParams p) {
+// A workgroup's LDS, each array its own variable (the compiler then sees that the tile loads do not
+// write the partials): per wave its K tile (then V over it) and V tile, and the 4 heads' partials.
+template <bool VREG, int KT>
+using KvSlice = u32x4_t[VREG ? 1 : 2][KT * 16];
+using PartO = float[kGQA][kHeadDim];
+using PartMl = float[kGQA][2];
+
+// The tiles t0 .. t1-1 (KT keys each) of (sequence b, kv head g) with S positions: the NW waves
+// take every NW-th tile and leave their partials (m, l, o) of the 4 q heads in xo / xml
+// (a barrier ends it).  VREG: one LDS slice per wave, K through it and V staged in registers then
+// written over K (120 KiB for the 12-wave form); otherwise K and V each have a slice (136 KiB, one
+// workgroup per CU; 0.7% faster per decode step at batch 1 than K fragments loaded straight into
+// registers).
+// 32-key tiles: with 12 waves (batched: 3 per SIMD within the registers) a context of 17-24 half
+// tiles is two rounds of half the work: 10.6 against 11.8 us per layer for 8 waves on 64-key
+// tiles at bs = 16, S = 517-564, where one wave's ninth full tile ended each workgroup ~3 us after
+// the others.  The batch-1 split form likewise runs 8 waves on 32-key tiles (the same tiles per
+// split, half the work per wave): 4.85 against 5.07 us at S = 550-610.
+// AUX: the loads' cache policy (0, or 2: nontemporal).
+template <bool VREG, int NW, int KT, int AUX>
+__device__ __forceinline__ void attend_tiles(const AttnDecodeParams& p, int tid, int b, int g, int S,
+                                             int t0, int t1, KvSlice<VREG, KT>* kv, PartO* xo,
+                                             PartMl* xml) {
   // KT: keys per tile, 64 or 32 (half tiles: twice the waves on a context's tiles; a page
   // holds two)
   static_assert(KT == 64 || KT == 32, "tile of 64 or 32 keys");
   constexpr int KB = KT / 16;   // 16-key MFMA blocks per tile
   constexpr int KS2 = KT / 32;  // 32-key P.V contraction chunks per tile
   constexpr int NJ = KT / 4;    // 1 KiB loads per tile (4 rows each)
-  const int split = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
   // wave id made provably uniform: the tile indices and buffer descriptors derived from it stay
   // in SGPRs (otherwise every buffer load becomes a readfirstlane loop)
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, G = lane >> 4;
-  const int S = p.d_seq_len ? p.d_seq_len[b] : p.seq_len;
-  const int ntiles = (S + KT - 1) / KT;
-  // (split count in 64-key tiles whatever KT: the merge and the O projection count the same)
-  const int ns = attn_decode_splits((S + kAttnTile - 1) / kAttnTile, p.max_splits);
-  if (split >= ns) return;  // whole workgroup: nobody reads a partial past ns
-  const int tps = (ntiles + ns - 1) / ns;
-  const int t0 = split * tps, t1 = min(ntiles, t0 + tps);
-
-  __shared__ u32x4_t kvlds[NW][VREG ? 1 : 2][KT * 16];  // per wave: K tile (then V over it), V tile
-  __shared__ float xo[NW][kGQA][kHeadDim];
-  __shared__ float xml[NW][kGQA][2];
   const uint16_t* Kh = p.k_cache + (size_t)b * p.cache_batch_stride + (size_t)g * kKVPlane;
   const uint16_t* Vh = p.v_cache + (size_t)b * p.cache_batch_stride + (size_t)g * kKVPlane;
   // rows past S read as zero (buffer bounds) and are masked below
@@ -112,8 +110,8 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_split_kernel(AttnDecodePa
   f32x4_t o[8];
 #pragma unroll
   for (int db = 0; db < 8; ++db) o[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  u32x4_t* kt = kvlds[wave][0];
-  u32x4_t* vt = kvlds[wave][VREG ? 0 : 1];
+  u32x4_t* kt = kv[wave][0];
+  u32x4_t* vt = kv[wave][VREG ? 0 : 1];
 
   // paged KV: lane i holds the page of this wave's i-th tile (one load ahead of the loop)
   const bool paged = p.block_table != nullptr;
@@ -150,7 +148,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_split_kernel(AttnDecodePa
     for (int j = 0; j < NJ; ++j) {
       const int r = 4 * j + G;
       const uint32_t off = (uint32_t)((kr0 + r) * kRowBytes + ((fr ^ (r & 15)) * 16));
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (lds_void*)&kt[64 * j], 16, off, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (lds_void*)&kt[64 * j], 16, off, 0, 0, AUX);
       if constexpr (!VREG)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(vrs, (lds_void*)&vt[64 * j], 16, off, 0, 0, 0);
     }
@@ -158,7 +156,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_split_kernel(AttnDecodePa
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
         vv[j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
-            vrs, (uint32_t)((kr0 + 4 * j + G) * kRowBytes + fr * 16), 0, 0));
+            vrs, (uint32_t)((kr0 + 4 * j + G) * kRowBytes + fr * 16), 0, AUX));
     }
     // K fragments kk[kb][ks] = K[key0 + 16 kb + fr][32 ks + 8 G .. +8] from the LDS tile
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(VREG ? NJ : 0) : "memory");
@@ -257,43 +255,224 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_split_kernel(AttnDecodePa
     }
   }
   __syncthreads();
-  if (wave >= kGQA) return;  // (NW > 4) waves past the 4 q heads only contribute partials
-  const int h = wave;  // wave h merges q head 4g + h; lane d owns dims 2d, 2d+1
+}
+
+// Wave h (of the first 4) merges the waves' partials of q head 4g + h: lane d receives the
+// unnormalised dims 2d, 2d+1, and the max and sum.
+struct AttnMerged {
+  float o0, o1, M, L;
+};
+template <int NW>
+__device__ __forceinline__ AttnMerged merge_waves(const PartO* xo, const PartMl* xml, int h, int lane) {
   const float mw = lane < NW ? xml[lane][h][0] : -INFINITY;
   const float lw = lane < NW ? xml[lane][h][1] : 0.f;
-  const float M = wave_max(mw);
-  const float wl = lw > 0.f ? __expf(mw - M) : 0.f;
-  const float L = wave_sum(lw * wl);
-  float o0 = 0.f, o1 = 0.f;
+  AttnMerged r{0.f, 0.f, wave_max(mw), 0.f};
+  const float wl = lw > 0.f ? __expf(mw - r.M) : 0.f;
+  r.L = wave_sum(lw * wl);
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
     const float ww = readlane_f(wl, w);
-    o0 = fmaf(xo[w][h][2 * lane], ww, o0);
-    o1 = fmaf(xo[w][h][2 * lane + 1], ww, o1);
+    r.o0 = fmaf(xo[w][h][2 * lane], ww, r.o0);
+    r.o1 = fmaf(xo[w][h][2 * lane + 1], ww, r.o1);
   }
-  if (p.max_splits == 1) {
-    // one split: the merged result is final (attn.cu:433-438), no partials
-    const float inv = 1.0f / L;
-    uint32_t* dst = reinterpret_cast<uint32_t*>(p.out + ((size_t)b * kQHeads + g * kGQA + h) * kHeadDim);
-    dst[lane] = pack_bf2(o0 * inv, o1 * inv);
-    return;
-  }
-  const size_t slot = (((size_t)b * kKVHeads + g) * kAttnSplits + split) * kGQA + h;
-  *reinterpret_cast<float2*>(p.part_o + slot * kHeadDim + 2 * lane) = make_float2(o0, o1);
-  if (lane == 0) *reinterpret_cast<float2*>(p.part_ml + slot * 2) = make_float2(M, L);
+  return r;
 }
 
-// Phase 2 (next kernel on the stream, so phase 1's writes are visible): one
-// workgroup per (batch, kv head), wave w merges q head 4g + w.  Lane s holds
+// Batch 1, phase 1: split s of kv head g attends its run of tiles and writes the unnormalised
+// partial (m, l, o) of each of the 4 q heads.  Splits are counted in 64-key tiles whatever the
+// tile, as the merge counts them.
+template <int NW, int KT>
+__global__ __launch_bounds__(NW * 64) void attn_decode_split_kernel(AttnDecodeParams p) {
+  __shared__ KvSlice<false, KT> kv[NW];
+  __shared__ PartO xo[NW];
+  __shared__ PartMl xml[NW];
+  const int split = blockIdx.x, g = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int S = p.d_seq_len ? p.d_seq_len[0] : p.seq_len;
+  const int ntiles = (S + KT - 1) / KT;
+  // (split count in 64-key tiles whatever KT: the merge and the O projection count the same)
+  const int ns = attn_decode_splits((S + kAttnTile - 1) / kAttnTile, p.max_splits);
+  if (split >= ns) return;  // whole workgroup: nobody reads a partial past ns
+  const int tps = (ntiles + ns - 1) / ns;
+  const int t0 = split * tps, t1 = min(ntiles, t0 + tps);
+  attend_tiles<false, NW, KT, 0>(p, threadIdx.x, 0, g, S, t0, t1, kv, xo, xml);
+  if (wave >= kGQA) return;  // (NW > 4) waves past the 4 q heads only contribute partials
+  const AttnMerged r = merge_waves<NW>(xo, xml, wave, lane);
+  const size_t slot = ((size_t)g * kAttnSplits + split) * kGQA + wave;
+  *reinterpret_cast<float2*>(p.part_o + slot * kHeadDim + 2 * lane) = make_float2(r.o0, r.o1);
+  if (lane == 0) *reinterpret_cast<float2*>(p.part_ml + slot * 2) = make_float2(r.M, r.L);
+}
+
+template <int CTRL>
+__device__ __forceinline__ int dpp_i(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+}
+
+// Two floats to / from memory past the XCDs' L2s (device-scope accesses): what one workgroup hands
+// to another within a launch.
+__device__ __forceinline__ void agent_store2(float* p, float a, float b) {
+  const uint64_t v = (uint64_t)__float_as_uint(b) << 32 | __float_as_uint(a);
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 agent_load2(const float* p) {
+  const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+  return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
+}
+
+// The partials of q head 4g + h of (sequence, kv head) bg merged in run order; every lane's loads
+// of 8 runs in flight at a time (indices clamped to the last run).
+__device__ __forceinline__ AttnMerged merge_runs(const AttnDecodeParams& p, size_t bg, int h,
+                                                 int lane, int ns) {
+  const size_t slot0 = bg * kAttnSplits * kGQA + h;
+  const float2 ml = agent_load2(p.part_ml + (slot0 + (size_t)min(lane, ns - 1) * kGQA) * 2);
+  const float ms = lane < ns ? ml.x : -INFINITY, ls = lane < ns ? ml.y : 0.f;
+  AttnMerged r{0.f, 0.f, wave_max(ms), 0.f};
+  const float wl = ls > 0.f ? __expf(ms - r.M) : 0.f;
+  r.L = wave_sum(ls * wl);
+  for (int s0 = 0; s0 < ns; s0 += 8) {
+    float2 ov[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      ov[u] = agent_load2(p.part_o + (slot0 + (size_t)min(s0 + u, ns - 1) * kGQA) * kHeadDim + 2 * lane);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float ww = s0 + u < ns ? __shfl(wl, s0 + u, 64) : 0.f;
+      r.o0 = fmaf(ov[u].x, ww, r.o0);
+      r.o1 = fmaf(ov[u].y, ww, r.o1);
+    }
+  }
+  return r;
+}
+
+// Rounds of the waves in a run (of one (sequence, kv head)'s tiles), for a lane's sequence of
+// ntiles tiles.  SHORT (no sequence past kAttnShortMaxCtx): by the sequence's own length, so that
+// its result does not depend on what shares its step: two rounds where one such run covers it (a
+// second run of a short context costs more than its round), else one (more workgroups at once: 2
+// sequences of 225-1800 take 11 us, 21 in one run each).  Otherwise one for the whole batch: the
+// candidate with the least (workgroups' turns, half counted whole) x (rounds + 0.5, an item's
+// own cost) whose longest sequence has at most kAttnSplits runs.  Measured / fixed at 1, 2, 3, 4, 6
+// rounds, us a layer: 16 sequences of 2850-7000 85, 70, 68, 75, 73; 6 of 2500-20000 60 (2 rounds
+// at the longest), 66, 66, 57, 67; 2 of 20000 37, 37, 43, 31, 35.
+template <bool SHORT, int NW>
+__device__ __forceinline__ int run_rounds(int ntiles) {
+  if constexpr (SHORT) return ntiles <= 2 * NW ? 2 : 1;
+  int most = ntiles;
+  most = max(most, dpp_i<kDppQuadXor1>(most));
+  most = max(most, dpp_i<kDppQuadXor2>(most));
+  most = max(most, dpp_i<kDppRowHalfMirror>(most));
+  most = max(most, dpp_i<kDppRowMirror>(most));
+  const int r0 = max(1, (most + kAttnSplits * NW - 1) / (kAttnSplits * NW));  // (1: unused lanes)
+  int best = r0, best_cost = 0x7fffffff;
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    const int r = r0 + c;
+    int items = (ntiles + r * NW - 1) / (r * NW);
+    items += dpp_i<kDppQuadXor1>(items);
+    items += dpp_i<kDppQuadXor2>(items);
+    items += dpp_i<kDppRowHalfMirror>(items);
+    items += dpp_i<kDppRowMirror>(items);
+    items *= kKVHeads;
+    const int cost = ((items + 255) / 256 * 256 + items) * (2 * r + 1);
+    if (cost < best_cost) best = r, best_cost = cost;
+  }
+  return best;
+}
+
+// Batched: one launch over the work items (sequence, kv head, run of its tiles; run_rounds).  A
+// sequence of one run writes its output; the others' partials go out by device-scope stores and
+// the last run of a (sequence, kv head) to arrive (a device-scope counter, reset by it) merges them
+// in run order -- no workgroup waits, and no merge launch.
+// Workgroups (one a CU: 120 KiB of LDS) walk the items a grid apart; an item list, since a grid of
+// (most runs) x 8 x batch would hold mostly idle workgroups, which take their turns on the CUs.
+// Bound by the K/V loads (a copy without the arithmetic took the same time): 5.0-5.6 TB/s past
+// 100 MB a layer.  Before (one 12-wave workgroup per (sequence, kv head) up to 2048 positions, else
+// up to 32 splits of 4-wave workgroups and a merge launch), us a layer with the K/V from HBM: 16
+// sequences of 225-1800 25.3, now 23.2; 2 of them 20.7, 11.5; 16 of 375-3000 37, 33; 16 of
+// 2850-7000 86, 69; 6 of 2500-20000 67, 57.
+// NT: nontemporal K/V loads, for K/V that cannot stay in the 256 MB cache until the next step.
+template <int NW, int KT, bool SHORT, bool NT>
+__global__ __launch_bounds__(NW * 64) void attn_decode_batched_kernel(AttnDecodeParams p, int batch) {
+  __shared__ KvSlice<true, KT> kv[NW];
+  __shared__ PartO xo[NW];
+  __shared__ PartMl xml[NW];
+  __shared__ int s_last;
+  __shared__ int2 s_seq[16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // lane b: sequence b's length and the runs of the sequences up to it.  The first item takes
+  // them from registers; LDS keeps them for the next ones (through the tiles they would cost
+  // registers that those need)
+  int len = lane < batch ? p.d_seq_len[lane] : 0;
+  const int nt = (len + KT - 1) / KT;
+  int rounds = run_rounds<SHORT, NW>(nt);
+  if constexpr (!SHORT) rounds = __builtin_amdgcn_readlane(rounds, 0);  // (one for the batch)
+  int upto = lane < batch ? (nt + rounds * NW - 1) / (rounds * NW) : 0;
+  upto += dpp_i<0x111>(upto);  // row_shr 1, 2, 4, 8: inclusive scan of 16 lanes
+  upto += dpp_i<0x112>(upto);
+  upto += dpp_i<0x114>(upto);
+  upto += dpp_i<0x118>(upto);
+  if (threadIdx.x < 16) s_seq[threadIdx.x] = make_int2(upto, len);  // (read past a barrier)
+  const int total = __builtin_amdgcn_readlane(upto, 15) * kKVHeads;
+  for (int w = blockIdx.x; w < total; w += gridDim.x) {
+    const int b = __popcll(__ballot(lane < batch && upto * kKVHeads <= w));
+    const int S = __builtin_amdgcn_readlane(len, b);
+    const int ntiles = (S + KT - 1) / KT;
+    const int tps = NW * (SHORT ? run_rounds<SHORT, NW>(ntiles) : rounds);
+    const int ns = (ntiles + tps - 1) / tps;
+    const int i = w - (__builtin_amdgcn_readlane(upto, b) - ns) * kKVHeads;
+    const int g = i % kKVHeads, split = i / kKVHeads;
+    // (the thread id made opaque per item: what is derived from it is not kept across the loop)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    attend_tiles<true, NW, KT, NT ? 2 : 0>(p, tid, b, g, S, split * tps, min(ntiles, split * tps + tps),
+                                             kv, xo, xml);
+    const size_t bg = (size_t)b * kKVHeads + g;
+    AttnMerged r{};
+    if (wave < kGQA) {
+      r = merge_waves<NW>(xo, xml, wave, lane);
+      if (ns > 1) {
+        const size_t slot = (bg * kAttnSplits + split) * kGQA + wave;
+        agent_store2(p.part_o + slot * kHeadDim + 2 * lane, r.o0, r.o1);
+        if (lane == 0) agent_store2(p.part_ml + slot * 2, r.M, r.L);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // performed, before the arrival counts
+      }
+    }
+    bool mine = true;
+    if (ns > 1) {
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        unsigned int* cnt = p.counters + bg * kCntStride;
+        const unsigned int old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = old == (unsigned)(ns - 1);
+        if (s_last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __syncthreads();
+      mine = s_last != 0;
+      if (mine && wave < kGQA) r = merge_runs(p, bg, wave, lane, ns);
+    }
+    if (mine && wave < kGQA) {
+      // (attn.cu:433-438)
+      const float inv = 1.0f / r.L;
+      uint32_t* dst = reinterpret_cast<uint32_t*>(p.out + (bg * kGQA + wave) * kHeadDim);
+      dst[lane] = pack_bf2(r.o0 * inv, r.o1 * inv);
+    }
+    __syncthreads();  // the LDS is the next item's
+    upto = s_seq[lane & 15].x;
+    len = s_seq[lane & 15].y;
+  }
+}
+
+// Batch 1, phase 2 (next kernel on the stream, so phase 1's writes are visible): one
+// workgroup per kv head, wave w merges q head 4g + w.  Lane s holds
 // split s's (m, l); every partial load is issued up front (one memory latency).
 __global__ __launch_bounds__(256) void attn_decode_merge_kernel(AttnDecodeParams p) {
-  const int g = blockIdx.x, b = blockIdx.y;
+  const int g = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int h = g * kGQA + wave;
-  const int S = p.d_seq_len ? p.d_seq_len[b] : p.seq_len;
+  const int S = p.d_seq_len ? p.d_seq_len[0] : p.seq_len;
   const int ns = attn_decode_splits((S + kAttnTile - 1) / kAttnTile, p.max_splits);
   __shared__ float wsh[4][64];
-  const size_t slot0 = (((size_t)b * kKVHeads + g) * kAttnSplits) * kGQA + wave;
+  const size_t slot0 = (size_t)g * kAttnSplits * kGQA + wave;
   float ms = -INFINITY, ls = 0.f;
   if (lane < ns) {
     const float2 v = *reinterpret_cast<const float2*>(p.part_ml + (slot0 + lane * kGQA) * 2);
@@ -319,7 +498,7 @@ __global__ __launch_bounds__(256) void attn_decode_merge_kernel(AttnDecodeParams
     o1 = fmaf(ov[sp].y, w, o1);
   }
   const float inv = 1.0f / L;
-  uint32_t* dst = reinterpret_cast<uint32_t*>(p.out + ((size_t)b * kQHeads + h) * kHeadDim);
+  uint32_t* dst = reinterpret_cast<uint32_t*>(p.out + (size_t)h * kHeadDim);
   dst[lane] = pack_bf2(o0 * inv, o1 * inv);
 }
 
@@ -330,33 +509,44 @@ size_t attn_decode_partials_bytes(int batch) {
   return slots * kHeadDim * sizeof(float) + slots * 2 * sizeof(float);
 }
 
-int launch_attn_decode(const AttnDecodeParams& p, int batch, bool merge, hipStream_t st) {
-  IE_REQUIRE(batch >= 1 && batch <= 16, "attn_decode: batch %d out of range [1,16]", batch);
-  // (a host-side length: one sequence; the paged cache holds up to kMaxLongCtx positions)
-  IE_REQUIRE(p.d_seq_len || (p.seq_len >= 1 && batch == 1 &&
-                             p.seq_len <= (p.block_table ? kMaxLongCtx : kMaxCtx)),
+int launch_attn_decode(const AttnDecodeParams& p, bool merge, hipStream_t st) {
+  // (a host-side length; the paged cache holds up to kMaxLongCtx positions)
+  IE_REQUIRE(p.d_seq_len || (p.seq_len >= 1 && p.seq_len <= (p.block_table ? kMaxLongCtx : kMaxCtx)),
              "attn_decode: seq_len %d out of range [1,%d]", p.seq_len,
              p.block_table ? kMaxLongCtx : kMaxCtx);
-  IE_REQUIRE(p.max_splits >= 1 && p.max_splits <= kAttnSplits, "attn_decode: max_splits %d",
+  IE_REQUIRE(p.max_splits > 1 && p.max_splits <= kAttnSplits, "attn_decode: max_splits %d",
              p.max_splits);
-  IE_REQUIRE(p.max_splits > 1 || (merge && p.out), "attn_decode: one split writes the output");
-  // one workgroup per possible split: idle ones would still cost dispatch (at batch 16 and
-  // 32 splits, 4096 mostly empty workgroups took 52 us)
-  if (p.max_splits == 1)  // one workgroup per (sequence, kv head): 12 waves share its tiles
-    hipLaunchKernelGGL((attn_decode_split_kernel<true, 12, 32>), dim3(1, kKVHeads, batch),
-                       dim3(12 * 64), 0, st, p);
-  else if (batch > 1)
-    hipLaunchKernelGGL((attn_decode_split_kernel<true, kSplitWaves>),
-                       dim3(p.max_splits, kKVHeads, batch), dim3(kSplitWaves * 64), 0, st, p);
-  else
-    hipLaunchKernelGGL((attn_decode_split_kernel<false, 8, 32>), dim3(p.max_splits, kKVHeads, batch),
-                       dim3(8 * 64), 0, st, p);
+  // one workgroup per possible split: idle ones would still cost dispatch
+  hipLaunchKernelGGL((attn_decode_split_kernel<8, 32>), dim3(p.max_splits, kKVHeads),
+                     dim3(8 * 64), 0, st, p);
   IE_CHECK_LAUNCH();
-  if (merge && p.max_splits > 1) {
+  if (merge) {
     IE_REQUIRE(p.out, "attn_decode: merge needs an output buffer");
-    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(kKVHeads, batch), dim3(256), 0, st, p);
+    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(kKVHeads), dim3(256), 0, st, p);
     IE_CHECK_LAUNCH();
   }
+  return IE_OK;
+}
+
+int launch_attn_decode_batched(const AttnDecodeParams& p, int batch, int max_len, bool nt,
+                               hipStream_t st) {
+  IE_REQUIRE(batch >= 1 && batch <= 16, "attn_decode: batch %d out of range [1,16]", batch);
+  IE_REQUIRE(p.d_seq_len && p.out && p.counters && max_len >= 1 && max_len <= kMaxLongCtx,
+             "attn_decode: batched lengths, output and counters");
+  // the most items: a run of one round per kBatchedWaves tiles, at most kAttnSplits of them
+  const int runs = std::min((max_len + kBatchedTile * kBatchedWaves - 1) / (kBatchedTile * kBatchedWaves), kAttnSplits);
+  const dim3 grid(std::min(runs * kKVHeads * batch, 256)), block(kBatchedWaves * 64);
+#define IE_ATTN(SHORT, NT) \
+  hipLaunchKernelGGL((attn_decode_batched_kernel<kBatchedWaves, kBatchedTile, SHORT, NT>), grid, block, 0, st, p, batch)
+  if (max_len <= kAttnShortMaxCtx) {
+    if (nt) IE_ATTN(true, true);
+    else IE_ATTN(true, false);
+  } else {
+    if (nt) IE_ATTN(false, true);
+    else IE_ATTN(false, false);
+  }
+#undef IE_ATTN
+  IE_CHECK_LAUNCH();
   return IE_OK;
 }
 

@@ -503,3 +503,47 @@ def test_generate_stops_at_eos(hip, model):
     first, _ = r.generate(ids, N, eos_token=full[0])
     assert first == full[:1]
     c.close()
+
+
+# lengths at the edges of the batched attention's tiles (32), rounds (384), the one-run contexts
+# (768) and the short batches (2048); a long batch takes its rounds from all its lengths
+@pytest.mark.parametrize("lens", [[1, 31, 32, 33, 383, 385, 767, 768, 769, 1152, 1153, 1537, 2047, 2048],
+                                  [769, 2049], [8192, 1, 384, 4097, 768, 6145], [2049]])
+def test_batched_layer_attention_runs(hip, ctx, model, lens):
+    """One batched layer over these contexts against the single-sequence layer of each (its K/V row
+    bit for bit is not asked: other kernels; 1e-2 of the scale), twice (the arrival counters were
+    reset) with the same bits, and in a short batch each row as in a batch of its own."""
+    from infengine_amd.engine import kv_cache_size, workspace_size
+    B, layer = len(lens), 7
+    say(f"batched layer attention runs {lens}")
+    g = torch.Generator(device="cuda").manual_seed(sum(lens))
+    kv = torch.zeros(B, kv_cache_size() // 2, dtype=torch.bfloat16, device="cuda")
+    planes = kv.view(B, 32, 2, 8, 8192, 128)[:, layer]
+    for b, n in enumerate(lens):
+        planes[b, :, :, :n - 1] = torch.empty(2, 8, n - 1, 128, dtype=torch.bfloat16,
+                                              device="cuda").normal_(0.0, 1.0, generator=g)
+    x0 = torch.empty(B, 4096, dtype=torch.bfloat16, device="cuda").normal_(0.0, 1.0, generator=g)
+    ws = torch.empty(hip.lib.ie_batch_workspace_size(B), dtype=torch.uint8, device="cuda")
+
+    def batched(rows):
+        x, attn = x0[rows].contiguous(), torch.empty(len(rows), 4096, dtype=torch.bfloat16, device="cuda")
+        caches = kv if len(rows) == B else kv[rows[0]:rows[0] + 1]
+        hip.check(hip.lib.ie_decoder_layer_batched(
+            ctx.handle, model.ref(), layer, len(rows), (C.c_int * len(rows))(*[lens[r] for r in rows]),
+            P(x), P(attn), P(ws), P(caches)))
+        torch.cuda.synchronize()
+        return x
+
+    got = batched(list(range(B)))
+    assert torch.equal(batched(list(range(B))), got)
+    if max(lens) <= 2048:
+        for b in range(B):
+            assert torch.equal(batched([b])[0], got[b]), lens[b]
+    dws = torch.empty(workspace_size(1), dtype=torch.uint8, device="cuda")
+    for b, n in enumerate(lens):
+        x, attn = x0[b:b + 1].clone(), torch.empty(1, 4096, dtype=torch.bfloat16, device="cuda")
+        hip.check(hip.lib.ie_decoder_layer_decode(ctx.handle, model.ref(), layer, n, P(x), P(attn),
+                                                  P(dws), P(kv[b])))
+        torch.cuda.synchronize()
+        err = (x[0].float() - got[b].float()).abs().max() / x.float().abs().max()
+        assert float(err) <= 1e-2, (n, float(err))
