@@ -892,8 +892,7 @@ int batched_layer(Context* c, hipStream_t st, const ie_model_weights& W, int l, 
   a.part_o = w.part_o;
   a.part_ml = w.part_ml;
   a.d_seq_len = d_sl;
-  a.counters = c->d_counters + kCntAttn;
-  IE_TRY(launch_attn_decode_batched(a, batch, cls.max_len, cls.nt, st));
+  IE_TRY(launch_attn_decode_batched(a, c->d_counters + kCntAttn, batch, cls.max_len, cls.nt, st));
   GemmParams o{};
   o.x = attn_buffer;
   o.w0 = L.transformer.w_o;

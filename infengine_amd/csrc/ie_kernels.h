@@ -60,7 +60,6 @@ struct AttnDecodeParams {
   const int* d_seq_len;     // [batch] device seq lens, or nullptr
   int seq_len;              // used when d_seq_len == nullptr (batch must be 1)
   int max_splits;           // splits per kv head cap (batch 1): kAttnFusedSplits or kAttnSplits
-  unsigned int* counters;   // batched: zeroed arrival counters [batch x 8], kCntStride apart
 };
 // Splits per (sequence, kv head) for a context of ntiles 64-row tiles: four tiles per split
 // (one per wave of the split workgroup) up to the cap.  Device and host must agree on it.
@@ -101,9 +100,9 @@ inline BatchClass batch_class(const int* lens, int batch, int cap) {
 // Batch 1.  merge = also launch the merge kernel (bf16 output in p.out)
 int launch_attn_decode(const AttnDecodeParams& p, bool merge, hipStream_t st);
 // Up to 16 sequences, none longer than max_len (which sizes the grid): bf16 output in p.out.
-// nt: nontemporal K/V loads.
-int launch_attn_decode_batched(const AttnDecodeParams& p, int batch, int max_len, bool nt,
-                               hipStream_t st);
+// counters: zeroed arrival counters [batch x 8], kCntStride apart.  nt: nontemporal K/V loads.
+int launch_attn_decode_batched(const AttnDecodeParams& p, unsigned int* counters, int batch,
+                               int max_len, bool nt, hipStream_t st);
 size_t attn_decode_partials_bytes(int batch);
 
 // ------------------------------------------------------------ elementwise

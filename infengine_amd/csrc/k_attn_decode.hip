@@ -286,19 +286,19 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_split_kernel(AttnDecodePa
   __shared__ KvSlice<false, KT> kv[NW];
   __shared__ PartO xo[NW];
   __shared__ PartMl xml[NW];
-  const int split = blockIdx.x, g = blockIdx.y;
+  const int split = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int S = p.d_seq_len ? p.d_seq_len[0] : p.seq_len;
+  const int S = p.d_seq_len ? p.d_seq_len[b] : p.seq_len;
   const int ntiles = (S + KT - 1) / KT;
   // (split count in 64-key tiles whatever KT: the merge and the O projection count the same)
   const int ns = attn_decode_splits((S + kAttnTile - 1) / kAttnTile, p.max_splits);
   if (split >= ns) return;  // whole workgroup: nobody reads a partial past ns
   const int tps = (ntiles + ns - 1) / ns;
   const int t0 = split * tps, t1 = min(ntiles, t0 + tps);
-  attend_tiles<false, NW, KT, 0>(p, threadIdx.x, 0, g, S, t0, t1, kv, xo, xml);
+  attend_tiles<false, NW, KT, 0>(p, threadIdx.x, b, g, S, t0, t1, kv, xo, xml);
   if (wave >= kGQA) return;  // (NW > 4) waves past the 4 q heads only contribute partials
   const AttnMerged r = merge_waves<NW>(xo, xml, wave, lane);
-  const size_t slot = ((size_t)g * kAttnSplits + split) * kGQA + wave;
+  const size_t slot = (((size_t)b * kKVHeads + g) * kAttnSplits + split) * kGQA + wave;
   *reinterpret_cast<float2*>(p.part_o + slot * kHeadDim + 2 * lane) = make_float2(r.o0, r.o1);
   if (lane == 0) *reinterpret_cast<float2*>(p.part_ml + slot * 2) = make_float2(r.M, r.L);
 }
@@ -392,7 +392,8 @@ __device__ __forceinline__ int run_rounds(int ntiles) {
 // 2850-7000 86, 69; 6 of 2500-20000 67, 57.
 // NT: nontemporal K/V loads, for K/V that cannot stay in the 256 MB cache until the next step.
 template <int NW, int KT, bool SHORT, bool NT>
-__global__ __launch_bounds__(NW * 64) void attn_decode_batched_kernel(AttnDecodeParams p, int batch) {
+__global__ __launch_bounds__(NW * 64) void attn_decode_batched_kernel(AttnDecodeParams p, unsigned int* counters,
+                                                               int batch) {
   __shared__ KvSlice<true, KT> kv[NW];
   __shared__ PartO xo[NW];
   __shared__ PartMl xml[NW];
@@ -441,7 +442,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_batched_kernel(AttnDecode
     if (ns > 1) {
       __syncthreads();
       if (threadIdx.x == 0) {
-        unsigned int* cnt = p.counters + bg * kCntStride;
+        unsigned int* cnt = counters + bg * kCntStride;
         const unsigned int old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         s_last = old == (unsigned)(ns - 1);
         if (s_last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -528,16 +529,16 @@ int launch_attn_decode(const AttnDecodeParams& p, bool merge, hipStream_t st) {
   return IE_OK;
 }
 
-int launch_attn_decode_batched(const AttnDecodeParams& p, int batch, int max_len, bool nt,
-                               hipStream_t st) {
+int launch_attn_decode_batched(const AttnDecodeParams& p, unsigned int* counters, int batch,
+                               int max_len, bool nt, hipStream_t st) {
   IE_REQUIRE(batch >= 1 && batch <= 16, "attn_decode: batch %d out of range [1,16]", batch);
-  IE_REQUIRE(p.d_seq_len && p.out && p.counters && max_len >= 1 && max_len <= kMaxLongCtx,
+  IE_REQUIRE(p.d_seq_len && p.out && counters && max_len >= 1 && max_len <= kMaxLongCtx,
              "attn_decode: batched lengths, output and counters");
   // the most items: a run of one round per kBatchedWaves tiles, at most kAttnSplits of them
   const int runs = std::min((max_len + kBatchedTile * kBatchedWaves - 1) / (kBatchedTile * kBatchedWaves), kAttnSplits);
   const dim3 grid(std::min(runs * kKVHeads * batch, 256)), block(kBatchedWaves * 64);
 #define IE_ATTN(SHORT, NT) \
-  hipLaunchKernelGGL((attn_decode_batched_kernel<kBatchedWaves, kBatchedTile, SHORT, NT>), grid, block, 0, st, p, batch)
+  hipLaunchKernelGGL((attn_decode_batched_kernel<kBatchedWaves, kBatchedTile, SHORT, NT>), grid, block, 0, st, p, counters, batch)
   if (max_len <= kAttnShortMaxCtx) {
     if (nt) IE_ATTN(true, true);
     else IE_ATTN(true, false);

@@ -250,6 +250,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvParams p) {
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int first = (blockIdx.x * WAVES + wave) * p.ppw;
+  // one input row (grid.y is 1); with the row in the address the compiler issues the input loads
+  // later, beside the weights': QKV 10.04 against 10.24 us, gate/up 36.4 against 36.5
+  const int row = blockIdx.y;
   const int npairs = max(0, min(p.ppw, p.n_pairs - first));
   const int nsteps = npairs * NG;
 
@@ -258,7 +261,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvParams p) {
   // staging below waits for it alone.  These loads and the first two weight steps are
   // unconditional (indices clamped): a load under a branch makes the compiler's wait at the
   // join conservative, which would stall the staging until the weights arrive.
-  const u32x4_t* x4 = reinterpret_cast<const u32x4_t*>(p.x);
+  const u32x4_t* x4 = reinterpret_cast<const u32x4_t*>(p.x + (size_t)row * p.x_stride);
   u32x4_t xin[XC], nwin[XC];
   AttnItem<ATTN ? ATTN : 1> ai[ATTN ? AI : 1];
   int ns = 0;
