@@ -582,27 +582,26 @@ void attn_part_room(AttnPrefillParams& a, char* wsb, int S) {
   a.part_rows = (int)std::min<size_t>(rows, kAttnPrefillPartRows);
 }
 
-// The op-level entries have no workspace: a context-owned scratch, grown on first use.  A call
-// recorded into a graph by the caller cannot allocate: without a large enough scratch it runs
-// unsplit.
+// The op-level entries have no workspace: a context-owned scratch, allocated once at its largest
+// (68 MB) by the first call that splits and kept until the context goes, so that a graph the caller
+// captured keeps valid pointers.  A call recorded into a graph cannot allocate: without the scratch
+// it runs unsplit, as a call does that finds no memory for it.
 int attn_part_scratch(Context* c, AttnPrefillParams& a) {
   if (a.S < 1 || a.start_pos < 0) return IE_OK;  // (the launcher refuses them)
-  const int splits = attn_prefill_splits(a.S, a.start_pos + a.S, kAttnPrefillPartRows);
-  const int rows = splits > 1 ? splits * a.S : 0;
-  if (rows > c->attn_part_rows) {
+  if (!c->attn_part && attn_prefill_splits(a.S, a.start_pos + a.S, kAttnPrefillPartRows) > 1) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     // (the legacy default stream cannot be captured)
     if (c->stream) IE_CHECK_HIP(hipStreamIsCapturing(c->stream, &cap));
     if (cap != hipStreamCaptureStatusNone) return IE_OK;
-    IE_CHECK_HIP(hipStreamSynchronize(c->stream));
-    if (c->attn_part) IE_CHECK_HIP(hipFree(c->attn_part));
-    c->attn_part = nullptr;
-    c->attn_part_rows = 0;
-    IE_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&c->attn_part), rows * kAttnPrefillPartRow * sizeof(float)));
-    c->attn_part_rows = rows;
+    if (hipMalloc(reinterpret_cast<void**>(&c->attn_part),
+                  kAttnPrefillPartRows * kAttnPrefillPartRow * sizeof(float)) != hipSuccess) {
+      (void)hipGetLastError();
+      c->attn_part = nullptr;
+      return IE_OK;
+    }
   }
   a.part = c->attn_part;
-  a.part_rows = c->attn_part_rows;
+  a.part_rows = c->attn_part ? kAttnPrefillPartRows : 0;
   return IE_OK;
 }
 

@@ -264,9 +264,8 @@ struct Context {
   unsigned long long bgraph_tick = 0;
   // the skinny GEMM's K-half partials (kSkPartBytes) for launches outside the batched step
   float* d_sk_part = nullptr;
-  // key-split partials of the op-level prefill attention entries (allocated on first use)
+  // key-split partials of the op-level prefill attention entries (allocated on first use, once)
   float* attn_part = nullptr;
-  int attn_part_rows = 0;
   // split-K partials of the op-level GEMM entry (allocated on first use)
   float* gemm_ws = nullptr;
   size_t gemm_ws_bytes = 0;

@@ -93,3 +93,46 @@ def test_attn_prefill_core_key_splits(hip, ctx, S, start_pos):
                  what=f"attn key splits S={S} start={start_pos}")
     assert torch.equal(out[:S], paged)
     assert bool((out[S] == 7.0).all())
+
+
+def test_attn_prefill_core_key_splits_captured(hip):
+    """Key-split attention recorded into a caller's graph: replays equal the eager call bit for bit,
+    also after an eager call with more partials (the context's scratch stays where it is), and a
+    recording on a context without the scratch yet takes the unsplit kernel."""
+    from infengine_amd.engine import Context
+    say("attn_prefill_core key splits captured")
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q = torch.randn(1300, 32, 128, generator=g, device="cuda").to(torch.bfloat16)
+    k = torch.randn(8, CTX, 128, generator=g, device="cuda").to(torch.bfloat16)
+    v = torch.randn(8, CTX, 128, generator=g, device="cuda").to(torch.bfloat16)
+    small, big, first = (torch.empty(S, 32 * 128, dtype=torch.bfloat16, device="cuda") for S in (64, 1300, 64))
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    c = Context(0, stream, graph=False)
+
+    def attend(S, start, out):
+        hip.check(hip.lib.ie_attn_prefill_core(c.handle, S, start, P(q), P(k), P(v), P(out)))
+
+    graphs = []
+    for out in (first, small):  # before and after the scratch is there
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            attend(64, 4001, out)
+        graphs.append(graph)
+        attend(64, 4001, small)
+        torch.cuda.synchronize()
+    eager = small.clone()
+    attend(1300, 6800, big)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        first.zero_(), small.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            for graph in graphs:
+                graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(small, eager)
+        want = reference(q[:64], k, v, 4001).cpu().numpy()
+        assert_close(first.float().view(64, 32, 128).cpu().numpy(), want, what="captured unsplit")
+    assert not torch.equal(first, eager)  # (another order of the sums: the split was taken)
+    c.close()
