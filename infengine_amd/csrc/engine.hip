@@ -372,6 +372,7 @@ int ie_context_destroy(ie_context* c) {
   if (c->capture) (void)hipStreamDestroy(c->capture);
   if (c->gemm_ws) (void)hipFree(c->gemm_ws);
   if (c->attn_part) (void)hipFree(c->attn_part);
+  for (float* part : c->attn_part_old) (void)hipFree(part);
   delete c;
   return IE_OK;
 }
@@ -582,26 +583,33 @@ void attn_part_room(AttnPrefillParams& a, char* wsb, int S) {
   a.part_rows = (int)std::min<size_t>(rows, kAttnPrefillPartRows);
 }
 
-// The op-level entries have no workspace: a context-owned scratch, allocated once at its largest
-// (68 MB) by the first call that splits and kept until the context goes, so that a graph the caller
-// captured keeps valid pointers.  A call recorded into a graph cannot allocate: without the scratch
-// it runs unsplit, as a call does that finds no memory for it.
+// The op-level entries have no workspace: a context-owned scratch, grown on use to at least twice
+// what it was (at most 68 MB, whose allocation alone takes 100 us) and kept until the context goes,
+// the smaller ones too, so that a graph the caller captured keeps valid pointers.  A call recorded
+// into a graph cannot allocate: without a large enough scratch it runs with fewer splits or none,
+// as a call does that finds no memory.
 int attn_part_scratch(Context* c, AttnPrefillParams& a) {
   if (a.S < 1 || a.start_pos < 0) return IE_OK;  // (the launcher refuses them)
-  if (!c->attn_part && attn_prefill_splits(a.S, a.start_pos + a.S, kAttnPrefillPartRows) > 1) {
+  const int splits = attn_prefill_splits(a.S, a.start_pos + a.S, kAttnPrefillPartRows);
+  const int need = splits > 1 ? splits * a.S : 0;
+  if (need > c->attn_part_rows) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     // (the legacy default stream cannot be captured)
     if (c->stream) IE_CHECK_HIP(hipStreamIsCapturing(c->stream, &cap));
-    if (cap != hipStreamCaptureStatusNone) return IE_OK;
-    if (hipMalloc(reinterpret_cast<void**>(&c->attn_part),
-                  kAttnPrefillPartRows * kAttnPrefillPartRow * sizeof(float)) != hipSuccess) {
-      (void)hipGetLastError();
-      c->attn_part = nullptr;
-      return IE_OK;
+    const int rows = std::min(std::max(need, 2 * c->attn_part_rows), kAttnPrefillPartRows);
+    float* part = nullptr;
+    if (cap == hipStreamCaptureStatusNone) {
+      if (hipMalloc(reinterpret_cast<void**>(&part), rows * kAttnPrefillPartRow * sizeof(float)) == hipSuccess) {
+        if (c->attn_part) c->attn_part_old.push_back(c->attn_part);
+        c->attn_part = part;
+        c->attn_part_rows = rows;
+      } else {
+        (void)hipGetLastError();
+      }
     }
   }
   a.part = c->attn_part;
-  a.part_rows = c->attn_part ? kAttnPrefillPartRows : 0;
+  a.part_rows = c->attn_part_rows;
   return IE_OK;
 }
 

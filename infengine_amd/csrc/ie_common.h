@@ -3,6 +3,7 @@
 // rounding points are the same as the CPU oracle's (round-to-nearest-even).
 #pragma once
 
+#include <vector>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stddef.h>
@@ -264,8 +265,11 @@ struct Context {
   unsigned long long bgraph_tick = 0;
   // the skinny GEMM's K-half partials (kSkPartBytes) for launches outside the batched step
   float* d_sk_part = nullptr;
-  // key-split partials of the op-level prefill attention entries (allocated on first use, once)
+  // key-split partials of the op-level prefill attention entries (grown on use; the smaller ones
+  // before stay for graphs that the caller captured with them)
   float* attn_part = nullptr;
+  int attn_part_rows = 0;
+  std::vector<float*> attn_part_old;
   // split-K partials of the op-level GEMM entry (allocated on first use)
   float* gemm_ws = nullptr;
   size_t gemm_ws_bytes = 0;

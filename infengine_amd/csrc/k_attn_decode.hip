@@ -6,12 +6,12 @@
 // sqrt(128)) . V for all 32 q heads runs as split-context ("flash decoding")
 // attention on MFMA:
 //
-//   grid  = (max_splits, 8 kv heads, batch), block = NW waves
+//   batch 1: grid = (max_splits, 8 kv heads), 8 waves
 //   split s of kv head g owns a contiguous run of the context 0..S-1 (at most 256 positions,
-//   while the split cap allows), cut into tiles of 64 or 32 keys that its waves take in turn
-//   (batch 1: 8 waves on 32-key tiles; batched: 12 waves on 32-key tiles for one split per
-//   sequence, 4 on 64-key tiles for several); a wave stages its tile's K and V rows in LDS (K by
-//   direct-to-LDS loads; V likewise at batch 1, through registers in the batched forms), and
+//   while the split cap allows), cut into tiles of 32 keys that its waves take in turn
+//   batched: 12 waves, workgroups walk an item list (sequence, kv head, run of 384-key rounds)
+//   a wave stages its tile's K and V rows in LDS (K by direct-to-LDS loads; V likewise at
+//   batch 1, through registers in the batched form), and
 //   computes, with
 //   v_mfma_f32_16x16x32_bf16, S^T = K . Q^T for the 4 GQA q heads of the kv head (GQA: q head h
 //   reads kv head h/4, attn.cu:51-53) as 4 of the 16 MFMA columns, an online softmax per head,
@@ -19,12 +19,12 @@
 //   ds_read_b64_tr_b16, as in the prefill kernel.  The waves are merged in LDS and the split
 //   writes one partial (m, l, o) per q head.
 //
-// The partials of the ns splits are merged either by the O projection itself (its
-// input-staging prologue reads them; decode with max_splits = 4, no extra launch)
-// or by a small merge kernel writing bf16 [h][128] (attn.cu:433-438) for the
-// batched GEMM path and long contexts (max_splits = 32).  A device-scope "last
-// workgroup merges" scheme is not used: its fence (L2 write-back / invalidate on
-// this multi-XCD part) per workgroup cost more than a launch.
+// Batch 1: the partials of the ns splits are merged either by the O projection itself (its
+// input-staging prologue reads them; decode with max_splits = 4, no extra launch) or by a small
+// merge kernel writing bf16 [h][128] (attn.cu:433-438) for long contexts (max_splits = 32).
+// Batched: the last run of a (sequence, kv head) to arrive merges them, handed over by
+// device-scope stores without a fence (whose L2 write-back and invalidate on this multi-XCD part
+// cost more than a launch).
 #include <algorithm>
 
 #include "ie_kernels.h"
