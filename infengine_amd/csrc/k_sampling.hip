@@ -305,7 +305,10 @@ __global__ __launch_bounds__(kTopPChunkThreads) void tp_gather_kernel(const floa
   const int cl = tp_chunk_len(vocab), beg = c * cl, end = min(vocab, beg + cl);
   const unsigned long long z = wave_sum_u64(R.zpart[lane]);
   const float mx = tp_row_max(R, temperature);
+  // (held to z: past 2^53 units, a row whose exp(l/T - max) sum to over 8192, (double)z may round
+  // up, and at top_p = 1 no bin would reach a target past the row's mass)
   unsigned long long target = (unsigned long long)((double)z * (double)top_p);
+  if (target > z) target = z;
   if (target < 1) target = 1;
   // the cut bin: thread t owns bins 2t, 2t + 1 (ascending distance), block inclusive scan
   const unsigned long long h0 = R.hist[2 * tid], h1 = R.hist[2 * tid + 1];

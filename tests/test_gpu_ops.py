@@ -866,6 +866,44 @@ def test_top_p_shapes(hip, ctx, vocab, temperature, p, std):
                 assert int(out[r].item()) == want, (r, step, int(out[r].item()), want)
 
 
+# (the largest float below 1 leaves out less than a token's mass)
+@pytest.mark.parametrize("p", [1.0, 0.99999994])
+def test_top_p_whole_mass_of_flat_rows(hip, ctx, p):
+    """Rows whose mass exceeds 2^53 units (their sum of exp(l - max) exceeds 8192), a good part of
+    which round up when the mass is converted to double: the target then lies past the row's mass
+    unless it is held to it.  The oracle's tokens, as in test_top_p_shapes."""
+    say(f"top-p of flat rows with masses past 2^53, p={p}")
+    R = 16
+    lg = np.empty((R, V), np.float32)
+    for r in range(0, R, 4):
+        rng = np.random.default_rng(r)
+        lg[r] = rng.standard_normal(V) * 0.3
+        lg[r, 77] = -13.1
+        lg[r + 1] = rng.standard_normal(V) * 0.2
+        lg[r + 1, 100000:] = rng.standard_normal(V - 100000) - 15.0  # a finite logit bias
+        lg[r + 2] = -rng.exponential(3.0, V)
+        lg[r + 3] = rng.uniform(-14.0, 0.0, V)
+    mass = [sum(int(m) for m in np.exp(row - row.max()) * np.float32(2.0 ** 40)) for row in lg]
+    assert min(mass) > 2 ** 53 and sum(int(float(z)) > z for z in mass) >= 3
+    logits = torch.from_numpy(lg).cuda()
+    out = torch.empty(R, dtype=torch.int32, device="cuda")
+    ws = torch.empty(hip.lib.ie_top_p_workspace_size(R, V), dtype=torch.uint8, device="cuda")
+    for step in range(2):
+        hip.check(hip.lib.ie_sample_top_p(ctx.handle, R, V, P(logits), 1.0, p, 9, step, P(out), P(ws)))
+        noalloc = torch.empty_like(out)
+        hip.check(hip.lib.ie_sample_top_p_noalloc(ctx.handle, R, V, P(logits), 1.0, p, 9, step,
+                                                  P(noalloc)))
+        sync()
+        assert torch.equal(out, noalloc)
+        for r in range(R):
+            tok = int(out[r].item())
+            want, info = orc.top_p(lg[r], 1.0, p, 9, r, step)
+            margin = min(info["t"] - info["lo"], info["hi"] - info["t"]) / info["z_kept"]
+            assert 0 <= tok < V
+            if margin > 1e-6:
+                assert tok == want, (r, step, tok, want)
+
+
 @pytest.mark.parametrize("rows", [2, 4, 5, 8, 9, 16, 17, 64])
 def test_final_norm_lm_head_rows(hip, ctx, rows):
     """The head of 2 .. 64 rows, at the edges of its 4-, 8- and 16-row kernels and of the 16-row
