@@ -1382,7 +1382,8 @@ int ie_gemm_ex(ie_context* c, int epilogue, int m, int k, int n, const ie_bf16* 
   g.K = k;
   g.ldy = n;
   // split K's partials: a context-owned scratch, grown on first use (op-level entry; the
-  // engine passes its own workspace)
+  // engine passes its own workspace).  The product is offered the bytes of its own size however
+  // large the scratch is, so that its K split (and its bits) do not depend on earlier calls.
   const size_t need = epilogue == IE_GEMM_F32 ? 0 : gemm_split_bytes(m, epilogue == IE_GEMM_SWIGLU ? 2 * n : n);
   if (need > c->gemm_ws_bytes) {
     IE_CHECK_HIP(hipStreamSynchronize(c->stream));
@@ -1392,8 +1393,8 @@ int ie_gemm_ex(ie_context* c, int epilogue, int m, int k, int n, const ie_bf16* 
     IE_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&c->gemm_ws), need));
     c->gemm_ws_bytes = need;
   }
-  g.split_ws = c->gemm_ws;
-  g.split_ws_bytes = (long long)c->gemm_ws_bytes;
+  g.split_ws = need ? c->gemm_ws : nullptr;
+  g.split_ws_bytes = (long long)need;
   skinny_split(c, epilogue, g, c->d_sk_part);
   return launch_gemm(epilogue, g, c->stream);
 }

@@ -389,8 +389,9 @@ def test_gemm_schedules_bit_identical(hip, ctx, epi, m, k, n):
 
 
 # Every tile shape of the prefill GEMM past 128 rows at the first, last or a middle row count that
-# picks it, K split (planes of 2-8) and not, ragged columns (n = 1000, 4104; n = 4100 never
-# splits), one and three k-steps, and bases off 16 bytes (the register-staged kernel).
+# picks it, ragged columns (n = 1000, 4104), one and three k-steps.  K split: resid of 130-512 rows
+# at k = 4096 (8, 4, 4, 2 and 2 planes) and of 300-901 at 14336 (4), bf16 of 161 rows (8); the rest
+# unsplit, as SwiGLU, fp32 and this entry point past 1024 rows always are.
 @pytest.mark.parametrize("epi,m,k,n", [
     ("resid", 130, 4096, 4096), ("resid", 192, 4096, 4096), ("resid", 257, 4096, 4096),
     ("resid", 385, 4096, 4104), ("resid", 512, 4096, 4096), ("resid", 929, 4096, 4096),
@@ -439,6 +440,32 @@ def test_gemm_tile_shapes(hip, ctx, epi, m, k, n):
     assert_close(got, orc.bf16_to_f32(host(want)), what=f"tile shapes {epi}")
     assert_bf16_close(host(outs[0][:m].view(torch.int16)), host(want), ulps=4 if epi == "swiglu" else 2,
                       what=f"tile shapes {epi}", outlier_frac=1e-3 if epi == "resid" else 0.0)
+
+
+@pytest.mark.parametrize("epi,m,k,n", [("resid", 300, 14336, 4096), ("bf16", 700, 4096, 6144),
+                                       ("resid", 1100, 14336, 4096), ("bf16", 1600, 4096, 4096)])
+def test_gemm_ex_same_on_any_context(hip, ctx, epi, m, k, n):
+    """A product's bits do not depend on the split-K scratch that earlier calls left in its
+    context: a fresh context's result equals that of one which ran larger products."""
+    from infengine_amd.engine import Context
+    say(f"gemm_ex on a fresh and a used context {epi} m={m} k={k} n={n}")
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.empty(m, k, dtype=torch.bfloat16, device="cuda").normal_(0.0, 1.0, generator=g)
+    w = torch.empty(n, k, dtype=torch.bfloat16, device="cuda").normal_(0.0, 0.02, generator=g)
+    big_w = torch.zeros(16384, 64, dtype=torch.bfloat16, device="cuda")
+    big_y = torch.empty(1024, 16384, dtype=torch.bfloat16, device="cuda")
+    outs = []
+    for used in (False, True):
+        c = Context(0, torch.cuda.current_stream(), graph=False)
+        if used:  # (256 MiB of scratch)
+            hip.check(hip.lib.ie_gemm_ex(c.handle, GEMM_EPI["bf16"], 1024, 64, 16384, P(x), P(big_w), None,
+                                         P(big_y)))
+        y = torch.ones(m, n, dtype=torch.bfloat16, device="cuda")
+        hip.check(hip.lib.ie_gemm_ex(c.handle, GEMM_EPI[epi], m, k, n, P(x), P(w), None, P(y)))
+        sync()
+        outs.append(y)
+        c.close()
+    assert torch.equal(outs[0], outs[1])
 
 
 def test_gemm_unaligned_operands(hip, ctx):
