@@ -372,7 +372,7 @@ int ie_context_destroy(ie_context* c) {
   if (c->capture) (void)hipStreamDestroy(c->capture);
   if (c->gemm_ws) (void)hipFree(c->gemm_ws);
   if (c->attn_part) (void)hipFree(c->attn_part);
-  for (float* part : c->attn_part_old) (void)hipFree(part);
+  for (float* s : c->outgrown) (void)hipFree(s);
   delete c;
   return IE_OK;
 }
@@ -583,33 +583,46 @@ void attn_part_room(AttnPrefillParams& a, char* wsb, int S) {
   a.part_rows = (int)std::min<size_t>(rows, kAttnPrefillPartRows);
 }
 
-// The op-level entries have no workspace: a context-owned scratch, grown on use to at least twice
-// what it was (at most 68 MB, whose allocation alone takes 100 us) and kept until the context goes,
-// the smaller ones too, so that a graph the caller captured keeps valid pointers.  A call recorded
+// Replaces a scratch of the context by one of at least `need` bytes, of twice the earlier one's where
+// memory and `most` allow.  The earlier one stays until the context goes: kernels in flight and graphs
+// that the caller recorded with it still use it.  False: no memory, or the context's own stream is
+// capturing.  (A capture on another stream is left alone: in its default mode it would fail the
+// allocation and be broken by it.)
+bool grow_scratch(Context* c, float*& buf, size_t& bytes, size_t need, size_t most = SIZE_MAX) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  // (the legacy default stream cannot be captured)
+  if (c->stream && hipStreamIsCapturing(c->stream, &cap) != hipSuccess) return false;
+  if (cap != hipStreamCaptureStatusNone) return false;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  float* p = nullptr;
+  for (const size_t want : {std::min(std::max(need, 2 * bytes), most), need}) {
+    if (hipMalloc(reinterpret_cast<void**>(&p), want) == hipSuccess) {
+      if (buf) c->outgrown.push_back(buf);
+      buf = p;
+      bytes = want;
+      break;
+    }
+    p = nullptr;
+    (void)hipGetLastError();
+  }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return p != nullptr;
+}
+
+// The op-level entries have no workspace: a context-owned scratch, grown on use (at most 68 MB,
+// whose allocation alone takes 100 us).  A call recorded
 // into a graph cannot allocate: without a large enough scratch it runs with fewer splits or none,
 // as a call does that finds no memory.
 int attn_part_scratch(Context* c, AttnPrefillParams& a) {
   if (a.S < 1 || a.start_pos < 0) return IE_OK;  // (the launcher refuses them)
+  constexpr size_t row = kAttnPrefillPartRow * sizeof(float);
   const int splits = attn_prefill_splits(a.S, a.start_pos + a.S, kAttnPrefillPartRows);
-  const int need = splits > 1 ? splits * a.S : 0;
-  if (need > c->attn_part_rows) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    // (the legacy default stream cannot be captured)
-    if (c->stream) IE_CHECK_HIP(hipStreamIsCapturing(c->stream, &cap));
-    const int rows = std::min(std::max(need, 2 * c->attn_part_rows), kAttnPrefillPartRows);
-    float* part = nullptr;
-    if (cap == hipStreamCaptureStatusNone) {
-      if (hipMalloc(reinterpret_cast<void**>(&part), rows * kAttnPrefillPartRow * sizeof(float)) == hipSuccess) {
-        if (c->attn_part) c->attn_part_old.push_back(c->attn_part);
-        c->attn_part = part;
-        c->attn_part_rows = rows;
-      } else {
-        (void)hipGetLastError();
-      }
-    }
-  }
+  const size_t need = splits > 1 ? splits * a.S * row : 0;
+  if (need > c->attn_part_bytes)
+    grow_scratch(c, c->attn_part, c->attn_part_bytes, need, kAttnPrefillPartRows * row);
   a.part = c->attn_part;
-  a.part_rows = c->attn_part_rows;
+  a.part_rows = (int)(c->attn_part_bytes / row);
   return IE_OK;
 }
 
@@ -1385,13 +1398,9 @@ int ie_gemm_ex(ie_context* c, int epilogue, int m, int k, int n, const ie_bf16* 
   // engine passes its own workspace).  The product is offered the bytes of its own size however
   // large the scratch is, so that its K split (and its bits) do not depend on earlier calls.
   const size_t need = epilogue == IE_GEMM_F32 ? 0 : gemm_split_bytes(m, epilogue == IE_GEMM_SWIGLU ? 2 * n : n);
-  if (need > c->gemm_ws_bytes) {
-    IE_CHECK_HIP(hipStreamSynchronize(c->stream));
-    if (c->gemm_ws) IE_CHECK_HIP(hipFree(c->gemm_ws));
-    c->gemm_ws = nullptr;
-    c->gemm_ws_bytes = 0;
-    IE_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&c->gemm_ws), need));
-    c->gemm_ws_bytes = need;
+  if (need > c->gemm_ws_bytes && !grow_scratch(c, c->gemm_ws, c->gemm_ws_bytes, need)) {
+    set_error("gemm_ex: no %zu bytes of scratch (or the stream is capturing)", need);
+    return IE_ERR_HIP;
   }
   g.split_ws = need ? c->gemm_ws : nullptr;
   g.split_ws_bytes = (long long)need;

@@ -265,14 +265,13 @@ struct Context {
   unsigned long long bgraph_tick = 0;
   // the skinny GEMM's K-half partials (kSkPartBytes) for launches outside the batched step
   float* d_sk_part = nullptr;
-  // key-split partials of the op-level prefill attention entries (grown on use; the smaller ones
-  // before stay for graphs that the caller captured with them)
+  // key-split partials of the op-level prefill attention entries, split-K partials of the op-level
+  // GEMM entry (grown on use), and the smaller ones before them
   float* attn_part = nullptr;
-  int attn_part_rows = 0;
-  std::vector<float*> attn_part_old;
-  // split-K partials of the op-level GEMM entry (allocated on first use)
+  size_t attn_part_bytes = 0;
   float* gemm_ws = nullptr;
   size_t gemm_ws_bytes = 0;
+  std::vector<float*> outgrown;
 };
 
 // Per-row reduction state sits one 128-byte line apart: device-scope atomics on one line

@@ -468,6 +468,49 @@ def test_gemm_ex_same_on_any_context(hip, ctx, epi, m, k, n):
     assert torch.equal(outs[0], outs[1])
 
 
+def test_gemm_ex_captured_then_larger(hip, ctx):
+    """A split product recorded into a caller's graph replays as the eager call after a larger
+    product has grown the context's scratch (the earlier scratch stays where it is), and a
+    recording whose scratch is not there yet is refused."""
+    from infengine_amd.engine import Context
+    say("gemm_ex captured, then a larger product")
+    g = torch.Generator(device="cuda").manual_seed(11)
+    m, k, n = 300, 14336, 4096
+    x = torch.empty(m, k, dtype=torch.bfloat16, device="cuda").normal_(0.0, 1.0, generator=g)
+    w = torch.empty(n, k, dtype=torch.bfloat16, device="cuda").normal_(0.0, 0.02, generator=g)
+    big_w = torch.zeros(16384, 64, dtype=torch.bfloat16, device="cuda")
+    y, big_y = (torch.empty(r, q, dtype=torch.bfloat16, device="cuda") for r, q in ((m, n), (1024, 16384)))
+    sync()
+    stream = torch.cuda.Stream()
+    c = Context(0, stream, graph=False)
+
+    def small():
+        return hip.lib.ie_gemm_ex(c.handle, GEMM_EPI["bf16"], m, k, n, P(x), P(w), None, P(y))
+
+    refused = []
+    with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=stream):
+        refused.append(small())
+        y.zero_()
+    assert refused[0] < 0 and "capturing" in hip.last_error()
+    hip.check(small())
+    sync()
+    eager = y.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        hip.check(small())
+    hip.check(hip.lib.ie_gemm_ex(c.handle, GEMM_EPI["bf16"], 1024, 64, 16384, P(x), P(big_w), None,
+                                 P(big_y)))
+    sync()
+    fill = torch.full((1 << 26,), 3.0, device="cuda")  # (256 MiB that a freed scratch could have become)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        sync()
+        assert torch.equal(y, eager)
+        assert bool((fill == 3.0).all())
+    c.close()
+
+
 def test_gemm_unaligned_operands(hip, ctx):
     """X and W bases off 16 bytes (8): the register-staged kernel, the aligned call's values."""
     m, k, n = 300, 256, 512
