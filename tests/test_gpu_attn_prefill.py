@@ -136,3 +136,30 @@ def test_attn_prefill_core_key_splits_captured(hip):
         assert_close(first.float().view(64, 32, 128).cpu().numpy(), want, what="captured unsplit")
     assert not torch.equal(first, eager)  # (another order of the sums: the split was taken)
     c.close()
+
+
+def test_attn_prefill_core_key_splits_beside_a_capture(hip):
+    """The first split call of a context, which allocates its scratch, while another stream is being
+    captured: the call runs split, and the capture ends and replays."""
+    from infengine_amd.engine import Context
+    say("attn_prefill_core key splits beside a capture")
+    g = torch.Generator(device="cuda").manual_seed(4)
+    q = torch.randn(64, 32, 128, generator=g, device="cuda").to(torch.bfloat16)
+    k = torch.randn(8, CTX, 128, generator=g, device="cuda").to(torch.bfloat16)
+    v = torch.randn(8, CTX, 128, generator=g, device="cuda").to(torch.bfloat16)
+    outs = [torch.empty(64, 32 * 128, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    mark = torch.zeros(8, device="cuda")
+    torch.cuda.synchronize()
+    work, captured = torch.cuda.Stream(), torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    contexts = [Context(0, work, graph=False) for _ in outs]
+    with torch.cuda.graph(graph, stream=captured):
+        mark += 1
+        hip.check(hip.lib.ie_attn_prefill_core(contexts[0].handle, 64, 4001, P(q), P(k), P(v), P(outs[0])))
+    hip.check(hip.lib.ie_attn_prefill_core(contexts[1].handle, 64, 4001, P(q), P(k), P(v), P(outs[1])))
+    for _ in range(3):
+        graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and mark.tolist() == [3.0] * 8
+    for c in contexts:
+        c.close()
