@@ -363,7 +363,11 @@ IE_API int ie_gemm_bf16(ie_context* ctx, int m, int k, int n, const ie_bf16* d_x
  *   IE_GEMM_RESID   y[m,n] = bf16(y + bf16(X . W0^T))               (d_y bf16, read+written)
  *   IE_GEMM_F32     y[m,n] = X . W0^T                               (d_y fp32)
  *   IE_GEMM_SWIGLU  y[m,n] = swiglu(bf16(X . W0^T), bf16(X . W1^T)) (d_y bf16; W0 gate, W1 up)
- * W0/W1 are [n][k]; n % 4 == 0, k % 64 == 0. */
+ * W0/W1 are [n][k]; n % 4 == 0, k % 64 == 0.
+ * Up to 1024 rows the product may split K over a scratch of the context, allocated by the first
+ * call that needs more of it (refused while the context's stream is captured: run such a call
+ * once before) and kept until the context is destroyed.  Graphs recorded from one context with
+ * such calls share it: they must not replay at once, nor after the context. */
 #define IE_GEMM_BF16 0
 #define IE_GEMM_RESID 1
 #define IE_GEMM_F32 2
@@ -374,7 +378,13 @@ IE_API int ie_gemm_ex(ie_context* ctx, int epilogue, int m, int k, int n, const 
  * kernels/attn.cu:309-371, without the projections): d_q [seq_len][32][128] (RoPE applied),
  * d_k / d_v one layer's K and V planes [8][8192][128] holding key rows 0..start_pos+seq_len-1,
  * d_out [seq_len][4096] bf16 in the [s][h][d] layout of attn_permute.cu:15-31.  Query row i sits
- * at position start_pos + i and sees keys 0..start_pos+i. */
+ * at position start_pos + i and sees keys 0..start_pos+i.
+ * Few rows over many keys are split over the keys, with partials in a scratch of the context that
+ * the first such call allocates (at most 68 MB, kept until the context is destroyed).  A call
+ * recorded into a graph of the caller's, or without memory for the scratch, runs unsplit: it
+ * uses no memory of the context (its graphs may replay at once and outlive the context), takes up
+ * to 3 times as long (200 rows at position 30000: 443 against 135 us) and sums in another order,
+ * so that its bits differ from the split call's. */
 IE_API int ie_attn_prefill_core(ie_context* ctx, int seq_len, int start_pos, const ie_bf16* d_q,
                                 const ie_bf16* d_k, const ie_bf16* d_v, ie_bf16* d_out);
 /* The same attention core over a page pool (ie_kv_page_size() pages; block_table (device) maps

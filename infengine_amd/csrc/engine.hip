@@ -583,16 +583,20 @@ void attn_part_room(AttnPrefillParams& a, char* wsb, int S) {
   a.part_rows = (int)std::min<size_t>(rows, kAttnPrefillPartRows);
 }
 
+// Whether the caller records the context's stream into a graph (the legacy default stream cannot
+// be captured; a stream whose state is unknown counts as recording).
+bool recording(const Context* c) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  return c->stream && (hipStreamIsCapturing(c->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone);
+}
+
 // Replaces a scratch of the context by one of at least `need` bytes, of twice the earlier one's where
 // memory and `most` allow.  The earlier one stays until the context goes: kernels in flight and graphs
 // that the caller recorded with it still use it.  False: no memory, or the context's own stream is
 // capturing.  (A capture on another stream is left alone: in its default mode it would fail the
 // allocation and be broken by it.)
 bool grow_scratch(Context* c, float*& buf, size_t& bytes, size_t need, size_t most = SIZE_MAX) {
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  // (the legacy default stream cannot be captured)
-  if (c->stream && hipStreamIsCapturing(c->stream, &cap) != hipSuccess) return false;
-  if (cap != hipStreamCaptureStatusNone) return false;
+  if (recording(c)) return false;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   (void)hipThreadExchangeStreamCaptureMode(&mode);
   float* p = nullptr;
@@ -610,20 +614,20 @@ bool grow_scratch(Context* c, float*& buf, size_t& bytes, size_t need, size_t mo
   return p != nullptr;
 }
 
-// The op-level entries have no workspace: a context-owned scratch, grown on use (at most 68 MB,
-// whose allocation alone takes 100 us).  A call recorded
-// into a graph cannot allocate: without a large enough scratch it runs with fewer splits or none,
-// as a call does that finds no memory.
-int attn_part_scratch(Context* c, AttnPrefillParams& a) {
-  if (a.S < 1 || a.start_pos < 0) return IE_OK;  // (the launcher refuses them)
+// The op-level entries have no workspace: their key splits take a context-owned scratch, grown on use
+// (at most 68 MB, whose allocation alone takes 100 us).  Calls on one context follow each other on
+// its stream, but graphs recorded from it may be replayed at once and after it is gone: a recorded
+// call holds no state of the context and runs unsplit, as does one that finds no memory.
+void attn_part_scratch(Context* c, AttnPrefillParams& a) {
+  if (a.S < 1 || a.start_pos < 0 || recording(c)) return;  // (the launcher refuses the former)
   constexpr size_t row = kAttnPrefillPartRow * sizeof(float);
   const int splits = attn_prefill_splits(a.S, a.start_pos + a.S, kAttnPrefillPartRows);
   const size_t need = splits > 1 ? splits * a.S * row : 0;
-  if (need > c->attn_part_bytes)
-    grow_scratch(c, c->attn_part, c->attn_part_bytes, need, kAttnPrefillPartRows * row);
+  if (need > c->attn_part_bytes &&
+      !grow_scratch(c, c->attn_part, c->attn_part_bytes, need, kAttnPrefillPartRows * row))
+    return;
   a.part = c->attn_part;
-  a.part_rows = (int)(c->attn_part_bytes / row);
-  return IE_OK;
+  a.part_rows = (int)(need / row);
 }
 
 // aux_ready: aux_buffer already holds this layer's input RMSNorm of data_buffer (written by
@@ -1355,7 +1359,7 @@ int ie_attn_prefill_core(ie_context* c, int seq_len, int start_pos, const ie_bf1
   CTX_OK(c);
   IE_REQUIRE(d_q && d_k && d_v && d_out, "attn_prefill_core: null pointer");
   AttnPrefillParams a{d_q, d_k, d_v, d_out, seq_len, start_pos};
-  IE_TRY(attn_part_scratch(c, a));
+  attn_part_scratch(c, a);
   return launch_attn_prefill(a, c->stream);
 }
 
@@ -1369,7 +1373,7 @@ int ie_attn_prefill_core_paged(ie_context* c, int seq_len, int start_pos, const 
   const uint16_t* kl = static_cast<const uint16_t*>(kv_pages) + (size_t)layer * kPageLayer;
   AttnPrefillParams a{d_q, kl, kl + (size_t)kKVHeads * kPageHead, d_out, seq_len, start_pos,
                       block_table, n_pages};
-  IE_TRY(attn_part_scratch(c, a));
+  attn_part_scratch(c, a);
   return launch_attn_prefill(a, c->stream);
 }
 

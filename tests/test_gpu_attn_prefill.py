@@ -96,46 +96,55 @@ def test_attn_prefill_core_key_splits(hip, ctx, S, start_pos):
 
 
 def test_attn_prefill_core_key_splits_captured(hip):
-    """Key-split attention recorded into a caller's graph: replays equal the eager call bit for bit,
-    also after an eager call with more partials (the context's scratch stays where it is), and a
-    recording on a context without the scratch yet takes the unsplit kernel."""
+    """Key-split sizes recorded into a caller's graphs: a recorded call takes no scratch of the
+    context and runs unsplit, before and after an eager call with splits alike.  The graphs replay
+    one after the other, at once on two streams beside eager split calls, and after the context
+    is gone."""
     from infengine_amd.engine import Context
     say("attn_prefill_core key splits captured")
     g = torch.Generator(device="cuda").manual_seed(3)
     q = torch.randn(1300, 32, 128, generator=g, device="cuda").to(torch.bfloat16)
     k = torch.randn(8, CTX, 128, generator=g, device="cuda").to(torch.bfloat16)
     v = torch.randn(8, CTX, 128, generator=g, device="cuda").to(torch.bfloat16)
-    small, big, first = (torch.empty(S, 32 * 128, dtype=torch.bfloat16, device="cuda") for S in (64, 1300, 64))
+    first, second, eager, big = (torch.empty(S, 32 * 128, dtype=torch.bfloat16, device="cuda")
+                                 for S in (64, 64, 64, 1300))
     torch.cuda.synchronize()
-    stream = torch.cuda.Stream()
+    stream, other = torch.cuda.Stream(), torch.cuda.Stream()
     c = Context(0, stream, graph=False)
 
     def attend(S, start, out):
         hip.check(hip.lib.ie_attn_prefill_core(c.handle, S, start, P(q), P(k), P(v), P(out)))
 
     graphs = []
-    for out in (first, small):  # before and after the scratch is there
+    for out in (first, second):  # before and after the scratch is there
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=stream):
             attend(64, 4001, out)
         graphs.append(graph)
-        attend(64, 4001, small)
+        attend(64, 4001, eager)
         torch.cuda.synchronize()
-    eager = small.clone()
-    attend(1300, 6800, big)
+    want = reference(q[:64], k, v, 4001).cpu().numpy()
+    assert_close(eager.float().view(64, 32, 128).cpu().numpy(), want, what="eager, split")
+    graphs[0].replay()
     torch.cuda.synchronize()
-    for _ in range(3):
-        first.zero_(), small.zero_()
+    unsplit = first.clone()
+    assert_close(unsplit.float().view(64, 32, 128).cpu().numpy(), want, what="captured, unsplit")
+    assert not torch.equal(unsplit, eager)  # (another order of the sums: the eager call was split)
+    split = eager.clone()
+    for turn in range(4):
+        first.zero_(), second.zero_(), eager.zero_()
         torch.cuda.synchronize()
-        with torch.cuda.stream(stream):
-            for graph in graphs:
+        if turn < 3:
+            attend(64, 4001, eager)
+            attend(1300, 6800, big)
+        else:
+            c.close()
+        for s, graph in zip((stream, other), graphs):
+            with torch.cuda.stream(s):
                 graph.replay()
         torch.cuda.synchronize()
-        assert torch.equal(small, eager)
-        want = reference(q[:64], k, v, 4001).cpu().numpy()
-        assert_close(first.float().view(64, 32, 128).cpu().numpy(), want, what="captured unsplit")
-    assert not torch.equal(first, eager)  # (another order of the sums: the split was taken)
-    c.close()
+        assert torch.equal(first, unsplit) and torch.equal(second, unsplit)
+        assert turn == 3 or torch.equal(eager, split)
 
 
 def test_attn_prefill_core_key_splits_beside_a_capture(hip):
