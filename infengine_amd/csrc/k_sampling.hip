@@ -21,7 +21,6 @@
 //      uniform of (seed, row, step)
 //   4. the sampled token is the smallest id whose kept prefix mass exceeds t
 //      (inverse CDF in token-id order), found with a block-wide exclusive scan.
-#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -160,11 +159,15 @@ __device__ __forceinline__ T wave_scan(T v) {
 //              masses, t, the chunk holding t, then its token by a scan in token-id order
 // 16 rows of the 128256-entry vocabulary: 30 us, 1 row 23; the six launches that cached
 // the exponentials, used 2048 bins and summed the kept masses over all tokens took 53-57 and 37.
-// 512 bins of 0.055 nats in place of 2048: the device-scope additions of the histograms (the
-// largest part, 700 thousand a call at 16 rows) fall to a quarter, and a cut bin of a row whose
-// scaled logits spread over more than ~0.3 nats still fits the candidate list.
+// 512 bins in place of 2048: the device-scope additions of the histograms (the largest part, 700
+// thousand a call at 16 rows) fall to a quarter.
+// The bins are octaves of 1.08 d + 2 in 128 steps each, 0.0145 nats wide at the top, 0.029 past 1.9 and
+// 0.058 past 5.6: a row's cut lies at a few times the spread of its scaled logits, so that a flatter
+// row has its cut where the bins are finer.  The cut bin of N(0, s) logits holds up to about 128256 x
+// width / (2.5 s) tokens: the candidate list takes them from s = 0.08 on.  512 even bins took them from
+// 0.27 on; 16 rows at p = 0.5, us, even bins / these: s = 0.1 275 / 46, 0.3 46 / 34, 0.8 34.5 / 32, 2.0
+// 29.0 / 29.2 (p = 0.9: 31.3 / 31.9).  (576 bins, even past 1.2 nats: 30.3 and 32.9 at s = 2.0.)
 constexpr int kTopPBins = 512;
-constexpr float kTopPBinScale = kTopPBins / 28.0f;
 constexpr int kTopPChunks = 64;
 constexpr int kTopPChunkThreads = 256;
 constexpr int kTopPCandMax = 10240;
@@ -182,9 +185,11 @@ struct TopPRow {
   unsigned long long cand_q[kTopPCandMax];  // mass (41 bits) | chunk << 48
 };
 
-__device__ __forceinline__ int top_p_bin(float d) {
-  return min(kTopPBins - 1, (int)(d * kTopPBinScale));
+// The octaves 2-4, 4-8, 8-16 and 16-32 of 1.08 d + 2 (from 32 on, and NaN: any bin, without mass).
+__host__ __device__ __forceinline__ int top_p_bin(float d) {
+  return (int)(__builtin_bit_cast(uint32_t, fmaf(d, 1.08f, 2.0f)) >> 16 & (uint32_t)(kTopPBins - 1));
 }
+static_assert(kTopPBins == 512 && 1.08 * 27.73 + 2 < 32, "128 bins an octave; exp(-27.73) * 2^40 < 1");
 
 __device__ __forceinline__ int tp_chunk_len(int vocab) {
   return (vocab + kTopPChunks - 1) / kTopPChunks;
@@ -398,7 +403,7 @@ __global__ __launch_bounds__(kTopPThreads) void tp_finish_kernel(const float* lo
   if (tid == 0) s_tok = -1;
   if (in_lds)
     for (int j = tid; j < ncand; j += kTopPThreads) ck[j] = R.cand_key[j], cq[j] = R.cand_q[j];
-  // f(key, mass, chunk) over the tokens of the cut bin
+  // f(key, mass, chunk) over the tokens of the cut bin (chunk 0 for those of a row that is not listed)
   const auto each = [&](auto f) {
     if (listed) {
       for (int j = tid; j < ncand; j += kTopPThreads) {
@@ -411,7 +416,7 @@ __global__ __launch_bounds__(kTopPThreads) void tp_finish_kernel(const float* lo
         const float sv = L[i] / temperature;
         if (top_p_bin(mx - sv) != bcut) continue;
         const unsigned long long q = fix_mass(expf(sv - mx));
-        if (q) f(order_key(sv), q, i / cl);
+        if (q) f(order_key(sv), q, 0);
       }
     }
   };
@@ -432,9 +437,25 @@ __global__ __launch_bounds__(kTopPThreads) void tp_finish_kernel(const float* lo
   }
   const uint32_t kappa = prefix;
   // the chunks' kept masses: lower bins whole, the cut bin's keys from kappa up
-  each([&](uint32_t k, unsigned long long q, int c) {
-    if (k >= kappa) atomicAdd(&kpart[c], q);
-  });
+  if (listed) {
+    each([&](uint32_t k, unsigned long long q, int c) {
+      if (k >= kappa) atomicAdd(&kpart[c], q);
+    });
+  } else {
+    // a wave per chunk (adding token by token to 64 sums took 50 us of a row of equal logits; rolled
+    // up: more code for these rows cost the listed ones 0.3 us)
+    for (int c = wave; c < kTopPChunks; c += kTopPThreads / 64) {
+      const int end = min(vocab, c * cl + cl);
+      unsigned long long kept = 0;
+#pragma unroll 1
+      for (int i = c * cl + lane; i < end; i += 64) {
+        const float sv = L[i] / temperature;
+        if (top_p_bin(mx - sv) == bcut && order_key(sv) >= kappa) kept += fix_mass(expf(sv - mx));
+      }
+      kept = wave_sum_u64(kept);
+      if (lane == 0) kpart[c] += kept;
+    }
+  }
   __syncthreads();
   // t, and the chunk holding it (kept masses in chunk order = token-id order)
   if (wave == 0) {
@@ -546,7 +567,7 @@ int launch_top_p(int rows, int vocab, const float* logits, float temperature, fl
   // below the (1 - p) Z left out (half of it, for the roundings).
   const double left = 1.0 - (double)top_p;
   const double d0 = left > 1e-9 ? std::log(2.0 * vocab / left) : 28.0;
-  const int last_bin = (int)std::min<double>(kTopPBins - 1, d0 * kTopPBinScale + 1);
+  const int last_bin = d0 < 27.0 ? top_p_bin((float)d0) + 1 : kTopPBins - 1;
   const dim3 chunks(kTopPChunks, rows);
   hipLaunchKernelGGL(tp_max_kernel, chunks, dim3(kTopPChunkThreads), 0, st, logits, vocab, R);
   hipLaunchKernelGGL(tp_hist_kernel, chunks, dim3(kTopPChunkThreads), 0, st, logits, vocab,

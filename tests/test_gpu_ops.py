@@ -907,12 +907,14 @@ def test_top_p_ties_and_flat_rows(hip, ctx):
 
 
 # chunks of one token, empty chunks (vocab 7, 65), two rounds a chunk (131072), ragged ones; nearly
-# nothing left out (p = 1: every bin can hold the cut) and nearly everything; spreads that put more
-# candidates in the cut bin than tp_finish keeps in LDS (0.25) and than the list holds (0.1)
+# nothing left out (p = 1: every bin can hold the cut) and nearly everything; spreads with the cut in
+# the finest bins (0.25), with more candidates in the cut bin than tp_finish keeps in LDS (0.1) and
+# than the list holds (0.03)
 @pytest.mark.parametrize("vocab,temperature,p,std", [(7, 1.0, 0.5, 1.0), (65, 0.7, 0.9, 2.0),
                                                      (1000, 1.0, 1.0, 3.0), (50001, 0.4, 0.02, 2.0),
                                                      (131072, 1.2, 0.98, 2.0), (V, 1.0, 0.7, 0.25),
-                                                     (V, 1.0, 0.5, 0.1), (V, 2.0, 1.0, 4.0)])
+                                                     (V, 1.0, 0.5, 0.1), (V, 1.0, 0.5, 0.03),
+                                                     (V, 2.0, 1.0, 4.0)])
 def test_top_p_shapes(hip, ctx, vocab, temperature, p, std):
     """Top-p sampling at the edges of its chunks, bins and candidate list: the oracle's tokens (the
     masses are exact; a t within 1e-6 of a token's edge may fall on either side, as expf's last
@@ -934,6 +936,30 @@ def test_top_p_shapes(hip, ctx, vocab, temperature, p, std):
             margin = min(info["t"] - info["lo"], info["hi"] - info["t"]) / info["z_kept"]
             if margin > 1e-6:
                 assert int(out[r].item()) == want, (r, step, int(out[r].item()), want)
+
+
+def test_top_p_near_flat_rows_time(hip, ctx):
+    """A near-flat row (logits spread over 0.1) stays on the candidate list: 1.6 times an ordinary
+    row's time at 16 rows, and 9.5 where its cut bin overflows the list and the row itself is
+    selected over.  The bound is 4; the least of five rounds of 20 calls each."""
+    say("top-p time of near-flat rows")
+    g = torch.Generator(device="cuda").manual_seed(6)
+    out = torch.empty(16, dtype=torch.int32, device="cuda")
+    ws = torch.empty(hip.lib.ie_top_p_workspace_size(16, V), dtype=torch.uint8, device="cuda")
+    ms = []
+    for std in (2.0, 0.1):
+        logits = torch.empty(16, V, device="cuda").normal_(0.0, std, generator=g)
+        rounds = []
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(20):
+                hip.check(hip.lib.ie_sample_top_p(ctx.handle, 16, V, P(logits), 1.0, 0.5, 1, 0, P(out), P(ws)))
+            b.record()
+            sync()
+            rounds.append(a.elapsed_time(b))
+        ms.append(min(rounds[1:]))
+    assert ms[1] <= 4 * ms[0], ms
 
 
 # (the largest float below 1 leaves out less than a token's mass)
