@@ -241,7 +241,10 @@ __global__ __launch_bounds__(256 * SUB, (QI == 2 && SUB == 2) ? 1 : 2) void flas
   auto tile_rsrc = [&](int t, int page, __amdgpu_buffer_rsrc_t& tk, __amdgpu_buffer_rsrc_t& tv) {
     const bool ok = page >= 0 && page < p.n_pages;
     const size_t base = (size_t)(ok ? page : 0) * kPageElems + (size_t)g * kPageHead;
-    const int bytes = ok ? max(0, min(BKEY, nkeys - t * BKEY)) * kRowBytes : 0;
+    // (a split's tiles past its keys have no bytes; uniform by hand, since the clamp between two bounds
+    // is a vector instruction and would take the descriptor's loads through readfirstlane loops)
+    int bytes = ok ? min(BKEY, nkeys - t * BKEY) * kRowBytes : 0;
+    if constexpr (SPLIT) bytes = __builtin_amdgcn_readfirstlane(max(0, bytes));
     tk = __builtin_amdgcn_make_buffer_rsrc((void*)(p.k + base), 0, bytes, kBufferFlags);
     tv = __builtin_amdgcn_make_buffer_rsrc((void*)(p.v + base), 0, bytes, kBufferFlags);
   };
