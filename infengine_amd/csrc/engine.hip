@@ -619,15 +619,16 @@ bool grow_scratch(Context* c, float*& buf, size_t& bytes, size_t need, size_t mo
 // its stream, but graphs recorded from it may be replayed at once and after it is gone: a recorded
 // call holds no state of the context and runs unsplit, as does one that finds no memory.
 void attn_part_scratch(Context* c, AttnPrefillParams& a) {
-  if (a.S < 1 || a.start_pos < 0 || recording(c)) return;  // (the launcher refuses the former)
+  if (a.S < 1 || a.start_pos < 0) return;  // (the launcher refuses them)
   constexpr size_t row = kAttnPrefillPartRow * sizeof(float);
   const int splits = attn_prefill_splits(a.S, a.start_pos + a.S, kAttnPrefillPartRows);
-  const size_t need = splits > 1 ? splits * a.S * row : 0;
+  if (splits < 2 || recording(c)) return;
+  const size_t need = splits * a.S * row;
   if (need > c->attn_part_bytes &&
       !grow_scratch(c, c->attn_part, c->attn_part_bytes, need, kAttnPrefillPartRows * row))
     return;
   a.part = c->attn_part;
-  a.part_rows = (int)(need / row);
+  a.part_rows = splits * a.S;
 }
 
 // aux_ready: aux_buffer already holds this layer's input RMSNorm of data_buffer (written by
