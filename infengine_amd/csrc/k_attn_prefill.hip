@@ -420,14 +420,14 @@ void launch_form(const AttnPrefillParams& p, hipStream_t st) {
 
 }  // namespace
 
-// Without a split the time is the
-// longest row block's walk over its key tiles however few CUs that keeps busy: 200 rows at
-// position 30000 took 521 us on 104 workgroups, 135 in 9 splits (504 workgroups); 32 rows at 2500
-// 48 -> 17, 700 at 8000 186 -> 130.  The model, in tiles: workgroups per CU (the second costs 0.85
-// of the first) x a split's tiles + 2, plus the merge kernel's launch (4) and its partials (0.5 per
-// 64 rows and split); a split has to save 15% of it.  Within 3% of the best split count on average
-// over 1-1300 rows at 500-60000 keys; from about 1000 rows on few keys the row blocks fill the chip
-// and it answers 1.
+// Without a split the time is the longest row block's walk over its key tiles however few CUs that
+// keeps busy: 200 rows at position 30000 took 521 us on 104 workgroups, 135 in 9 splits (504
+// workgroups); 32 rows at 2500 48 -> 17, 700 at 8000 186 -> 130.  The model, in tiles: workgroups per CU
+// (the second costs 0.85 of the first) x a split's tiles + 2, plus the merge kernel's launch (4) and
+// its partials (0.5 per 64 rows and split); a split has to save 15% of it.  Within 3% of the best split
+// count on average over 1-1300 rows at 500-60000 keys; from about 1000 rows on few keys the row blocks
+// fill the chip and it answers 1.  Below 64 tiles, where that saving is a few us, the partials count half
+// as much again (256 rows at 1000 ran 22.6 us in 3 splits, 19.9 unsplit; 512 at 2000 39.6 and 36.2).
 int attn_prefill_splits(int S, int nkeys, int part_rows) {
   const int wgs = (S + 31) / 32 * kKVHeads, tiles = (nkeys + BKEY - 1) / BKEY;
   const auto cost = [&](int s) {
@@ -439,6 +439,7 @@ int attn_prefill_splits(int S, int nkeys, int part_rows) {
   double best_cost = 0.85 * cost(1);
   for (int s = 2; s <= 32 && 2 * s <= tiles && s * S <= std::min(part_rows, kAttnPrefillPartRows); ++s)
     if (cost(s) < best_cost) best = s, best_cost = cost(s);
+  if (best > 1 && tiles < 64 && best_cost + 0.25 / 64 * best * S >= 0.85 * cost(1)) best = 1;
   return best;
 }
 
