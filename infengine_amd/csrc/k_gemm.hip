@@ -1299,25 +1299,29 @@ double tile_us(int bn, int bm, double step, double kt, double wgs) {
 TilePlan plan_tiles(int epi, const GemmParams& p) {
   const bool sw = epi == kGemmSwiglu, rope = rope_product(epi, p);
   const int kt = p.K / 64;
-  const bool can_split = p.split_ws && !sw && epi != kGemmF32 && p.N % 8 == 0 && p.ldy % 8 == 0;
-  const double plane = (double)p.M * p.N * 4;
-  const double weights = (double)p.N * p.K * (sw ? 4 : 2) / 3.5e6;
+  // SwiGLU: unsplit a tile's W rows are half gate, half up; split it is a plain product of 2N columns
+  const int cols = sw ? 2 * p.N : p.N;
+  const bool can_split =
+      p.split_ws && epi != kGemmF32 && p.N % (sw ? 16 : 8) == 0 && p.ldy % 8 == 0;
+  const double plane = (double)p.M * cols * 4;
+  const double weights = (double)cols * p.K * 2 / 3.5e6;
   TilePlan best;
   for (int k = 0; k < kTileKinds; ++k) {
     const TileKind& t = kTiles[k];
-    if (sw && (t.bn / 2 * t.wx / 4) % 64 != 0) continue;
     if (!rope && t.bn == 192) continue;
-    const long long tiles =
-        (long long)((p.M + t.bm - 1) / t.bm) * ((p.N + (sw ? t.bn / 2 : t.bn) - 1) / (sw ? t.bn / 2 : t.bn));
+    const long long m_tiles = (p.M + t.bm - 1) / t.bm;
     for (int s = 1; s <= 16; ++s) {
-      if (s > 1 && (!can_split || kt % s != 0 || tiles * s > 512 || t.bn == 192 ||
-                    s * plane > (double)p.split_ws_bytes))
+      const bool split = s > 1;
+      const int width = sw && !split ? t.bn / 2 : t.bn;
+      const long long tiles = m_tiles * (((split ? cols : p.N) + width - 1) / width);
+      if (split ? !can_split || kt % s != 0 || tiles * s > 512 || t.bn == 192 ||
+                      s * plane > (double)p.split_ws_bytes
+                : (rope && t.bn != 192) || (sw && (t.bn / 2 * t.wx / 4) % 64 != 0))
         continue;
-      if (s == 1 && rope && t.bn != 192) continue;
       const double wgs = (double)tiles * s;
       const double rounds = wgs <= 256 ? 1 : 0.71 * ((tiles * s + 255) / 256) + 0.29 * wgs / 256;
       double us = std::max(rounds * tile_us(t.bn, t.bm, t.step, (double)kt / s, wgs), weights) + 1.4;
-      if (s > 1) us += 3.2 + 0.245e-6 * s * plane;
+      if (split) us += 3.2 + 0.245e-6 * s * plane;
       else if (epi == kGemmResid) us += 2 + 0.0021 * p.M;
       if (us < best.us) best = {k, s, us};
     }
@@ -1632,7 +1636,12 @@ int launch_tiled(int epi, const GemmParams& p, hipStream_t st) {
   if (plan.splits > 1) {
     GemmParams q = p;
     q.yf = p.split_ws;
-    q.ldy = p.N;
+    if (epi == kGemmSwiglu) {
+      q.N = 2 * p.N;  // rows [0, N) of w0 (gate), then [N, 2N) of w1 (up)
+      q.n0 = p.N;
+      q.n1 = p.N;
+    }
+    q.ldy = q.N;
     q.k_splits = plan.splits;
     IE_TRY(launch_kind<kGemmF32>(plan.kind, q, st));
     return launch_split_reduce(epi, p, plan.splits, st);

@@ -390,8 +390,9 @@ def test_gemm_schedules_bit_identical(hip, ctx, epi, m, k, n):
 
 # Every tile shape of the prefill GEMM past 128 rows at the first, last or a middle row count that
 # picks it, ragged columns (n = 1000, 4104), one and three k-steps.  K split: resid of 130-512 rows
-# at k = 4096 (8, 4, 4, 2 and 2 planes) and of 300-901 at 14336 (4), bf16 of 161 rows (8); the rest
-# unsplit, as SwiGLU, fp32 and this entry point past 1024 rows always are.
+# at k = 4096 (8, 4, 4, 2 and 2 planes), of 300-901 at 14336 (4), bf16 of 161 rows (8), SwiGLU of
+# 200 and 777 rows at 14336 (8 and 4, over gate then up columns); the rest unsplit, as fp32 and this
+# entry point past 1024 rows always are.
 @pytest.mark.parametrize("epi,m,k,n", [
     ("resid", 130, 4096, 4096), ("resid", 192, 4096, 4096), ("resid", 257, 4096, 4096),
     ("resid", 385, 4096, 4104), ("resid", 512, 4096, 4096), ("resid", 929, 4096, 4096),
@@ -402,7 +403,7 @@ def test_gemm_schedules_bit_identical(hip, ctx, epi, m, k, n):
     ("f32", 129, 4096, 4096), ("f32", 1025, 192, 4100), ("f32", 2100, 4096, 4096),
     ("swiglu", 129, 4096, 14336), ("swiglu", 256, 4096, 14336), ("swiglu", 257, 4096, 14336),
     ("swiglu", 384, 4096, 14336), ("swiglu", 385, 4096, 14336), ("swiglu", 449, 4096, 14340),
-    ("swiglu", 2100, 256, 1000)])
+    ("swiglu", 2100, 256, 1000), ("swiglu", 200, 14336, 128), ("swiglu", 777, 14336, 1040)])
 def test_gemm_tile_shapes(hip, ctx, epi, m, k, n):
     """Products past 128 rows against torch in float32 on every row (|y - y_ref| <= 2 bf16 steps of
     the value, as in assert_bf16_close), nothing written past the last row, and the same bits from
@@ -466,6 +467,31 @@ def test_gemm_ex_same_on_any_context(hip, ctx, epi, m, k, n):
         outs.append(y)
         c.close()
     assert torch.equal(outs[0], outs[1])
+
+
+def test_gemm_swiglu_few_columns_time(hip, ctx):
+    """SwiGLU over few columns and a long K splits K as the plain product of its gate and up columns
+    does: about that product's time (unsplit it took 5 times it).  The bound is 2; the least of
+    five rounds of 20 calls each."""
+    say("gemm_ex SwiGLU time over few columns")
+    m, k, n = 200, 14336, 128
+    g = torch.Generator(device="cuda").manual_seed(8)
+    x, w = (torch.empty(r, k, dtype=torch.bfloat16, device="cuda").normal_(0.0, 1.0, generator=g)
+            for r in (m, 2 * n))
+    y = torch.empty(m, 2 * n, dtype=torch.bfloat16, device="cuda")
+    ms = []
+    for epi, cols, w1 in (("bf16", 2 * n, None), ("swiglu", n, P(w[n:]))):
+        rounds = []
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(20):
+                hip.check(hip.lib.ie_gemm_ex(ctx.handle, GEMM_EPI[epi], m, k, cols, P(x), P(w), w1, P(y)))
+            b.record()
+            sync()
+            rounds.append(a.elapsed_time(b))
+        ms.append(min(rounds[1:]))
+    assert ms[1] <= 2 * ms[0], ms
 
 
 def test_gemm_ex_captured_then_larger(hip, ctx):
