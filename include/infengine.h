@@ -364,7 +364,7 @@ IE_API int ie_gemm_bf16(ie_context* ctx, int m, int k, int n, const ie_bf16* d_x
  *   IE_GEMM_F32     y[m,n] = X . W0^T                               (d_y fp32)
  *   IE_GEMM_SWIGLU  y[m,n] = swiglu(bf16(X . W0^T), bf16(X . W1^T)) (d_y bf16; W0 gate, W1 up)
  * W0/W1 are [n][k]; n % 4 == 0, k % 64 == 0.
- * Up to 1024 rows the product may split K over a scratch of the context, allocated by the first
+ * The product may split K over a scratch of the context, allocated by the first
  * call that needs more of it (refused while the context's stream is captured: run such a call
  * once before) and kept until the context is destroyed.  Graphs recorded from one context with
  * such calls share it: they must not replay at once, nor after the context. */

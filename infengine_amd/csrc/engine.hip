@@ -717,6 +717,7 @@ int prefill_layer(Context* c, hipStream_t st, const ie_model_weights& W, int l, 
   skinny_split(c, kGemmResid, o, c->d_sk_part);
   // with K split the reduction applies the post-attention RMSNorm too
   int normed = 0;
+  o.norm_follows = true;
   o.rn_w = L.post_attention_layernorm;
   o.rn_out = aux_buffer;
   o.rn_done = &normed;
@@ -750,6 +751,7 @@ int prefill_layer(Context* c, hipStream_t st, const ie_model_weights& W, int l, 
                                   align256((size_t)S * kFFN * 2));
   skinny_split(c, kGemmResid, dn, c->d_sk_part);
   int next_normed = 0;
+  dn.norm_follows = true;  // (a layer run alone splits as in the chain)
   if (next_norm_w) {
     dn.rn_w = next_norm_w;
     dn.rn_out = aux_buffer;
@@ -1402,7 +1404,7 @@ int ie_gemm_ex(ie_context* c, int epilogue, int m, int k, int n, const ie_bf16* 
   // split K's partials: a context-owned scratch, grown on first use (op-level entry; the
   // engine passes its own workspace).  The product is offered the bytes of its own size however
   // large the scratch is, so that its K split (and its bits) do not depend on earlier calls.
-  const size_t need = epilogue == IE_GEMM_F32 ? 0 : gemm_split_bytes(m, epilogue == IE_GEMM_SWIGLU ? 2 * n : n);
+  const size_t need = epilogue == IE_GEMM_F32 ? 0 : gemm_op_split_bytes(m, epilogue == IE_GEMM_SWIGLU ? 2 * n : n);
   if (need > c->gemm_ws_bytes && !grow_scratch(c, c->gemm_ws, c->gemm_ws_bytes, need)) {
     set_error("gemm_ex: no %zu bytes of scratch (or the stream is capturing)", need);
     return IE_ERR_HIP;

@@ -214,6 +214,7 @@ struct GemmParams {
   const uint16_t* rn_w;
   uint16_t* rn_out;
   int* rn_done;
+  bool norm_follows;  // a layer's product: such an RMSNorm follows it, here or in the next layer
   int k_splits;  // set by the launcher for the wide kernel (0 / 1: no split)
   // Skinny GEMM (M <= 16): the last sk_tail of its tiles (16 rows; 32 for the fp32 epilogue
   // at K = 4096 or 14336) run as two workgroups each, one per K half, so that every CU gets the
@@ -231,6 +232,14 @@ constexpr int kSplitMaxRows = 1024;
 // output columns): 2048 partial rows, i.e. up to 16 planes at M <= 128, 4 at M = 512.
 inline size_t gemm_split_bytes(int M, int n) {
   return M <= kSplitMaxRows ? (size_t)(4 * M > 2048 ? 4 * M : 2048) * n * sizeof(float) : 0;
+}
+// The same for the op-level entry, whose products have any shape: 16 planes, or as many as 64 MiB
+// hold (two planes of the 2048-row down projection), where that is more.
+inline size_t gemm_op_split_bytes(int M, int n) {
+  const size_t plane = (size_t)M * n * sizeof(float);
+  const size_t planes = plane ? ((size_t)64 << 20) / plane : 0;
+  const size_t room = planes < 2 ? 0 : (planes < 16 ? planes : 16) * plane;
+  return room > gemm_split_bytes(M, n) ? room : gemm_split_bytes(M, n);
 }
 int launch_gemm(int epi, const GemmParams& p, hipStream_t st);
 // Prefill QKV projection with RoPE and the K/V scatter in the GEMM epilogue (kGemmQkvRope,

@@ -1291,8 +1291,8 @@ double tile_us(int bn, int bm, double step, double kt, double wgs) {
 //   launch 1.4 + rounds x (k-steps x step + 3.95 + 4.18 x tile / 64 Ki)
 // a step 28% faster on an empty chip than on a full one; past one round 0.71 of the time goes
 // with whole rounds, 0.29 with the tiles; K splits add 3.2 + 0.245 per MB of fp32 partials; the
-// weights stream at 3.5 TB/s at best beside the products.  What follows an unsplit residual product
-// as a launch of its own (the RMSNorm, which the split reduction runs) counts too.
+// weights stream at 3.5 TB/s at best beside the products.  The RMSNorm that follows a layer's residual
+// product counts too where it is a launch of its own (unsplit; the split reduction runs it).
 // Before, tiles were 256 x 256, 256 x 128 or 192 x 256 (and 128 x 128 with an older kernel), K
 // split up to 1024 rows only: 640 rows 201 -> 134 us (gate/up), 117 -> 77 (down), 1200 rows down
 // 189 -> 125, 6000 rows down 661 -> 551.
@@ -1322,7 +1322,7 @@ TilePlan plan_tiles(int epi, const GemmParams& p) {
       const double rounds = wgs <= 256 ? 1 : 0.71 * ((tiles * s + 255) / 256) + 0.29 * wgs / 256;
       double us = std::max(rounds * tile_us(t.bn, t.bm, t.step, (double)kt / s, wgs), weights) + 1.4;
       if (split) us += 3.2 + 0.245e-6 * s * plane;
-      else if (epi == kGemmResid) us += 2 + 0.0021 * p.M;
+      else if (p.norm_follows) us += 2 + 0.0021 * p.M;
       if (us < best.us) best = {k, s, us};
     }
   }
@@ -1404,7 +1404,7 @@ int dual_tail(int epi, const GemmParams& p, double plan_us) {
   const long long tail = (long long)((p.M + 127) / 128) * ((p.N - head + tn - 1) / tn);
   const double us = 1.4 + (double)(tiles / 256) * tile_us(256, 256, kTiles[kTileBig].step, kt, 256) +
                     (double)((tail + 255) / 256) * tile_us(256, 128, kStep256x128, kt, 256) +
-                    (epi == kGemmResid ? 2 + 0.0021 * p.M : 0);
+                    (p.norm_follows ? 2 + 0.0021 * p.M : 0);
   return us < plan_us ? p.N - head : 0;
 }
 
