@@ -39,27 +39,31 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) short4_t lds_short4;
 
-constexpr int kBatchedWaves = 12, kBatchedTile = 32;
+constexpr int kSplitWaves = 8, kBatchedWaves = 12;  // waves a workgroup: batch 1, batched
+constexpr int kKeys = 32;                           // keys per wave tile (a page holds two)
 constexpr int kRowBytes = kHeadDim * 2;
 constexpr int kBufferFlags = 0x00020000;   // buffer descriptor word 3 (raw 32-bit access)
-static_assert(kAttnTile == 64, "tile = 4 x 16-key MFMA blocks");
+static_assert(kAttnTile % kKeys == 0, "a wave tile lies in one page");
 
 // chunk c of key r of a tile at slot c ^ (r & 15) (LDS bank spread for the fragment reads)
 __device__ __forceinline__ int kv_slot(int r, int c) { return r * 16 + (c ^ (r & 15)); }
 
 static_assert(kAttnSplits <= 64, "the merge gives each split one lane");
-// A wave preloads the page ids of its tiles, one per lane: with kAttnSplits splits of
-// kSplitWaves waves, the longest context keeps that within 64 tiles per wave.
-static_assert(kMaxLongCtx / kAttnTile <= 64 * kAttnSplits * 4, "page ids per wave exceed a wave");
+// A wave preloads the page ids of its tiles, one per lane: with kAttnSplits splits of kSplitWaves
+// waves the longest context keeps that within 64 tiles per wave; a batched run has at most 5 rounds
+// more than kAttnSplits runs of kBatchedWaves waves need (run_rounds).
+static_assert(kMaxLongCtx / kKeys <= 64 * kAttnSplits * kSplitWaves &&
+                  kMaxLongCtx / kKeys <= (64 - 6) * kAttnSplits * kBatchedWaves,
+              "page ids per wave exceed a wave");
 
 // A workgroup's LDS, each array its own variable (the compiler then sees that the tile loads do not
 // write the partials): per wave its K tile (then V over it) and V tile, and the 4 heads' partials.
-template <bool VREG, int KT>
-using KvSlice = u32x4_t[VREG ? 1 : 2][KT * 16];
+template <bool VREG>
+using KvSlice = u32x4_t[VREG ? 1 : 2][kKeys * 16];
 using PartO = float[kGQA][kHeadDim];
 using PartMl = float[kGQA][2];
 
-// The tiles t0 .. t1-1 (KT keys each) of (sequence b, kv head g) with S positions: the NW waves
+// The tiles t0 .. t1-1 (kKeys keys each) of (sequence b, kv head g) with S positions: the NW waves
 // take every NW-th tile and leave their partials (m, l, o) of the 4 q heads in xo / xml
 // (a barrier ends it).  VREG: one LDS slice per wave, K through it and V staged in registers then
 // written over K (120 KiB for the 12-wave form); otherwise K and V each have a slice (136 KiB, one
@@ -71,16 +75,13 @@ using PartMl = float[kGQA][2];
 // the others.  The batch-1 split form likewise runs 8 waves on 32-key tiles (the same tiles per
 // split, half the work per wave): 4.85 against 5.07 us at S = 550-610.
 // AUX: the loads' cache policy (0, or 2: nontemporal).
-template <bool VREG, int NW, int KT, int AUX>
+template <bool VREG, int NW, int AUX>
 __device__ __forceinline__ void attend_tiles(const AttnDecodeParams& p, int tid, int b, int g, int S,
-                                             int t0, int t1, KvSlice<VREG, KT>* kv, PartO* xo,
+                                             int t0, int t1, KvSlice<VREG>* kv, PartO* xo,
                                              PartMl* xml) {
-  // KT: keys per tile, 64 or 32 (half tiles: twice the waves on a context's tiles; a page
-  // holds two)
-  static_assert(KT == 64 || KT == 32, "tile of 64 or 32 keys");
-  constexpr int KB = KT / 16;   // 16-key MFMA blocks per tile
-  constexpr int KS2 = KT / 32;  // 32-key P.V contraction chunks per tile
-  constexpr int NJ = KT / 4;    // 1 KiB loads per tile (4 rows each)
+  static_assert(kKeys == 32, "one P.V contraction per tile");
+  constexpr int KB = kKeys / 16;  // 16-key MFMA blocks per tile
+  constexpr int NJ = kKeys / 4;   // 1 KiB loads per tile (4 rows each)
   // wave id made provably uniform: the tile indices and buffer descriptors derived from it stay
   // in SGPRs (otherwise every buffer load becomes a readfirstlane loop)
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -118,11 +119,11 @@ __device__ __forceinline__ void attend_tiles(const AttnDecodeParams& p, int tid,
   int page_of = 0;
   if (paged) {
     const int t = t0 + wave + NW * lane;
-    page_of = t < t1 ? p.block_table[(size_t)b * p.table_stride + t * KT / kAttnTile] : -1;
+    page_of = t < t1 ? p.block_table[(size_t)b * p.table_stride + t * kKeys / kAttnTile] : -1;
   }
   int it = 0;
   for (int t = t0 + wave; t < t1; t += NW, ++it) {
-    const int key0 = t * KT;
+    const int key0 = t * kKeys;
     // the tile's buffers: rows key0.. of the sequence's cache, or rows 0.. of its page (a page
     // id outside the pool reads as zero)
     __amdgpu_buffer_rsrc_t krs = krs_seq, vrs = vrs_seq;
@@ -203,16 +204,10 @@ __device__ __forceinline__ void attend_tiles(const AttnDecodeParams& p, int tid,
     m = mn;
 #pragma unroll
     for (int db = 0; db < 8; ++db) o[db] *= alpha;
-    // P^T fragments: slot 8 G + r <-> key 32 ks2 + 4 G + r, slot 8 G + 4 + r <-> key
-    // 32 ks2 + 16 + 4 G + r
-    bf16x8_t pb[KS2];
-#pragma unroll
-    for (int ks2 = 0; ks2 < KS2; ++ks2) {
-      const u32x4_t w = {pack_bf2(s[2 * ks2][0], s[2 * ks2][1]), pack_bf2(s[2 * ks2][2], s[2 * ks2][3]),
-                         pack_bf2(s[2 * ks2 + 1][0], s[2 * ks2 + 1][1]),
-                         pack_bf2(s[2 * ks2 + 1][2], s[2 * ks2 + 1][3])};
-      pb[ks2] = __builtin_bit_cast(bf16x8_t, w);
-    }
+    // P^T fragment: slot 8 G + r <-> key 4 G + r, slot 8 G + 4 + r <-> key 16 + 4 G + r
+    const u32x4_t pw = {pack_bf2(s[0][0], s[0][1]), pack_bf2(s[0][2], s[0][3]),
+                        pack_bf2(s[1][0], s[1][1]), pack_bf2(s[1][2], s[1][3])};
+    const bf16x8_t pb = __builtin_bit_cast(bf16x8_t, pw);
     // ---- O^T[d][q] += V^T[d][keys] . P^T[keys][q]; V^T by transposed LDS reads (source lane
     //      s of a 16-lane group reads V[key0 + s/4][d0 + 4 (s%4) .. +3])
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the V tile has landed (LDS or registers)
@@ -226,17 +221,13 @@ __device__ __forceinline__ void attend_tiles(const AttnDecodeParams& p, int tid,
 #pragma unroll
     for (int db = 0; db < 8; ++db) {
       const int c = 2 * db + (dq >> 1), hb = (dq & 1) * 8;
-#pragma unroll
-      for (int ks2 = 0; ks2 < KS2; ++ks2) {
-        const int ka = 32 * ks2 + 4 * G + kr;
-        const char* va = reinterpret_cast<const char*>(&vt[kv_slot(ka, c)]) + hb;
-        const char* vb = reinterpret_cast<const char*>(&vt[kv_slot(ka + 16, c)]) + hb;
-        const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)va);
-        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)vb);
-        const short4_t both[2] = {lo, hi};
-        o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, both), pb[ks2],
-                                                        o[db], 0, 0, 0);
-      }
+      const char* va = reinterpret_cast<const char*>(&vt[kv_slot(4 * G + kr, c)]) + hb;
+      const char* vb = reinterpret_cast<const char*>(&vt[kv_slot(4 * G + kr + 16, c)]) + hb;
+      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)va);
+      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)vb);
+      const short4_t both[2] = {lo, hi};
+      o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, both), pb, o[db],
+                                                      0, 0, 0);
     }
     // the next tile's loads overwrite this slice: every read of it has returned
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -279,31 +270,29 @@ __device__ __forceinline__ AttnMerged merge_waves(const PartO* xo, const PartMl*
 }
 
 // Batch 1, phase 1: split s of kv head g attends its run of tiles and writes the unnormalised
-// partial (m, l, o) of each of the 4 q heads.  Splits are counted in 64-key tiles whatever the
-// tile, as the merge counts them.
-template <int NW, int KT>
-__global__ __launch_bounds__(NW * 64) void attn_decode_split_kernel(AttnDecodeParams p) {
-  __shared__ KvSlice<false, KT> kv[NW];
+// partial (m, l, o) of each of the 4 q heads.  Splits are counted in 64-key tiles, as the merge and
+// the O projection count them.
+__global__ __launch_bounds__(kSplitWaves * 64) void attn_decode_split_kernel(AttnDecodeParams p) {
+  constexpr int NW = kSplitWaves;
+  __shared__ KvSlice<false> kv[NW];
   __shared__ PartO xo[NW];
   __shared__ PartMl xml[NW];
-  const int split = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
+  const int split = blockIdx.x, g = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // (the arguments in one go: a cache line of them first touched later is a wait of its own:
   // a decode step of 32 launches took 2736-2744 us without, 2731-2734 with, 4.84 us a launch)
-  asm volatile("" ::"s"(p.q), "s"(p.k_cache), "s"(p.v_cache), "s"(p.cache_batch_stride),
-               "s"(p.block_table), "s"(p.n_pages), "s"(p.part_o), "s"(p.part_ml), "s"(p.d_seq_len),
-               "s"(p.seq_len), "s"(p.max_splits));
-  const int S = p.d_seq_len ? p.d_seq_len[b] : p.seq_len;
-  const int ntiles = (S + KT - 1) / KT;
-  // (split count in 64-key tiles whatever KT: the merge and the O projection count the same)
+  asm volatile("" ::"s"(p.q), "s"(p.k_cache), "s"(p.v_cache), "s"(p.block_table), "s"(p.n_pages),
+               "s"(p.part_o), "s"(p.part_ml), "s"(p.d_seq_len), "s"(p.seq_len), "s"(p.max_splits));
+  const int S = p.d_seq_len ? p.d_seq_len[0] : p.seq_len;
+  const int ntiles = (S + kKeys - 1) / kKeys;
   const int ns = attn_decode_splits((S + kAttnTile - 1) / kAttnTile, p.max_splits);
   if (split >= ns) return;  // whole workgroup: nobody reads a partial past ns
   const int tps = (ntiles + ns - 1) / ns;
   const int t0 = split * tps, t1 = min(ntiles, t0 + tps);
-  attend_tiles<false, NW, KT, 0>(p, threadIdx.x, b, g, S, t0, t1, kv, xo, xml);
-  if (wave >= kGQA) return;  // (NW > 4) waves past the 4 q heads only contribute partials
+  attend_tiles<false, NW, 0>(p, threadIdx.x, 0, g, S, t0, t1, kv, xo, xml);
+  if (wave >= kGQA) return;  // waves past the 4 q heads only contribute partials
   const AttnMerged r = merge_waves<NW>(xo, xml, wave, lane);
-  const size_t slot = (((size_t)b * kKVHeads + g) * kAttnSplits + split) * kGQA + wave;
+  const size_t slot = ((size_t)g * kAttnSplits + split) * kGQA + wave;
   *reinterpret_cast<float2*>(p.part_o + slot * kHeadDim + 2 * lane) = make_float2(r.o0, r.o1);
   if (lane == 0) *reinterpret_cast<float2*>(p.part_ml + slot * 2) = make_float2(r.M, r.L);
 }
@@ -396,10 +385,11 @@ __device__ __forceinline__ int run_rounds(int ntiles) {
 // sequences of 225-1800 25.3, now 23.2; 2 of them 20.7, 11.5; 16 of 375-3000 37, 33; 16 of
 // 2850-7000 86, 69; 6 of 2500-20000 67, 57.
 // NT: nontemporal K/V loads, for K/V that cannot stay in the 256 MB cache until the next step.
-template <int NW, int KT, bool SHORT, bool NT>
-__global__ __launch_bounds__(NW * 64) void attn_decode_batched_kernel(AttnDecodeParams p, unsigned int* counters,
-                                                               int batch) {
-  __shared__ KvSlice<true, KT> kv[NW];
+template <bool SHORT, bool NT>
+__global__ __launch_bounds__(kBatchedWaves * 64) void attn_decode_batched_kernel(
+    AttnDecodeParams p, unsigned int* counters, int batch) {
+  constexpr int NW = kBatchedWaves;
+  __shared__ KvSlice<true> kv[NW];
   __shared__ PartO xo[NW];
   __shared__ PartMl xml[NW];
   __shared__ int s_last;
@@ -411,7 +401,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_batched_kernel(AttnDecode
   // them from registers; LDS keeps them for the next ones (through the tiles they would cost
   // registers that those need)
   int len = lane < batch ? p.d_seq_len[lane] : 0;
-  const int nt = (len + KT - 1) / KT;
+  const int nt = (len + kKeys - 1) / kKeys;
   int rounds = run_rounds<SHORT, NW>(nt);
   if constexpr (!SHORT) rounds = __builtin_amdgcn_readlane(rounds, 0);  // (one for the batch)
   int upto = lane < batch ? (nt + rounds * NW - 1) / (rounds * NW) : 0;
@@ -424,7 +414,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_batched_kernel(AttnDecode
   for (int w = blockIdx.x; w < total; w += gridDim.x) {
     const int b = __popcll(__ballot(lane < batch && upto * kKVHeads <= w));
     const int S = __builtin_amdgcn_readlane(len, b);
-    const int ntiles = (S + KT - 1) / KT;
+    const int ntiles = (S + kKeys - 1) / kKeys;
     const int tps = NW * (SHORT ? run_rounds<SHORT, NW>(ntiles) : rounds);
     const int ns = (ntiles + tps - 1) / tps;
     const int i = w - (__builtin_amdgcn_readlane(upto, b) - ns) * kKVHeads;
@@ -432,7 +422,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_batched_kernel(AttnDecode
     // (the thread id made opaque per item: what is derived from it is not kept across the loop)
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
-    attend_tiles<true, NW, KT, NT ? 2 : 0>(p, tid, b, g, S, split * tps, min(ntiles, split * tps + tps),
+    attend_tiles<true, NW, NT ? 2 : 0>(p, tid, b, g, S, split * tps, min(ntiles, split * tps + tps),
                                              kv, xo, xml);
     const size_t bg = (size_t)b * kKVHeads + g;
     AttnMerged r{};
@@ -525,8 +515,8 @@ int launch_attn_decode(const AttnDecodeParams& p, bool merge, hipStream_t st) {
   IE_REQUIRE(p.max_splits > 1 && p.max_splits <= kAttnSplits, "attn_decode: max_splits %d",
              p.max_splits);
   // one workgroup per possible split: idle ones would still cost dispatch
-  hipLaunchKernelGGL((attn_decode_split_kernel<8, 32>), dim3(p.max_splits, kKVHeads),
-                     dim3(8 * 64), 0, st, p);
+  hipLaunchKernelGGL(attn_decode_split_kernel, dim3(p.max_splits, kKVHeads),
+                     dim3(kSplitWaves * 64), 0, st, p);
   IE_CHECK_LAUNCH();
   if (merge) {
     IE_REQUIRE(p.out, "attn_decode: merge needs an output buffer");
@@ -542,10 +532,10 @@ int launch_attn_decode_batched(const AttnDecodeParams& p, unsigned int* counters
   IE_REQUIRE(p.d_seq_len && p.out && counters && max_len >= 1 && max_len <= kMaxLongCtx,
              "attn_decode: batched lengths, output and counters");
   // the most items: a run of one round per kBatchedWaves tiles, at most kAttnSplits of them
-  const int runs = std::min((max_len + kBatchedTile * kBatchedWaves - 1) / (kBatchedTile * kBatchedWaves), kAttnSplits);
+  const int runs = std::min((max_len + kKeys * kBatchedWaves - 1) / (kKeys * kBatchedWaves), kAttnSplits);
   const dim3 grid(std::min(runs * kKVHeads * batch, 256)), block(kBatchedWaves * 64);
 #define IE_ATTN(SHORT, NT) \
-  hipLaunchKernelGGL((attn_decode_batched_kernel<kBatchedWaves, kBatchedTile, SHORT, NT>), grid, block, 0, st, p, counters, batch)
+  hipLaunchKernelGGL((attn_decode_batched_kernel<SHORT, NT>), grid, block, 0, st, p, counters, batch)
   if (max_len <= kAttnShortMaxCtx) {
     if (nt) IE_ATTN(true, true);
     else IE_ATTN(true, false);
