@@ -154,7 +154,9 @@ IE_API int ie_generate(ie_context* ctx, const ie_model_weights* weights, const i
  * tokenid_buffs is a device array [batch][8192]; row b's K/V live in
  * kv_caches + b * ie_kv_cache_size().  data/attn buffers are [batch, 4096];
  * output_distr [batch, 128256]; output_tokens (device) [batch]; tokens_out
- * (host, may be NULL) receives the greedy ids. */
+ * (host, may be NULL) receives the greedy ids.  While no sequence is past 2048
+ * positions a row's results do not depend on the other rows; past that its
+ * attention is cut by all the lengths, and its rounding depends on them. */
 IE_API size_t ie_batch_workspace_size(int batch);
 IE_API int ie_decode_step_batched(ie_context* ctx, const ie_model_weights* weights, int batch,
                                   const int* seq_lens, int* tokenid_buffs,

@@ -279,10 +279,6 @@ __global__ __launch_bounds__(kSplitWaves * 64) void attn_decode_split_kernel(Att
   __shared__ PartMl xml[NW];
   const int split = blockIdx.x, g = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // (the arguments in one go: a cache line of them first touched later is a wait of its own:
-  // a decode step of 32 launches took 2736-2744 us without, 2731-2734 with, 4.84 us a launch)
-  asm volatile("" ::"s"(p.q), "s"(p.k_cache), "s"(p.v_cache), "s"(p.block_table), "s"(p.n_pages),
-               "s"(p.part_o), "s"(p.part_ml), "s"(p.d_seq_len), "s"(p.seq_len), "s"(p.max_splits));
   const int S = p.d_seq_len ? p.d_seq_len[0] : p.seq_len;
   const int ntiles = (S + kKeys - 1) / kKeys;
   const int ns = attn_decode_splits((S + kAttnTile - 1) / kAttnTile, p.max_splits);
@@ -343,8 +339,12 @@ __device__ __forceinline__ AttnMerged merge_runs(const AttnDecodeParams& p, size
 // ntiles tiles.  SHORT (no sequence past kAttnShortMaxCtx): by the sequence's own length, so that
 // its result does not depend on what shares its step: two rounds where one such run covers it (a
 // second run of a short context costs more than its round), else one (more workgroups at once: 2
-// sequences of 225-1800 take 11 us, 21 in one run each).  Otherwise one for the whole batch: the
-// candidate with the least (workgroups' turns, half counted whole) x (rounds + 0.5, an item's
+// sequences of 225-1800 take 11 us, 21 in one run each).  That serves few sequences and mixed lengths
+// at the cost of full batches of one length, whose 3 or 4 runs are two turns of the chip: a step of 16 of
+// 769-1200 takes 3561-3669 us, 3374-3568 in one run each; of 2 of 800-2048 3059-3040 and 3101-3478.  (One
+// run of three rounds to 1024 positions, and two runs past them, mended the full batches and cost
+// 2-8 sequences 2-7%.)  Otherwise one for the whole batch, so that a row's rounding then depends on
+// the lengths that share its step: the candidate with the least (workgroups' turns, half counted whole) x (rounds + 0.5, an item's
 // own cost) whose longest sequence has at most kAttnSplits runs.  Measured / fixed at 1, 2, 3, 4, 6
 // rounds, us a layer: 16 sequences of 2850-7000 85, 70, 68, 75, 73; 6 of 2500-20000 60 (2 rounds
 // at the longest), 66, 66, 57, 67; 2 of 20000 37, 37, 43, 31, 35.
@@ -379,8 +379,9 @@ __device__ __forceinline__ int run_rounds(int ntiles) {
 // in run order -- no workgroup waits, and no merge launch.
 // Workgroups (one a CU: 120 KiB of LDS) walk the items a grid apart; an item list, since a grid of
 // (most runs) x 8 x batch would hold mostly idle workgroups, which take their turns on the CUs.
-// Bound by the K/V loads (a copy without the arithmetic took the same time): 5.0-5.6 TB/s past
-// 100 MB a layer.  Before (one 12-wave workgroup per (sequence, kv head) up to 2048 positions, else
+// Bound by the K/V loads as a wave takes them, one tile at a time (a copy without the arithmetic that
+// kept these turns took the same time; nothing of a wave's next tile is in flight while it computes):
+// 5.0-5.6 TB/s past 100 MB a layer.  Before (one 12-wave workgroup per (sequence, kv head) up to 2048 positions, else
 // up to 32 splits of 4-wave workgroups and a merge launch), us a layer with the K/V from HBM: 16
 // sequences of 225-1800 25.3, now 23.2; 2 of them 20.7, 11.5; 16 of 375-3000 37, 33; 16 of
 // 2850-7000 86, 69; 6 of 2500-20000 67, 57.
@@ -395,7 +396,8 @@ __global__ __launch_bounds__(kBatchedWaves * 64) void attn_decode_batched_kernel
   __shared__ int s_last;
   __shared__ int2 s_seq[16];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // (the arguments in one go: a cache line of them first touched later is a wait of its own)
+  // (the arguments in one go: a cache line of them first touched later is a wait of its own: steps of
+  // 8 and 16 sequences of 500-600 took 3091-3289 us without, 3073-3275 with)
   asm volatile("" ::"s"(p.q), "s"(p.d_seq_len), "s"(p.block_table), "s"(counters), "s"(batch));
   // lane b: sequence b's length and the runs of the sequences up to it.  The first item takes
   // them from registers; LDS keeps them for the next ones (through the tiles they would cost
