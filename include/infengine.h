@@ -278,7 +278,8 @@ IE_API int ie_sample_argmax_rows(ie_context* ctx, int rows, int vocab, const flo
 /* Temperature + top-p (nucleus) sampling over [rows, vocab] fp32 logits; no
  * reference counterpart (sampling.cu has argmax only).  Deterministic:
  * uniform u = counter RNG(seed, row, step); inverse CDF in token-id order over
- * the kept set.  workspace: ie_top_p_workspace_size(rows, vocab) bytes. */
+ * the kept set.  workspace: ie_top_p_workspace_size(rows, vocab) bytes, a float a
+ * logit (not used by the present sampler) and the rows' state. */
 IE_API size_t ie_top_p_workspace_size(int rows, int vocab);
 IE_API int ie_sample_top_p(ie_context* ctx, int rows, int vocab, const float* d_logits,
                            float temperature, float top_p, uint64_t seed, uint64_t step,

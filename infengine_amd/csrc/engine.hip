@@ -1558,7 +1558,7 @@ int ie_sample_argmax_rows(ie_context* c, int rows, int vocab, const float* d_log
 }
 
 size_t ie_top_p_workspace_size(int rows, int vocab) {
-  // the rows' state (all that the sampler uses), past a float a logit: the size is the interface's
+  // the rows' state (all that the sampler uses) and a float a logit: the size is the interface's
   const size_t r = rows < 1 ? 1 : rows, v = vocab < 1 ? 1 : vocab;
   return align256(r * v * sizeof(float)) + top_p_workspace_bytes((int)r);
 }

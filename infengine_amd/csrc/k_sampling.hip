@@ -164,13 +164,13 @@ __device__ __forceinline__ T wave_scan(T v) {
 // The bins are octaves of 1.08 d + 2 in 128 steps each, 0.0145 nats wide at the top, 0.029 past 1.9 and
 // 0.058 past 5.6: a row's cut lies at a few times the spread of its scaled logits, so that a flatter
 // row has its cut where the bins are finer.  The cut bin of N(0, s) logits holds up to about 128256 x
-// width / (2.5 s) tokens: the candidate list takes them from s = 0.08 on.  512 even bins took them from
+// width / (2.5 s) tokens: the candidate list takes them from s = 0.09 on.  512 even bins took them from
 // 0.27 on; 16 rows at p = 0.5, us, even bins / these: s = 0.1 275 / 46, 0.3 46 / 34, 0.8 34.5 / 32, 2.0
 // 29.0 / 29.2 (p = 0.9: 31.3 / 31.9).  (576 bins, even past 1.2 nats: 30.3 and 32.9 at s = 2.0.)
 constexpr int kTopPBins = 512;
 constexpr int kTopPChunks = 64;
 constexpr int kTopPChunkThreads = 256;
-constexpr int kTopPCandMax = 10240;
+constexpr int kTopPCandMax = 9216;
 constexpr int kTopPCandLds = 4096;  // candidates that tp_finish keeps in LDS
 
 struct TopPRow {
@@ -183,7 +183,9 @@ struct TopPRow {
   unsigned long long above, target;
   uint32_t cand_key[kTopPCandMax];
   unsigned long long cand_q[kTopPCandMax];  // mass (41 bits) | chunk << 48
+  unsigned long long pad;
 };
+static_assert(sizeof(TopPRow) == 116000, "callers' workspaces are sized by it (ie_top_p_workspace_size)");
 
 // The octaves 2-4, 4-8, 8-16 and 16-32 of 1.08 d + 2 (from 32 on, and NaN: any bin, without mass).
 __host__ __device__ __forceinline__ int top_p_bin(float d) {

@@ -71,9 +71,16 @@ def test_sizes(hip):
     assert lib.ie_ffn_workspace_size(S) >= S * 14336 * 2
     # decode needs a fixed amount, so a small-S workspace still serves long decodes
     assert lib.ie_attn_workspace_size(1) == lib.ie_attn_workspace_size(0)
-    # top-p: the fp32 exponentials, then per-row state (< 128 KiB a row)
+    # top-p: a float a logit and per-row state (< 128 KiB a row)
     assert 16 * 128256 * 4 < lib.ie_top_p_workspace_size(16, 128256) <= 16 * 128256 * 4 + 16 * (128 << 10)
     assert lib.ie_top_p_workspace_size(1, 128256) < lib.ie_top_p_workspace_size(2, 128256)
+
+
+@pytest.mark.parametrize("rows,vocab,size", [(1, 7, 116256), (1, 128256, 629024),
+                                             (16, 128256, 10064384), (64, 50001, 20224256)])
+def test_top_p_workspace_size_is_fixed(hip, rows, vocab, size):
+    """The size that callers may have laid out: a float a logit to 256 bytes, 116000 bytes a row."""
+    assert hip.lib.ie_top_p_workspace_size(rows, vocab) == size
 
 
 BOGUS = C.c_void_p(0x1000)   # never dereferenced: every call below fails validation first
