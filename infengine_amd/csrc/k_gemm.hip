@@ -1308,7 +1308,9 @@ TilePlan plan_tiles(int epi, const GemmParams& p) {
   TilePlan best;
   for (int k = 0; k < kTileKinds; ++k) {
     const TileKind& t = kTiles[k];
-    if (!rope && t.bn == 192) continue;
+    // (192 W rows: the fused QKV's; a plain bf16 product of one round may take them too, 2048 x 4096 x
+    // 6144 at 85.8 us against 89.3 -- past one round the model is too coarse to tell them apart)
+    if (t.bn == 192 && !rope && epi != kGemmBf16) continue;
     const long long m_tiles = (p.M + t.bm - 1) / t.bm;
     for (int s = 1; s <= 16; ++s) {
       const bool split = s > 1;
@@ -1316,7 +1318,8 @@ TilePlan plan_tiles(int epi, const GemmParams& p) {
       const long long tiles = m_tiles * (((split ? cols : p.N) + width - 1) / width);
       if (split ? !can_split || kt % s != 0 || tiles * s > 512 || t.bn == 192 ||
                       s * plane > (double)p.split_ws_bytes
-                : (rope && t.bn != 192) || (sw && (t.bn / 2 * t.wx / 4) % 64 != 0))
+                : (rope && t.bn != 192) || (!rope && t.bn == 192 && tiles > 256) ||
+                      (sw && (t.bn / 2 * t.wx / 4) % 64 != 0))
         continue;
       const double wgs = (double)tiles * s;
       const double rounds = wgs <= 256 ? 1 : 0.71 * ((tiles * s + 255) / 256) + 0.29 * wgs / 256;

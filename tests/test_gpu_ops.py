@@ -392,7 +392,7 @@ def test_gemm_schedules_bit_identical(hip, ctx, epi, m, k, n):
 # picks it, ragged columns (n = 1000, 4104), one and three k-steps.  K split: resid of 130-512 rows
 # at k = 4096 (8, 4, 4, 2 and 2 planes), of 300-901 at 14336 (4) and 1100 at 14336 (2), bf16 of 161
 # rows (16), SwiGLU of 200 and 777 rows at 14336 (16 and 7, over gate then up columns); the rest
-# unsplit, as fp32 always is.
+# unsplit, as fp32 always is.  bf16 of 2000 and 2048 rows: 192-row W tiles.
 @pytest.mark.parametrize("epi,m,k,n", [
     ("resid", 130, 4096, 4096), ("resid", 192, 4096, 4096), ("resid", 257, 4096, 4096),
     ("resid", 385, 4096, 4104), ("resid", 512, 4096, 4096), ("resid", 929, 4096, 4096),
@@ -404,7 +404,7 @@ def test_gemm_schedules_bit_identical(hip, ctx, epi, m, k, n):
     ("swiglu", 129, 4096, 14336), ("swiglu", 256, 4096, 14336), ("swiglu", 257, 4096, 14336),
     ("swiglu", 384, 4096, 14336), ("swiglu", 385, 4096, 14336), ("swiglu", 449, 4096, 14340),
     ("swiglu", 2100, 256, 1000), ("swiglu", 200, 14336, 128), ("swiglu", 777, 14336, 1040),
-    ("resid", 1100, 14336, 4096)])
+    ("resid", 1100, 14336, 4096), ("bf16", 2048, 4096, 6144), ("bf16", 2000, 4096, 6100)])
 def test_gemm_tile_shapes(hip, ctx, epi, m, k, n):
     """Products past 128 rows against torch in float32 on every row (|y - y_ref| <= 2 bf16 steps of
     the value, as in assert_bf16_close), nothing written past the last row, and the same bits from
