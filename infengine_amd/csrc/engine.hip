@@ -79,8 +79,9 @@ DecodeWs decode_ws(void* ws, int batch) {
 size_t prefill_attn_bytes(int S) {
   return align256((size_t)S * kQKVDim * 2) + align256((size_t)S * kHidden * 2);
 }
-// [h (S x 14336 bf16) | split-K partials of the 4096-column projections (S <= kSplitMaxRows)];
-// the O projection's partials reuse the start (q/k/v and rotated q are dead by then).
+// [h (S x 14336 bf16) | split-K partials of the 4096-column projections (sized for up to
+// kSplitMaxRows rows; more rows split as far as they fit)]; the O projection's partials reuse the
+// start (q/k/v and rotated q are dead by then).
 size_t prefill_split_bytes(int S) { return align256(gemm_split_bytes(std::min(S, kSplitMaxRows), kHidden)); }
 size_t prefill_ffn_bytes(int S) { return align256((size_t)S * kFFN * 2) + prefill_split_bytes(S); }
 
@@ -670,8 +671,9 @@ int prefill_layer(Context* c, hipStream_t st, const ie_model_weights& W, int l, 
   // split K's partials after q/k/v and the rotated q (the rest of the workspace)
   g.split_ws = reinterpret_cast<float*>(wsb + prefill_attn_bytes(S));
   g.split_ws_bytes = (long long)(ie_attn_workspace_size(S) - prefill_attn_bytes(S));
-  // RoPE and the K/V scatter in the product's epilogue where the product runs on the 192 x 256
-  // ping-pong tiles (long prompts), else the product to [S][6144] and the scatter kernel
+  // RoPE and the K/V scatter in the product's epilogue (past 128 rows the 192-row ping-pong tiles) or
+  // in its split reduction; to 16 rows, off 16 bytes and under schedule 0 the product to [S][6144] and
+  // the scatter kernel
   GemmParams f = g;
   f.y = qrot;
   f.ldy = kHidden;

@@ -168,8 +168,8 @@ enum GemmEpi : int {
   // QKV projection with RoPE and the K/V cache write (the [q|k|v] weights as w0/w1/w2):
   // bf16(acc), RoPE on q and k, q to y [M][32][128], k and v to the cache (rope.cu:53-64,
   // attn.cu:345-352).  Batched decode (skinny GEMM, M <= 16): row m at position d_seq_len[m] - 1
-  // of sequence m's cache.  Prefill (launch_qkv_rope_prefill, the 192 x 256 ping-pong tiles): row
-  // m at position start_pos + m of one sequence's cache.
+  // of sequence m's cache.  Prefill (launch_qkv_rope_prefill, the 192-row ping-pong tiles or the
+  // split reduction): row m at position start_pos + m of one sequence's cache.
   kGemmQkvRope = 4,
 };
 struct GemmParams {
@@ -203,9 +203,9 @@ struct GemmParams {
   // Producer (kGemmResid, N = 16 kNormParts): also writes the sums of squares of each 16
   // columns of the new rows to ss_out[row][n / 16].
   float* ss_out;
-  // Split K (bf16 / residual / SwiGLU epilogues, 16 < M <= kSplitMaxRows): scratch for
-  // fp32 partial products [splits][M][N]; when set and the tiles would fill at most half the
-  // chip, K is split across workgroups and a reduction applies the epilogue.
+  // Split K (every epilogue but fp32, M > 16): scratch for fp32 partial products [splits][M][N]
+  // (SwiGLU: 2N columns).  When set, the launcher may split K across workgroups, as many ways as it
+  // models fastest and the bytes hold, and a reduction applies the epilogue.
   float* split_ws;
   long long split_ws_bytes;
   // Residual epilogue with K split, N = 4096: when rn_out is set the reduction also writes
@@ -228,8 +228,9 @@ struct GemmParams {
 // Bytes of sk_part for up to kSkTailMax split tiles.
 constexpr size_t kSkPartBytes = (size_t)kSkTailMax * 2 * 2 * 64 * 4 * sizeof(float);
 constexpr int kSplitMaxRows = 1024;
-// Scratch bytes split K may use for an M-row product with n output columns (SwiGLU: 2 x the
-// output columns): 2048 partial rows, i.e. up to 16 planes at M <= 128, 4 at M = 512.
+// Scratch bytes that the prefill workspaces hold for split K of an M-row product with n output
+// columns (SwiGLU: 2 x the output columns): 2048 partial rows, i.e. up to 16 planes at M <= 128, 4
+// at M = 512.
 inline size_t gemm_split_bytes(int M, int n) {
   return M <= kSplitMaxRows ? (size_t)(4 * M > 2048 ? 4 * M : 2048) * n * sizeof(float) : 0;
 }
@@ -242,10 +243,10 @@ inline size_t gemm_op_split_bytes(int M, int n) {
   return room > gemm_split_bytes(M, n) ? room : gemm_split_bytes(M, n);
 }
 int launch_gemm(int epi, const GemmParams& p, hipStream_t st);
-// Prefill QKV projection with RoPE and the K/V scatter in the GEMM epilogue (kGemmQkvRope,
-// start_pos): launched when the bf16 product would run as one launch of the 192 x 256
-// ping-pong tiles; returns 1 without launching otherwise (the caller then runs the bf16
-// product and the scatter kernel, with the same results bit for bit).
+// Prefill QKV projection with RoPE and the K/V scatter in the GEMM epilogue or the split reduction
+// (kGemmQkvRope, start_pos), past 16 rows; returns 1 without launching otherwise, for operands off
+// 16 bytes and under schedule 0 (the caller then runs the bf16 product and the scatter kernel, with
+// the same results bit for bit).
 int launch_qkv_rope_prefill(const GemmParams& p, hipStream_t st);
 
 // ------------------------------------------------------------ weight arena (engine.hip)

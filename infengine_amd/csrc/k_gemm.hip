@@ -1286,8 +1286,9 @@ double tile_us(int bn, int bm, double step, double kt, double wgs) {
 }
 
 // Model (us), fitted to 78 measured shapes (the four layer products at 130 .. 6000 rows, weights
-// from HBM, 16 tile shapes x their K splits; 6% rms, and the shape it picks is 1% off the best
-// measured one on average, 12% at most):
+// from HBM, tile shapes x K splits).  Against 1069 timings of the four products at 16 row counts it is
+// 6.7% rms off, and the shape that it picks is 1.4% off the best timed one on average (15% at most
+// but for down at 130 rows, 37%):
 //   launch 1.4 + rounds x (k-steps x step + 3.95 + 4.18 x tile / 64 Ki)
 // a step 28% faster on an empty chip than on a full one; past one round 0.71 of the time goes
 // with whole rounds, 0.29 with the tiles; K splits add 3.2 + 0.245 per MB of fp32 partials; the

@@ -574,6 +574,7 @@ int launch_gemv(int K, int epi, bool norm, GemvParams p, int rows, hipStream_t s
     }
     return IE_OK;
   }
+  // one row (gemv_kernel's row index is blockIdx.y = 0)
   if (p.ppw <= 0) p.ppw = default_ppw(p.n_pairs);
   if (K == 4096) return launch_k<4096>(epi, norm, p, st);
   if (K == 14336) return launch_k<14336>(epi, norm, p, st);

@@ -43,7 +43,7 @@ def _noalloc(hip, ctx, logits, rows, vocab, seed, step):
 
 
 def test_top_p_noalloc_matches_workspace_entry(hip, ctx):
-    # first call: 16 full-vocabulary rows (2,052,096 of the 2,097,152 scratch floats)
+    # first call: 16 full-vocabulary rows (2,052,096 of the 2,097,152 logits that a call may have)
     rows, vocab = 16, V
     say(f"top-p noalloc call 1: rows={rows} vocab={vocab}")
     big = _logits(rows, vocab, 1)
@@ -52,7 +52,7 @@ def test_top_p_noalloc_matches_workspace_entry(hip, ctx):
         want = _with_workspace(hip, ctx, big, rows, vocab, 42, step)
         assert got == want, (step, got, want)
         assert all(0 <= t < vocab for t in got)
-    # second call, smaller: the scratch still holds the first call's exponentials
+    # second call, smaller: the scratch still holds the first call's row state
     rows2, vocab2 = 3, 50_000
     say(f"top-p noalloc call 2: rows={rows2} vocab={vocab2}")
     small = _logits(rows2, vocab2, 2)
