@@ -154,7 +154,9 @@ int launch_top_p(int rows, int vocab, const float* logits, float temperature, fl
 constexpr size_t kTopPNoallocFloats = (size_t)IE_TOP_P_NOALLOC_MAX;  // rows * vocab accepted
 constexpr int kTopPNoallocRows = IE_TOP_P_NOALLOC_ROWS;
 constexpr size_t kTopPScratchBytes = (size_t)kTopPNoallocRows * (128 << 10);  // (< 128 KiB a row)
-// Workspace of launch_top_p: the per-row state.
+// Workspace of launch_top_p: the per-row state, kTopPRowBytes a row (callers have laid it out by
+// ie_top_p_workspace_size: fixed).
+constexpr size_t kTopPRowBytes = 116000;
 size_t top_p_workspace_bytes(int rows);
 int top_p_scratch_init(int device);
 float* top_p_scratch(int device);

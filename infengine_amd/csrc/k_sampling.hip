@@ -166,11 +166,11 @@ __device__ __forceinline__ T wave_scan(T v) {
 // row has its cut where the bins are finer.  The cut bin of N(0, s) logits holds up to about 128256 x
 // width / (2.5 s) tokens: the candidate list takes them from s = 0.09 on.  512 even bins took them from
 // 0.27 on; 16 rows at p = 0.5, us, even bins / these: s = 0.1 275 / 46, 0.3 46 / 34, 0.8 34.5 / 32, 2.0
-// 29.0 / 29.2 (p = 0.9: 31.3 / 31.9).  (576 bins, even past 1.2 nats: 30.3 and 32.9 at s = 2.0.)
+// 29.5 / 29.7 (p = 0.9: 31.2 / 31.7).  (576 bins, even past 1.2 nats: 30.3 and 32.9 at s = 2.0.)
 constexpr int kTopPBins = 512;
 constexpr int kTopPChunks = 64;
 constexpr int kTopPChunkThreads = 256;
-constexpr int kTopPCandMax = 9216;
+constexpr int kTopPCandMax = 9214;
 constexpr int kTopPCandLds = 4096;  // candidates that tp_finish keeps in LDS
 
 struct TopPRow {
@@ -183,9 +183,10 @@ struct TopPRow {
   unsigned long long above, target;
   uint32_t cand_key[kTopPCandMax];
   unsigned long long cand_q[kTopPCandMax];  // mass (41 bits) | chunk << 48
-  unsigned long long pad;
 };
-static_assert(sizeof(TopPRow) == 116000, "callers' workspaces are sized by it (ie_top_p_workspace_size)");
+// (rows that share cache lines make the histograms' additions slower: 16 rows 30.2 us, 29.1 so)
+static_assert(sizeof(TopPRow) <= kTopPRowBytes && sizeof(TopPRow) % 256 == 0,
+              "within the row of a caller's workspace, whole cache lines");
 
 // The octaves 2-4, 4-8, 8-16 and 16-32 of 1.08 d + 2 (from 32 on, and NaN: any bin, without mass).
 __host__ __device__ __forceinline__ int top_p_bin(float d) {
@@ -554,7 +555,7 @@ int launch_argmax_rows(int rows, int vocab, const float* logits, int* out,
   return IE_OK;
 }
 
-size_t top_p_workspace_bytes(int rows) { return (size_t)rows * sizeof(TopPRow); }
+size_t top_p_workspace_bytes(int rows) { return (size_t)rows * kTopPRowBytes; }
 
 int launch_top_p(int rows, int vocab, const float* logits, float temperature, float top_p,
                  uint64_t seed, uint64_t step, int* out, float* ws, hipStream_t st) {
