@@ -370,7 +370,8 @@ IE_API int ie_gemm_bf16(ie_context* ctx, int m, int k, int n, const ie_bf16* d_x
  * The product may split K over a scratch of the context, allocated by the first
  * call that needs more of it (refused while the context's stream is captured: run such a call
  * once before) and kept until the context is destroyed.  Graphs recorded from one context with
- * such calls share it: they must not replay at once, nor after the context. */
+ * such calls share it with each other and with its later calls: none of them may run at once, nor
+ * a replay after the context. */
 #define IE_GEMM_BF16 0
 #define IE_GEMM_RESID 1
 #define IE_GEMM_F32 2
